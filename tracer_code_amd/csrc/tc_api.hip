@@ -72,7 +72,8 @@ struct tc_dev {
     bool coarse_ready = false;
     bool trace = false;
     bool coarse_lu = false;
-    bool tb = true;            // temporally blocked sweeps on levels >= 2
+    bool tb = true;            // several sweeps per launch (TC_TB=0: one)
+    bool std_tables = false;   // the FD tables are those k_visit_ref has built in
     bool fuse_rr = true;       // residual+restriction in the last blocked launch of a visit (TC_FUSED_RR=0: apart)
     // defect-correction cycle: level-1 residual updated by increments (k_absorb_inc) with an exact
     // double-double residual before the stop test accepts (TC_INC_RESID=0: exact after every correction)
@@ -508,17 +509,28 @@ void cheb_factors(int n, int Niter, int dir, double& temp, double& cconst)
     }
 }
 
+// whether the reference form runs several sweeps per launch
+bool ref_blocked(const tc_ctx* ctx, const tc_dev& d)
+{
+    return d.tb && d.std_tables && ctx->mode == TC_MODE_FP64;
+}
+
 // The Niter sweeps of one visit of `level` on its error buffers (FP64
 // err[] or FP32 err32[]).  view.rhs is the FP64 right-hand side, rhs32 the
-// FP32 one.  In the defect-correction modes the levels >= 2 run several
-// sweeps per launch (k_sweep_tb, the 13-tap form of the operator) unless
-// TC_TB=0; the reference-form path and level 1 run one sweep per launch.
+// FP32 one.  Several sweeps run per launch unless TC_TB=0: in the reference
+// form on every level (k_visit_ref, the same bits as one sweep per launch;
+// level 1 after its first sweep of a solve), in the defect-correction modes
+// on levels >= 2 (k_sweep_tb, the 13-tap form of the operator).
 // rr (FP32 blocked sweeps): the visit's last launch also forms the next
 // coarser level's right-hand side; *rr_done says whether it did.
+// res (reference form): the residual of the result goes there where the
+// visit's last launch can form it; *res_done says whether it did.
 int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, const Level& view, const float* rhs32,
-               bool* first_sweep, bool zero_start = false, const RRTarget* rr = nullptr, bool* rr_done = nullptr)
+               bool* first_sweep, bool zero_start = false, const RRTarget* rr = nullptr, bool* rr_done = nullptr,
+               double* res = nullptr, bool* res_done = nullptr)
 {
     if (rr_done) *rr_done = false;
+    if (res_done) *res_done = false;
     Level& L = ctx->lv[level];
     const tc_params& P = ctx->p;
     const double zsg = (P.Vbc == 0) ? -1.0 : 1.0;
@@ -543,8 +555,29 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
     const bool timed = ctx->prof && level == 1 && !tb;
     const bool timed_visit = timed && !(first_sweep && *first_sweep);
     if (timed_visit) TC_TRY(prof_begin(ctx));
+    const bool ref = ref_blocked(ctx, d);
+    const VisitPlan plan = ref ? visit_plan_ref(L.g, d.cus) : VisitPlan{};
     int n = 1;
     while (n <= Niter) {
+        if (ref && !(first_sweep && *first_sweep)) {
+            const int nk = std::min(plan.k, Niter - n + 1);
+            double fac[VISIT_KMAX];
+            for (int s = 0; s < nk; ++s) {
+                double temp, cconst;
+                cheb_factors(n + s, Niter, dir, temp, cconst);
+                fac[s] = use_ratio ? temp : cconst;
+            }
+            const bool with_res = res && plan.whole && n + nk - 1 == Niter;
+            if (timed && !timed_visit) TC_TRY(prof_begin(ctx));
+            launch_visit_ref(ctx->stream, plan, d.pow2[level], use_ratio, view, view.rhs,
+                             (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk, zsg,
+                             with_res ? res : nullptr);
+            if (timed && !timed_visit) TC_TRY(prof_end(ctx, nk));
+            if (with_res && res_done) *res_done = true;
+            L.cur = 1 - L.cur;
+            n += nk;
+            continue;
+        }
         if (tb) {
             const int nk = std::min(tb_max_sweeps(K), Niter - n + 1);
             double temp[8], cc[8];
@@ -604,11 +637,19 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
     return 0;
 }
 
-int iterate_stream(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool& first_sweep)
+// zero_start: the visit starts from a zero correction, which error(level)
+// does not hold yet
+int iterate_stream(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool& first_sweep, bool zero_start)
 {
     Level& L = ctx->lv[level];
     const tc_params& P = ctx->p;
-    TC_TRY(run_sweeps(ctx, d, level, Niter, dir, false, L, nullptr, &first_sweep));
+    bool res_done = false;
+    TC_TRY(run_sweeps(ctx, d, level, Niter, dir, false, L, nullptr, &first_sweep, zero_start, nullptr, nullptr,
+                      level > 1 ? L.res : nullptr, &res_done));
+    if (res_done) {
+        ctx->stats.residuals_exec[level - 1]++;
+        return 0;
+    }
     // compute_residual
     int nb = launch_residual(ctx->stream, d.pow2[level], L, L.err[L.cur], L.res, d.F, d.h[level], P.ivis,
                              level == 1 ? d.partialA : nullptr);
@@ -774,17 +815,20 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
         for (int p = 1; p <= P.nsteps; ++p) {
             const int level = multi[p];
             const int dir = (multi[p + 1] > multi[p]) ? 0 : 1;
+            bool zero_start = false;
             if (multi[p - 1] < multi[p]) {
                 // compute_RHS(level) = restrict(residual of level-1)
                 Level& Lf = ctx->lv[level - 1];
                 launch_restrict(ctx->stream, Lf.res, Lf.g, ctx->lv[level].rhs, ctx->lv[level].g);
-                if (P.fixes & TC_FIX_ZERO_COARSE) {
+                // (the blocked sweeps of a visit start from zeros without a fill)
+                zero_start = (P.fixes & TC_FIX_ZERO_COARSE) && level < G && P.Nmulti > 0 && ref_blocked(ctx, d);
+                if ((P.fixes & TC_FIX_ZERO_COARSE) && !zero_start) {
                     Level& Lc = ctx->lv[level];
                     TC_HIP(hipMemsetAsync(Lc.err[Lc.cur], 0, plane_bytes(Lc.g), ctx->stream));
                 }
             }
             if (level < G) {
-                TC_TRY(iterate_stream(ctx, d, level, P.Nmulti, dir, first_sweep));
+                TC_TRY(iterate_stream(ctx, d, level, P.Nmulti, dir, first_sweep, zero_start));
             } else {
                 Level& Lc = ctx->lv[G];
                 TC_TRY(wait_coarse(ctx, d));
@@ -2292,6 +2336,7 @@ int init_ctx(tc_ctx* ctx, const tc_params* p, int64_t ntr)
             d->F.Drrs[t] = p->D1[dk + 2] * p->D2[di + 2];
             d->F.Drrss[t] = p->D2[dk + 2] * p->D2[di + 2];
         }
+    d->std_tables = visit_tables(d->F);
     // level hierarchy (basics.f90:167-182)
     for (int j = 1; j <= ctx->grids; ++j) {
         Level& L = ctx->lv[j];

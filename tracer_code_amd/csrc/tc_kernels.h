@@ -214,6 +214,25 @@ bool launch_sweep_tb32(hipStream_t st, bool use_ratio, int K, const Level& L, co
                        double zsg, const float* Pc = nullptr, const Grid* gc = nullptr,
                        const RRTarget* rr = nullptr);
 
+// --- tc_visit.hip ---------------------------------------------------------------
+// How a level's sweeps are launched: the region of a workgroup (cfg), the
+// sweeps of a launch, and whether one workgroup holds the whole level.
+constexpr int VISIT_KMAX = 96;  // most sweeps of one launch
+struct VisitPlan {
+    int cfg = 0;
+    int k = 1;
+    bool whole = false;
+};
+bool visit_tables(const FD& F);
+VisitPlan visit_plan_ref(const Grid& g, int cus);
+// nk sweeps of the FP64 reference form from `in` (nullptr: a zero
+// correction) into `out`; fac: the sweeps' factors (use_ratio: the cosines
+// of the per-point factors); res (plan.whole only): the residual of the
+// result.  rhs, walls and bits as launch_sweep / launch_residual.
+void launch_visit_ref(hipStream_t st, const VisitPlan& p, bool pow2, bool use_ratio, const Level& L, const double* rhs,
+                      const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
+                      double* res);
+
 // --- tc_fields.hip -------------------------------------------------------------
 void launch_velocities(hipStream_t st, const double* SF, double* u, double* w, const Grid& g, const FD& F, double dr,
                        double ds, int Vbc);
