@@ -440,8 +440,7 @@ enum { TC_K_SWEEP_L1 = 0, TC_K_COUNT };
  * reset follows the first sweep); enable=0 stops. */
 int tc_set_profiling(tc_ctx* ctx, int enable);
 /* Average device duration (microseconds) and launch count of kernel `which`
- * since profiling was enabled; a launch that makes several sweeps (the FP64
- * reference form) counts as so many. */
+ * since profiling was enabled (a launch makes several sweeps). */
 int tc_kernel_timing(tc_ctx* ctx, int which, double* avg_us, int64_t* count);
 
 /* ---- learned initial guess (no counterpart in the reference) ----------- */

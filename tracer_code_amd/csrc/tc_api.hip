@@ -72,9 +72,9 @@ struct tc_dev {
     bool coarse_ready = false;
     bool trace = false;
     bool coarse_lu = false;
-    bool tb = true;            // several sweeps per launch (TC_TB=0: one)
-    bool std_tables = false;   // the FD tables are those k_visit_ref has built in
-    bool fuse_rr = true;       // residual+restriction in the last blocked launch of a visit (TC_FUSED_RR=0: apart)
+    bool tb = true;            // several sweeps per launch (TC_TB=0, or FD tables other than the second-order ones: one)
+    bool std_tables = false;   // the FD tables are those that the kernels of tc_visit.hip have built in
+    bool fuse_rr = true;       // residual+restriction in the last launch of a visit (TC_FUSED_RR=0: apart)
     // defect-correction cycle: level-1 residual updated by increments (k_absorb_inc) with an exact
     // double-double residual before the stop test accepts (TC_INC_RESID=0: exact after every correction)
     bool inc_res = true;
@@ -512,7 +512,17 @@ void cheb_factors(int n, int Niter, int dir, double& temp, double& cconst)
 // whether the reference form runs several sweeps per launch
 bool ref_blocked(const tc_ctx* ctx, const tc_dev& d)
 {
-    return d.tb && d.std_tables && ctx->mode == TC_MODE_FP64;
+    return d.tb && ctx->mode == TC_MODE_FP64;
+}
+
+// whether a level's visits in the defect-correction cycle run several sweeps
+// per launch (k_visit13): they can then start from a zero correction without
+// a fill (run_sweeps' zero_start).  Level 1 in the mixed mode does not where
+// the Gauss-Seidel smoother takes its place.
+bool dc_blocked(const tc_ctx* ctx, const tc_dev& d, int level, bool f32)
+{
+    return d.tb && level < ctx->grids && ctx->mode != TC_MODE_FP64 &&
+           !(level == 1 && f32 && ctx->gs_sweeps > 0 && ctx->mode == TC_MODE_MIXED);
 }
 
 // The Niter sweeps of one visit of `level` on its error buffers (FP64
@@ -520,8 +530,8 @@ bool ref_blocked(const tc_ctx* ctx, const tc_dev& d)
 // FP32 one.  Several sweeps run per launch unless TC_TB=0: in the reference
 // form on every level (k_visit_ref, the same bits as one sweep per launch;
 // level 1 after its first sweep of a solve), in the defect-correction modes
-// on levels >= 2 (k_sweep_tb, the 13-tap form of the operator).
-// rr (FP32 blocked sweeps): the visit's last launch also forms the next
+// in the 13-tap form of the operator (k_visit13).
+// rr (FP32, blocked): the visit's last launch also forms the next
 // coarser level's right-hand side; *rr_done says whether it did.
 // res (reference form): the residual of the result goes there where the
 // visit's last launch can form it; *res_done says whether it did.
@@ -546,73 +556,91 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
         ctx->stats.sweeps_exec[0] += ctx->gs_sweeps;
         return 0;
     }
-    const bool tb = d.tb && level >= 2 && ctx->mode != TC_MODE_FP64;
-    // sweeps per launch: 4, or 8 on FP32 levels of at most 16 tiles
-    const int K = (tb && f32 && L.tb_tile != 32 && L.tb_tile != 48) ? tb_sweeps_per_launch(L.g) : 4;
+    const bool tb = dc_blocked(ctx, d, level, f32);
     // level-1 timing (tc_set_profiling): one event pair around the visit's
     // back-to-back launches, or around each launch when the first sweep is
     // followed by the wall reset of the reference form
-    const bool timed = ctx->prof && level == 1 && !tb;
+    const bool timed = ctx->prof && level == 1;
     const bool timed_visit = timed && !(first_sweep && *first_sweep);
+    int launches = 0;
     if (timed_visit) TC_TRY(prof_begin(ctx));
+    // the factor of sweep n of the visit (the cosine on the ratio level).  The
+    // FP32 cycle's level-1 interval (tc_set_dc_cheb_interval) applies at a
+    // tuned count only: the Nmulti retry of a solve that diverged or
+    // stalled runs the reference's factors (a wide interval's steps reach
+    // 4x the local time step, and Nmulti of them amplify the FP32
+    // rounding of the high modes until the solve blows up)
+    const bool cheb1 = f32 && level == 1 && dir != 1 && ctx->dc_sweeps > 0 && ctx->dc_sweeps != P.Nmulti &&
+                       ctx->dc_sweeps_active == ctx->dc_sweeps;
+    auto factors = [&](int n, double& temp, double& cconst) {
+        cheb_factors(n, Niter, dir, temp, cconst);
+        if (cheb1) cconst = 2.0 / (-ctx->cheb1_lb - ctx->cheb1_la + (ctx->cheb1_lb - ctx->cheb1_la) * temp);
+    };
+    auto factor_row = [&](int n, int nk, double* fac) {
+        for (int s = 0; s < nk; ++s) {
+            double temp, cconst;
+            factors(n + s, temp, cconst);
+            fac[s] = use_ratio ? temp : cconst;
+        }
+    };
     const bool ref = ref_blocked(ctx, d);
     const VisitPlan plan = ref ? visit_plan_ref(L.g, d.cus) : VisitPlan{};
     int n = 1;
+    if (tb && Niter > 0) {
+        // the tile asked for by tc_set_tb_tile: 16, 32 or 48, small to large regions
+        const int only = L.tb_tile == 16 ? 2 : (L.tb_tile == 32 ? 1 : (L.tb_tile == 48 ? 3 : 0));
+        const Visit13Plan pl = visit_plan13(L.g, f32, Niter, f32 && rr, d.cus, only);
+        const int body = (pl.end && !pl.whole) ? Niter - pl.end_k : Niter;  // sweeps of the equal launches
+        double fac[VISIT_KMAX];
+        for (int j = 0; j < pl.launches || n <= Niter; ++j) {
+            const bool endl = j >= pl.launches;  // the launch after the equal ones
+            const int left = pl.launches - j;
+            const int nk = endl ? Niter - n + 1 : (body - n + 1 + left - 1) / left;
+            if (nk <= 0) continue;
+            factor_row(n, nk, fac);
+            const int cfg = endl ? pl.end_cfg : pl.cfg;
+            const bool last = n + nk - 1 == Niter;
+            if (f32) {
+                // the first launch of a zero-started visit starts from zeros instead of reading
+                // them; the first launch after an ascent adds the prolonged coarse correction
+                const float* in = (zero_start && n == 1) ? nullptr : L.err32[L.cur32];
+                const bool pro = n == 1 && ctx->pend_src && ctx->pend_level == level;
+                const bool with_rr = last && pl.end;
+                launch_visit13_32(ctx->stream, cfg, pl.whole, use_ratio, L, rhs32, in, L.err32[1 - L.cur32], d.h[level],
+                                  fac, nk, zsg, pro ? ctx->pend_src : nullptr,
+                                  pro ? &ctx->lv[ctx->pend_from].g : nullptr, with_rr ? rr : nullptr);
+                if (with_rr && rr_done) *rr_done = true;
+                if (pro) ctx->pend_src = nullptr;
+                L.cur32 = 1 - L.cur32;
+            } else {
+                launch_visit13_64(ctx->stream, cfg, pl.whole, use_ratio, L, view.rhs,
+                                  (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk,
+                                  zsg);
+                L.cur = 1 - L.cur;
+            }
+            ++launches;
+            n += nk;
+        }
+    }
     while (n <= Niter) {
         if (ref && !(first_sweep && *first_sweep)) {
             const int nk = std::min(plan.k, Niter - n + 1);
             double fac[VISIT_KMAX];
-            for (int s = 0; s < nk; ++s) {
-                double temp, cconst;
-                cheb_factors(n + s, Niter, dir, temp, cconst);
-                fac[s] = use_ratio ? temp : cconst;
-            }
+            factor_row(n, nk, fac);
             const bool with_res = res && plan.whole && n + nk - 1 == Niter;
             if (timed && !timed_visit) TC_TRY(prof_begin(ctx));
             launch_visit_ref(ctx->stream, plan, d.pow2[level], use_ratio, view, view.rhs,
                              (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk, zsg,
                              with_res ? res : nullptr);
-            if (timed && !timed_visit) TC_TRY(prof_end(ctx, nk));
+            if (timed && !timed_visit) TC_TRY(prof_end(ctx, 1));
             if (with_res && res_done) *res_done = true;
             L.cur = 1 - L.cur;
-            n += nk;
-            continue;
-        }
-        if (tb) {
-            const int nk = std::min(tb_max_sweeps(K), Niter - n + 1);
-            double temp[8], cc[8];
-            for (int s = 0; s < nk; ++s) cheb_factors(n + s, Niter, dir, temp[s], cc[s]);
-            if (f32) {
-                // the first launch of a zero-started visit stages zeros instead of reading them;
-                // the first launch after an ascent adds the prolonged coarse correction
-                const float* in = (zero_start && n == 1) ? nullptr : L.err32[L.cur32];
-                const bool pro = n == 1 && ctx->pend_src && ctx->pend_level == level;
-                const bool last = n + nk - 1 == Niter;
-                const bool fused =
-                    launch_sweep_tb32(ctx->stream, use_ratio, K, L, rhs32, in, L.err32[1 - L.cur32], d.F, d.h[level],
-                                      temp, cc, nk, zsg, pro ? ctx->pend_src : nullptr,
-                                      pro ? &ctx->lv[ctx->pend_from].g : nullptr, last ? rr : nullptr);
-                if (fused && rr_done) *rr_done = true;
-                if (pro) ctx->pend_src = nullptr;
-                L.cur32 = 1 - L.cur32;
-            } else {
-                launch_sweep_tb64(ctx->stream, use_ratio, K, L, view.rhs, L.err[L.cur], L.err[1 - L.cur], d.F,
-                                  d.h[level], temp, cc, nk, zsg);
-                L.cur = 1 - L.cur;
-            }
+            ++launches;
             n += nk;
             continue;
         }
         double temp, cconst;
-        cheb_factors(n, Niter, dir, temp, cconst);
-        // the FP32 cycle's level-1 interval (tc_set_dc_cheb_interval), at a
-        // tuned count only: the Nmulti retry of a solve that diverged or
-        // stalled runs the reference's factors (a wide interval's steps reach
-        // 4x the local time step, and Nmulti of them amplify the FP32
-        // rounding of the high modes until the solve blows up)
-        if (f32 && level == 1 && dir != 1 && ctx->dc_sweeps > 0 && ctx->dc_sweeps != P.Nmulti &&
-            ctx->dc_sweeps_active == ctx->dc_sweeps)
-            cconst = 2.0 / (-ctx->cheb1_lb - ctx->cheb1_la + (ctx->cheb1_lb - ctx->cheb1_la) * temp);
+        factors(n, temp, cconst);
         if (timed && !timed_visit) TC_TRY(prof_begin(ctx));
         if (f32) {
             launch_sweep32(ctx->stream, use_ratio, L, L.err32[L.cur32], L.err32[1 - L.cur32], rhs32, d.F, d.h[level],
@@ -630,9 +658,10 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
             launch_bc_stream(ctx->stream, L.err[1 - L.cur], L.g, P.Vbc);
             *first_sweep = false;
         }
+        ++launches;
         ++n;
     }
-    if (timed_visit) TC_TRY(prof_end(ctx, Niter));
+    if (timed_visit) TC_TRY(prof_end(ctx, launches));
     ctx->stats.sweeps_exec[level - 1] += Niter;
     return 0;
 }
@@ -1074,13 +1103,6 @@ int dc_alloc(tc_ctx* ctx)
 
 // Jacobi-Richardson sweeps of one visit on a correction level (FP32 or
 // FP64), followed (level > 1) by compute_residual of the level.
-// blocked FP32 sweeps on this level: its visits can start from a zero
-// correction without a fill (run_sweeps' zero_start)
-bool tb_zero_start(const tc_ctx* ctx, const tc_dev& d, int level, bool f32)
-{
-    return f32 && d.tb && level >= 2 && level < ctx->grids && ctx->mode != TC_MODE_FP64;
-}
-
 int dc_iterate(tc_ctx* ctx, tc_dev& d, int level, int dir, bool f32, bool zero_start = false,
                const RRTarget* rr = nullptr, bool* rr_done = nullptr)
 {
@@ -1091,8 +1113,13 @@ int dc_iterate(tc_ctx* ctx, tc_dev& d, int level, int dir, bool f32, bool zero_s
     if (level == 1) view.rhs = L.res;
     const float* rhs32 = (level == 1) ? L.res32 : L.rhs32;
     // a per-level count applies to the tuned cycle, not to the Nmulti retry
+    if (level == 1) zero_start = dc_blocked(ctx, d, 1, f32);  // e(1) is zero at the start of every visit
     int n = ctx->dc_sweeps_active;
     if (ctx->dc_level_sweeps[level] > 0 && ctx->dc_sweeps > 0 && n == ctx->dc_sweeps) n = ctx->dc_level_sweeps[level];
+    if (n <= 0 && zero_start) {  // no sweep that would write the zeros
+        if (f32) launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err32[L.cur32]), L.g.elems);
+        else launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err[L.cur]), 2 * L.g.elems);
+    }
     TC_TRY(run_sweeps(ctx, d, level, n, dir, f32, view, rhs32, nullptr, zero_start, rr, rr_done));
     // FP64: compute_residual now; FP32: fused into the restriction of the
     // next descent (k_residual_restrict32), the only reader of the residual
@@ -1114,9 +1141,12 @@ int dc_absorb_residual(tc_ctx* ctx, tc_dev& d, bool f32)
                                          f32 ? nullptr : L1.err[L1.cur], nullptr, L1, L1.res,
                                          f32 ? L1.res32 : nullptr, d.F, d.h[1], ctx->p.ivis, d.pow2[1], zsg,
                                          d.partialA);
-        // e(1) back to zero for the next visit (a fill kernel: capturable)
-        if (f32) launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L1.err32[L1.cur32]), L1.g.elems);
-        else launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L1.err[L1.cur]), 2 * L1.g.elems);
+        // e(1) back to zero for the next visit (a fill kernel: capturable);
+        // a blocked visit starts from zeros without reading them
+        if (!dc_blocked(ctx, d, 1, f32)) {
+            if (f32) launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L1.err32[L1.cur32]), L1.g.elems);
+            else launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L1.err[L1.cur]), 2 * L1.g.elems);
+        }
         launch_reduce_final(ctx->stream, d.partialA, nb, 0, d.d_scal, S_RESID1);
         ctx->stats.residuals_exec[0]++;
         d.res_exact = false;
@@ -1267,9 +1297,6 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
     TC_TRY(solve_setup(ctx, d));
     if (f32) {
         for (int L = 1; L <= G; ++L) launch_coeffs_to_f32(ctx->stream, ctx->lv[L], L == ctx->ratio_level, P.ivis);
-        if (d.tb)
-            for (int L = 2; L < G; ++L)
-                if (tb_uses_w13(ctx->lv[L])) launch_tb_weights32(ctx->stream, ctx->lv[L], d.F, d.h[L]);
         if (ctx->gs_sweeps > 0) {
             launch_tb_weights32(ctx->stream, L1, d.F, d.h[1]);
             if (!L1.w13) {
@@ -1387,7 +1414,7 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
         const int level = multi[p];
         const int dir = (multi[p + 1] > multi[p]) ? 0 : 1;
         Level& L = ctx->lv[level];
-        const bool zero_start = multi[p - 1] < multi[p] && tb_zero_start(ctx, d, level, f32);
+        const bool zero_start = multi[p - 1] < multi[p] && dc_blocked(ctx, d, level, f32);
         if (multi[p - 1] < multi[p]) {
             Level& Lf = ctx->lv[level - 1];
             if (f32) {
@@ -1402,12 +1429,12 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                     // the equilibration of the inverse in use (ready after the wait)
                     TC_TRY(wait_coarse(ctx, d));
                     launch_residual_restrict32(ctx->stream, Lf, Lf.err32[Lf.cur32], Lf.rhs32, d.F, d.h[level - 1],
-                                               L.rhs32, L.g, ctx->RowB, ctx->coarse_b);
+                                               L.rhs32, L.g, ctx->RowB, ctx->coarse_b, d.std_tables);
                     ctx->stats.residuals_exec[level - 2]++;
                     coarse_b_ready = true;
                 } else {
                     launch_residual_restrict32(ctx->stream, Lf, Lf.err32[Lf.cur32], Lf.rhs32, d.F, d.h[level - 1],
-                                               L.rhs32, L.g);
+                                               L.rhs32, L.g, nullptr, nullptr, d.std_tables);
                     ctx->stats.residuals_exec[level - 2]++;
                 }
                 // a fill kernel, not a memset: this can be recorded in a graph.  The
@@ -1417,7 +1444,7 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                     launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err32[L.cur32]), L.g.elems);
             } else {
                 launch_restrict(ctx->stream, Lf.res, Lf.g, L.rhs, L.g);
-                TC_HIP(hipMemsetAsync(L.err[L.cur], 0, plane_bytes(L.g), ctx->stream));
+                if (!zero_start) TC_HIP(hipMemsetAsync(L.err[L.cur], 0, plane_bytes(L.g), ctx->stream));
             }
         }
         if (level < G) {
@@ -1430,7 +1457,6 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                 Level& Lc = ctx->lv[level + 1];
                 rrt.out = Lc.rhs32;
                 rrt.go = Lc.g;
-                rrt.cus = d.cus;
                 if (level + 1 == G) {
                     TC_TRY(wait_coarse(ctx, d));
                     rrt.RowB = ctx->RowB;
@@ -1478,7 +1504,7 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                                        f32 ? Lf.res32 : nullptr, d.F, d.h[1], P.ivis, nullptr);
                 }
                 ctx->stats.residuals_exec[0]++;
-            } else if (f32 && tb_zero_start(ctx, d, level - 1, f32) && multi[p + 1] == level - 1) {
+            } else if (f32 && dc_blocked(ctx, d, level - 1, f32) && multi[p + 1] == level - 1) {
                 // folded into the first blocked launch of level-1's next visit
                 ctx->pend_src = L.err32[L.cur32];
                 ctx->pend_level = level - 1;
@@ -2337,6 +2363,7 @@ int init_ctx(tc_ctx* ctx, const tc_params* p, int64_t ntr)
             d->F.Drrss[t] = p->D2[dk + 2] * p->D2[di + 2];
         }
     d->std_tables = visit_tables(d->F);
+    d->tb = d->tb && d->std_tables;
     // level hierarchy (basics.f90:167-182)
     for (int j = 1; j <= ctx->grids; ++j) {
         Level& L = ctx->lv[j];

@@ -426,6 +426,8 @@ __global__ __launch_bounds__(256) void k_restrict32(const float* __restrict__ in
 // order -- the same values as the two kernels, without the residual plane.
 // With bout (the coarsest level), also the equilibrated right-hand side of
 // the coarse solve at the interior unknowns, as k_coarse_rhs32 forms it.
+// STD: the second-order tables, in the arithmetic of k_visit13's fused form.
+template <bool STD>
 __global__ __launch_bounds__(256) void k_residual_restrict32(const float* __restrict__ S, const float* __restrict__ vis,
                                                              const float* __restrict__ vx, const float* __restrict__ vz,
                                                              const float* __restrict__ a1,
@@ -460,9 +462,13 @@ __global__ __launch_bounds__(256) void k_residual_restrict32(const float* __rest
     if (!in) return;
     float rv[8];
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
-        rv[t] = (float)stream_space32_g<double>(F, h, Patch7At{P, RA[t], RB[t]}, cf[t][0], cf[t][1], cf[t][2], cf[t][3],
-                                                cf[t][4], cf[t][5]);
+    for (int t = 0; t < 8; ++t) {
+        const Patch7At at{P, RA[t], RB[t]};
+        if constexpr (STD)
+            rv[t] = residual32_std(taps13(at), h, cf[t][0], cf[t][1], cf[t][2], cf[t][3], cf[t][4], cf[t][5]);
+        else
+            rv[t] = (float)stream_space32_g<double>(F, h, at, cf[t][0], cf[t][1], cf[t][2], cf[t][3], cf[t][4], cf[t][5]);
+    }
     const float v = restrict_fw32(rv[0], rv[1], rv[2], rv[3], rv[4], rv[5], rv[6], rv[7]);
     out[go.at(i, k)] = v;
     if (bout) {
@@ -889,11 +895,16 @@ void launch_restrict32(hipStream_t st, const float* in, const Grid& gi, float* o
 }
 
 void launch_residual_restrict32(hipStream_t st, const Level& Lf, const float* S, const float* rhs, const FD& F,
-                                const Spacing& h, float* out, const Grid& go, const double* RowB, double* bout)
+                                const Spacing& h, float* out, const Grid& go, const double* RowB, double* bout,
+                                bool std_tables)
 {
     dim3 b(64, 4);
-    hipLaunchKernelGGL(k_residual_restrict32, grid2(go.nx - 1, go.nz - 1, b), b, 0, st, S, Lf.vis32, Lf.visx32,
-                       Lf.visz32, Lf.a132, Lf.visxz32, rhs, Lf.g, fd32_from(F), h32_from(h), out, go, RowB, bout);
+    if (std_tables)
+        hipLaunchKernelGGL(k_residual_restrict32<true>, grid2(go.nx - 1, go.nz - 1, b), b, 0, st, S, Lf.vis32, Lf.visx32,
+                           Lf.visz32, Lf.a132, Lf.visxz32, rhs, Lf.g, fd32_from(F), h32_from(h), out, go, RowB, bout);
+    else
+        hipLaunchKernelGGL(k_residual_restrict32<false>, grid2(go.nx - 1, go.nz - 1, b), b, 0, st, S, Lf.vis32, Lf.visx32,
+                           Lf.visz32, Lf.a132, Lf.visxz32, rhs, Lf.g, fd32_from(F), h32_from(h), out, go, RowB, bout);
 }
 
 void launch_prolong32(hipStream_t st, float* Ef, const Grid& gf, const float* Ec, const Grid& gc, double zsg)

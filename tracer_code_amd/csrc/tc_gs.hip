@@ -19,6 +19,7 @@
 // (:965-989) are refreshed in LDS as their interior cell is relaxed, and
 // written out with the tile.
 #include "tc_kernels.h"
+#include "tc_stencil32.h"
 
 namespace tc {
 
@@ -26,6 +27,34 @@ constexpr int GS_T = 48, GS_H = 2, GS_R = GS_T + 2 * GS_H, GS_THREADS = 256;
 static_assert(GS_T == 3 * 16 && GS_THREADS == 16 * 16, "one 3x3 block of the tile per thread");
 
 #pragma clang fp contract(fast)
+// The 13 dt-scaled tap weights of every interior cell of a level, once per
+// solve (the operator's coefficients are fixed during a solve), for any
+// tables: plane q of W holds tap q in the order c, xm1, xp1, xm2, xp2, zm1,
+// zp1, zm2, zp2, mm, pm, mp, pp.
+struct GsCoefs {
+    const float *vis, *vx, *vz, *a1, *vxz, *dts;
+};
+__global__ __launch_bounds__(256) void k_tb_weights32(GsCoefs C, FD32 F, H32 h, Grid g, float* __restrict__ W)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
+    const int k = blockIdx.y * blockDim.y + threadIdx.y + 1;
+    if (i > g.nx - 1 || k > g.nz - 1) return;
+    const size_t c = g.at(i, k), n = g.elems;
+    const float vis = C.vis[c], vx = C.vx[c], vz = C.vz[c], a1 = C.a1[c], vxz = C.vxz[c], dts = C.dts[c];
+    // axis parts: a1 (S_rr - S_ss) + 2 vx S_rrr + 2 vz S_sss + vis (S_rrrr + S_ssss)
+    auto wx = [&](int d) { return a1 * F.D2[d + 2] * h.idr2 + 2.0f * vx * F.D3[d + 2] * h.idr3 + vis * F.D4[d + 2] * h.idr4; };
+    auto wz = [&](int d) { return -a1 * F.D2[d + 2] * h.ids2 + 2.0f * vz * F.D3[d + 2] * h.ids3 + vis * F.D4[d + 2] * h.ids4; };
+    // 3x3 part: 4 vxz S_rs + 2 vx S_rss + 2 vz S_rrs + 2 vis S_rrss
+    auto wb = [&](int di, int dk) {
+        return 4.0f * vxz * F.D1[dk + 2] * F.D1[di + 2] * h.idrds + 2.0f * vx * F.D2[dk + 2] * F.D1[di + 2] * h.idrds2 +
+               2.0f * vz * F.D1[dk + 2] * F.D2[di + 2] * h.idr2ds + 2.0f * vis * F.D2[dk + 2] * F.D2[di + 2] * h.idr2ds2;
+    };
+    const float v[13] = {wx(0) + wz(0) + wb(0, 0), wx(-1) + wb(-1, 0), wx(1) + wb(1, 0), wx(-2), wx(2),
+                         wz(-1) + wb(0, -1), wz(1) + wb(0, 1), wz(-2), wz(2), wb(-1, -1), wb(1, -1), wb(-1, 1), wb(1, 1)};
+#pragma unroll
+    for (int q = 0; q < 13; ++q) W[q * n + c] = dts * v[q];
+}
+
 __global__ __launch_bounds__(GS_THREADS) void k_gs32(const float* __restrict__ Ein, float* __restrict__ Eout,
                                                      const float* __restrict__ W, const float* __restrict__ rhs,
                                                      const float* __restrict__ dts, Grid g, int nk, float omega,
@@ -85,6 +114,20 @@ __global__ __launch_bounds__(GS_THREADS) void k_gs32(const float* __restrict__ E
     }
 }
 #pragma clang fp contract(off)
+
+void launch_tb_weights32(hipStream_t st, Level& L, const FD& F, const Spacing& h)
+{
+    if (!L.w13) {
+        if (hipMalloc((void**)&L.w13, 13 * L.g.elems * sizeof(float)) != hipSuccess) {
+            L.w13 = nullptr;
+            return;
+        }
+    }
+    const GsCoefs C{L.vis32, L.visx32, L.visz32, L.a132, L.visxz32, L.dts32};
+    dim3 b(64, 4);
+    dim3 gr((L.g.nx - 1 + 63) / 64, (L.g.nz - 1 + 3) / 4);
+    hipLaunchKernelGGL(k_tb_weights32, gr, b, 0, st, C, fd32_from(F), h32_from(h), L.g, L.w13);
+}
 
 void launch_gs32(hipStream_t st, const Level& L, const float* rhs, const float* Ein, float* Eout, int nk, double omega,
                  double zsg)

@@ -174,45 +174,18 @@ void launch_sweep32(hipStream_t st, bool use_ratio, const Level& L, const float*
 void launch_residual32(hipStream_t st, const Level& L, const float* S, float* R, const float* rhs, const FD& F,
                        const Spacing& h);
 void launch_restrict32(hipStream_t st, const float* in, const Grid& gi, float* out, const Grid& go);
+// (std_tables: visit_tables(F); the arithmetic of the fused form)
 // with RowB and bout (descent into the coarsest level): also the coarse
 // solve's equilibrated right-hand side, as launch_coarse_apply32 forms it
 void launch_residual_restrict32(hipStream_t st, const Level& Lf, const float* S, const float* rhs, const FD& F,
                                 const Spacing& h, float* out, const Grid& go, const double* RowB = nullptr,
-                                double* bout = nullptr);
+                                double* bout = nullptr, bool std_tables = false);
 void launch_prolong32(hipStream_t st, float* Ef, const Grid& gf, const float* Ec, const Grid& gc, double zsg);
 // b_ready: b already holds the right-hand side (launch_residual_restrict32)
 void launch_coarse_apply32(hipStream_t st, const float* Ainv, const double* RowB, const Level& L, const float* rhs,
                            float* E, int ngc, double zsg, double* b, bool b_ready);
 void launch_to_f32(hipStream_t st, const double* in, float* out, size_t n);
 void launch_coeffs_to_f32(hipStream_t st, Level& L, bool with_lb, int ivis);
-
-// --- tc_tb.hip ------------------------------------------------------------------
-int tb_max_sweeps(int K);
-// levels whose temporally blocked sweeps read precomputed weights (Level::w13)
-bool tb_uses_w13(const Level& L);
-int tb_sweeps_per_launch(const Grid& g);
-void launch_tb_weights32(hipStream_t st, Level& L, const FD& F, const Spacing& h);
-void launch_sweep_tb64(hipStream_t st, bool use_ratio, int K, const Level& L, const double* rhs, const double* S0,
-                       double* E, const FD& F, const Spacing& h, const double* temp, const double* cconst, int nk,
-                       double zsg);
-// The next coarser level's right-hand side, formed at the end of a visit's
-// last blocked launch (what launch_residual_restrict32 would form from the
-// visit's result); RowB/bout as there.
-struct RRTarget {
-    float* out = nullptr;
-    Grid go;
-    const double* RowB = nullptr;
-    double* bout = nullptr;
-    int cus = 256;  // compute units: the fused launch serves levels of at most one tile per CU
-};
-// Pc (optional): a coarse correction on grid *gc to prolong into S0 while
-// staging (the prolongation folded into the visit's first launch).
-// rr (optional): also form rr's right-hand side; returns whether it did
-// (16x16 tiles on levels of at most rr->cus tiles only).
-bool launch_sweep_tb32(hipStream_t st, bool use_ratio, int K, const Level& L, const float* rhs, const float* S0,
-                       float* E, const FD& F, const Spacing& h, const double* temp, const double* cconst, int nk,
-                       double zsg, const float* Pc = nullptr, const Grid* gc = nullptr,
-                       const RRTarget* rr = nullptr);
 
 // --- tc_visit.hip ---------------------------------------------------------------
 // How a level's sweeps are launched: the region of a workgroup (cfg), the
@@ -232,6 +205,34 @@ VisitPlan visit_plan_ref(const Grid& g, int cus);
 void launch_visit_ref(hipStream_t st, const VisitPlan& p, bool pow2, bool use_ratio, const Level& L, const double* rhs,
                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
                       double* res);
+
+// The next coarser level's right-hand side, formed at the end of a visit's
+// last launch (what launch_residual_restrict32 would form from the visit's
+// result); RowB/bout as there.
+struct RRTarget {
+    float* out = nullptr;
+    Grid go;
+    const double* RowB = nullptr;
+    double* bout = nullptr;
+};
+// A visit of the defect-correction cycles: `launches` launches of region cfg
+// that share the sweeps evenly, and with `end` a last one of end_k sweeps of
+// region end_cfg that forms the next right-hand side (whole: the last of
+// the launches does).
+struct Visit13Plan {
+    int cfg = 2, launches = 1;
+    bool whole = false, end = false;
+    int end_cfg = 2, end_k = 0;
+};
+Visit13Plan visit_plan13(const Grid& g, bool f32, int n, bool end, int cus, int only);
+// nk sweeps of the 13-tap form from `in` (nullptr: a zero correction) into
+// `out`; Pc (optional): a coarse correction on grid *gc prolonged into `in`
+// first; rr (optional): also form its right-hand side
+void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const float* rhs,
+                       const float* in, float* out, const Spacing& h, const double* fac, int nk, double zsg,
+                       const float* Pc, const Grid* gc, const RRTarget* rr);
+void launch_visit13_64(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const double* rhs,
+                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg);
 
 // --- tc_fields.hip -------------------------------------------------------------
 void launch_velocities(hipStream_t st, const double* SF, double* u, double* w, const Grid& g, const FD& F, double dr,
@@ -280,6 +281,9 @@ struct CopyList {
 };
 void launch_copy_list(hipStream_t st, const CopyList& L, void* dst);
 void launch_scatter_i32(hipStream_t st, const int32_t* in, const int64_t* id, int32_t* out, int64_t n);
+// (tc_gs.hip) the 13 dt-scaled tap planes of a level's FP32 operator
+// (Level::w13), once per solve
+void launch_tb_weights32(hipStream_t st, Level& L, const FD& F, const Spacing& h);
 // multicolour Gauss-Seidel sweeps of a level's FP32 correction (tc_gs.hip):
 // nk sweeps from Ein into Eout, with the level's 13 dt-scaled tap planes w13
 void launch_gs32(hipStream_t st, const Level& L, const float* rhs, const float* Ein, float* Eout, int nk, double omega,

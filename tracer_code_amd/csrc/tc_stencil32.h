@@ -105,4 +105,38 @@ __device__ __forceinline__ float restrict_fw32(float rmm, float rmp, float rpp, 
 }
 #pragma clang fp contract(off)
 
+// rhs - L(S) of FP32 fields in FP64 with the second-order tables put in
+// (stream_space32_g; the products of FP32 values are exact, the sums round):
+// explicit operations, so that every kernel gets the same bits
+struct Tap13d {
+    double c, xm1, xp1, xm2, xp2, zm1, zp1, zm2, zp2, mm, pm, mp, pp;
+};
+__device__ __forceinline__ float residual32_std(const Tap13d& t, const H32& h, float vis, float vx, float vz, float a1,
+                                                float vxz, float rhs)
+{
+    const double Srr = fma(-2.0, t.c, t.xm1) + t.xp1, Sss = fma(-2.0, t.c, t.zm1) + t.zp1;
+    const double Srrr = fma(0.5, t.xp2, fma(-0.5, t.xm2, t.xm1) - t.xp1);
+    const double Ssss = fma(0.5, t.zp2, fma(-0.5, t.zm2, t.zm1) - t.zp1);
+    const double Srrrr = fma(6.0, t.c, fma(-4.0, t.xm1, t.xm2) + fma(-4.0, t.xp1, t.xp2));
+    const double Sssss = fma(6.0, t.c, fma(-4.0, t.zm1, t.zm2) + fma(-4.0, t.zp1, t.zp2));
+    const double dm = t.mm - t.pm, dp = t.pp - t.mp, sm = t.mm + t.pm, sp = t.pp + t.mp;
+    const double Srs = 0.25 * (dm + dp);
+    const double Srss = fma(0.5, dp - dm, t.xm1 - t.xp1);
+    const double Srrs = fma(0.5, sp - sm, t.zm1 - t.zp1);
+    const double Srrss = fma(-2.0, (t.xm1 + t.xp1) + (t.zm1 + t.zp1), fma(4.0, t.c, sm + sp));
+    double L = (double)a1 * fma(Srr, (double)h.idr2, -(Sss * (double)h.ids2));
+    L = fma((double)vis, fma(Srrrr, (double)h.idr4, Sssss * (double)h.ids4), L);
+    L = fma(2.0 * (double)vis, Srrss * (double)h.idr2ds2, L);
+    L = fma(4.0 * (double)vxz, Srs * (double)h.idrds, L);
+    L = fma(2.0 * (double)vx, fma(Srrr, (double)h.idr3, Srss * (double)h.idrds2), L);
+    L = fma(2.0 * (double)vz, fma(Ssss, (double)h.ids3, Srrs * (double)h.idr2ds), L);
+    return (float)((double)rhs - L);
+}
+template <typename G>
+__device__ __forceinline__ Tap13d taps13(const G& S)
+{
+    return Tap13d{S(0, 0),  S(-1, 0),  S(1, 0),  S(-2, 0), S(2, 0),  S(0, -1), S(0, 1),
+                  S(0, -2), S(0, 2),   S(-1, -1), S(1, -1), S(-1, 1), S(1, 1)};
+}
+
 }  // namespace tc

@@ -26,6 +26,7 @@
 #include <algorithm>
 
 #include "tc_kernels.h"
+#include "tc_stencil32.h"
 
 namespace tc {
 
@@ -49,6 +50,15 @@ __device__ __forceinline__ double from_right(double v)
                             __builtin_amdgcn_mov_dpp(lo, 0x130, 0xF, 0xF, true));
 }
 
+__device__ __forceinline__ float from_left(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float from_right(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xF, 0xF, true));
+}
+
 // ---- geometry ------------------------------------------------------------------
 // The region of tile (X, Y) starts at column 1 + X*tx - hx, row 1 + Y*ty - hz.
 // With tiles, hx and hz are at least 2 per sweep, the same beyond the own
@@ -58,9 +68,11 @@ __device__ __forceinline__ double from_right(double v)
 struct VisitTile {
     int tx, ty, hx, hz;
 };
-struct VisitFactors {
-    double v[VISIT_KMAX];  // the sweep's factor; on the ratio level the cosine that its per-point factor takes
+template <typename T>
+struct VisitFac {
+    T v[VISIT_KMAX];  // the sweep's factor; on the ratio level the cosine that its per-point factor takes
 };
+using VisitFactors = VisitFac<double>;
 
 // The 13 values a sweep at one point reads.
 template <typename T>
@@ -295,16 +307,259 @@ void visit_ref_launch(hipStream_t st, bool ratio, dim3 gr, const double* in, dou
                            sf, nk, zsg, res);
 }
 
+// ---- the 13-tap operator of the defect-correction cycles ---------------------
+// The dt-scaled weights of the 13 taps of one point with the second-order
+// tables put in, from the five coefficients (42 operations, once per launch),
+// and the scaled right-hand side.
+template <typename T>
+struct Cell13 {
+    T c, xm1, xp1, xm2, xp2, zm1, zp1, zm2, zp2, mm, pm, mp, pp, rd;
+};
+template <typename T>
+struct H13 {
+    T idr2, ids2, idr3, ids3, idr4, ids4, idrds, idrds2, idr2ds, idr2ds2;
+};
+template <typename T>
+struct Args13 {
+    const T *vis, *vx, *vz, *a1, *vxx, *vzz, *vxz, *rhs, *dts, *lb;  // FP32: a1, lb; FP64: vxx, vzz, lb = the ratio
+};
+// the next level's right-hand side, formed after the last sweep (FP32); RowB
+// and bout: for the coarsest level, the coarse solve's equilibrated
+// right-hand side too
+struct End13 {
+    float* out;
+    Grid go;
+    const double* RowB;
+    double* bout;
+    H32 h;
+};
+struct Prolong13 {
+    const float* Ec;
+    Grid gc;
+};
+
+template <typename T>
+__device__ __forceinline__ Cell13<T> weights13(T vis, T vx, T vz, T a1, T vxz, T dts, T rhs, const H13<T>& h)
+{
+    const T e = dts * vis, b = T(2) * dts * vx, c = T(2) * dts * vz, a = dts * a1, xq = dts * vxz * h.idrds;
+    const T e4x = e * h.idr4, e4z = e * h.ids4, et = T(2) * e * h.idr2ds2;
+    const T b3 = b * h.idr3, bp = b * h.idrds2, c3 = c * h.ids3, cr = c * h.idr2ds;
+    const T ax = a * h.idr2, az = a * h.ids2;
+    Cell13<T> w;
+    w.xm2 = fma(T(-0.5), b3, e4x);
+    w.xp2 = fma(T(0.5), b3, e4x);
+    w.zm2 = fma(T(-0.5), c3, e4z);
+    w.zp2 = fma(T(0.5), c3, e4z);
+    const T mx = fma(T(-2), et, fma(T(-4), e4x, ax)), bx = b3 + bp;
+    w.xm1 = mx + bx;
+    w.xp1 = mx - bx;
+    const T mz = fma(T(-2), et, fma(T(-4), e4z, -az)), cz = c3 + cr;
+    w.zm1 = mz + cz;
+    w.zp1 = mz - cz;
+    w.c = fma(T(4), et, fma(T(6), e4x + e4z, T(2) * (az - ax)));
+    const T d1 = et + xq, d2 = et - xq, s1 = T(0.5) * (bp + cr), s2 = T(0.5) * (bp - cr);
+    w.mm = d1 - s1;
+    w.pp = d1 + s1;
+    w.pm = d2 + s2;
+    w.mp = d2 - s2;
+    w.rd = dts * rhs;
+    return w;
+}
+
+// 1/x of the per-point factor (1 <= x <= 5): the hardware's reciprocal with a
+// Newton step, which rounds to within an ulp of the quotient
+__device__ __forceinline__ float recip(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fma(fma(-x, r, 1.0f), r, r);
+}
+__device__ __forceinline__ double recip(double x) { return 1.0 / x; }
+
+// dts (rhs - L(S)): three chains of FMAs
+template <typename T>
+__device__ __forceinline__ T step13(const Taps<T>& t, const Cell13<T>& w)
+{
+    T a = fma(-w.c, t.c, w.rd);
+    T b = -w.xm1 * t.xm1;
+    T d = -w.mm * t.mm;
+    a = fma(-w.zm1, t.zm1, a);
+    b = fma(-w.xp1, t.xp1, b);
+    d = fma(-w.pm, t.pm, d);
+    a = fma(-w.zp1, t.zp1, a);
+    b = fma(-w.xm2, t.xm2, b);
+    d = fma(-w.mp, t.mp, d);
+    a = fma(-w.zm2, t.zm2, a);
+    b = fma(-w.xp2, t.xp2, b);
+    d = fma(-w.pp, t.pp, d);
+    a = fma(-w.zp2, t.zp2, a);
+    return a + (b + d);
+}
+
+// Bound: the launch and the loads (3.4 us with a 32x32 region of one row a
+// lane, of which 256 fit the chip), then 0.2 us a sweep (about 25
+// instructions a point and the barrier); on the levels of more tiles, the
+// loads of the staged cells (32 B each, FP32).
+// END: after the last sweep, FP32: the residual in FP64 of the held cells and
+// its restriction to the next level (residual32_std, restrict_fw32: the
+// values of k_residual_restrict32), for which the region reaches 2 cells
+// before and 3 behind the own ones.
+template <typename T, bool RATIO, int LW, int R, int NW, bool END>
+__global__ __launch_bounds__(NW * 64) void k_visit13(const T* __restrict__ Ein, T* __restrict__ Eout, Args13<T> A,
+                                                     Grid g, H13<T> h, VisitTile vt, VisitFac<T> sf, int nk, T zsg,
+                                                     Prolong13 pr, End13 en)
+{
+    constexpr int GR = 64 / LW, ROWS = NW * GR * R;
+    __shared__ T buf[2][ROWS * LW];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane % LW, row0 = (wv * GR + lane / LW) * R;
+    const int2 tile = xcd_tile();
+    const int i0 = 1 + tile.x * vt.tx - vt.hx, kg = 1 + tile.y * vt.ty - vt.hz;  // the region's origin
+    const int i = i0 + li, k0 = kg + row0;
+    const bool col = i >= 1 && i <= g.nx - 1;
+    T S[R];
+    Cell13<T> q[R];
+    T lb[RATIO ? R : 1];
+    float rc[END ? R : 1][6];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int k = k0 + r;
+        const bool in = col && k >= 1 && k <= g.nz - 1;
+        const size_t c = g.at(in ? i : 1, in ? k : 1);
+        S[r] = Ein ? Ein[c] : T(0);
+        const T vis = A.vis[c], vx = A.vx[c], vz = A.vz[c], vxz = A.vxz[c], dts = A.dts[c], rhs = A.rhs[c];
+        T a1;
+        if constexpr (sizeof(T) == 4) a1 = A.a1[c];
+        else a1 = A.vxx[c] - A.vzz[c];
+        if constexpr (sizeof(T) == 4) {
+            // the coarse correction prolonged into this level (prolong_add32, its
+            // four sources loaded by every thread and the parity's value selected)
+            if (pr.Ec) {
+                const int pi = in ? i : 1, pk = in ? k : 1;
+                const int c0 = pi >> 1, c1 = (pi + 1) >> 1, d0 = pk >> 1, d1 = (pk + 1) >> 1;
+                const float e00 = pr.Ec[pr.gc.at(c0, d0)], e10 = pr.Ec[pr.gc.at(c1, d0)];
+                const float e11 = pr.Ec[pr.gc.at(c1, d1)], e01 = pr.Ec[pr.gc.at(c0, d1)];
+                const bool ie = (pi & 1) == 0, ke = (pk & 1) == 0;
+                const float two = __fmul_rn(__fadd_rn(e00, ie ? e01 : e10), 0.5f);
+                const float four = __fmul_rn(__fadd_rn(__fadd_rn(__fadd_rn(e00, e10), e11), e01), 0.25f);
+                S[r] = __fadd_rn(S[r], (ie && ke) ? e00 : ((ie || ke) ? two : four));
+            }
+        }
+        if (!in) S[r] = T(0);
+        q[r] = weights13<T>(vis, vx, vz, a1, vxz, in ? dts : T(0), rhs, h);
+        if constexpr (END) { rc[r][0] = vis; rc[r][1] = vx; rc[r][2] = vz; rc[r][3] = a1; rc[r][4] = vxz; rc[r][5] = rhs; }
+        if constexpr (RATIO) {
+            if constexpr (sizeof(T) == 4) {
+                lb[r] = in ? A.lb[c] : T(-2);
+            } else {
+                const T a = A.lb[c];
+                lb[r] = (!in || a > T(1e99)) ? T(-2) : T(-2) * (a * a) / (T(1) + a * a);
+            }
+        }
+    }
+    const bool wl = i == 1, wr = i == g.nx - 1;
+    const bool sides = i0 <= 1 || i0 + LW > g.nx - 1;
+    const int w0 = wv * GR * R, w1 = w0 + GR * R - 1;
+    auto gather = [&](const T* __restrict__ b, T (&v)[R + 4], T (&lf)[R + 2], T (&rt)[R + 2]) {
+        const int up = row0 * LW + li;
+        v[0] = row0 >= 2 ? b[up - 2 * LW] : T(0);
+        v[1] = row0 >= 1 ? b[up - LW] : T(0);
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r + 2] = S[r];
+        v[R + 2] = row0 + R < ROWS ? b[up + R * LW] : T(0);
+        v[R + 3] = row0 + R + 1 < ROWS ? b[up + (R + 1) * LW] : T(0);
+#pragma unroll
+        for (int r = 0; r < R + 2; ++r) {
+            lf[r] = from_left(v[r + 1]);
+            rt[r] = from_right(v[r + 1]);
+        }
+    };
+    auto taps = [&](int r, const T (&v)[R + 4], const T (&lf)[R + 2], const T (&rt)[R + 2]) {
+        Taps<T> t;
+        t.c = v[r + 2];
+        t.zm1 = v[r + 1]; t.zp1 = v[r + 3]; t.zm2 = v[r]; t.zp2 = v[r + 4];
+        t.xm1 = lf[r + 1]; t.xp1 = rt[r + 1];
+        t.mm = lf[r]; t.pm = rt[r]; t.mp = lf[r + 2]; t.pp = rt[r + 2];
+        t.xm2 = from_left(t.xm1); t.xp2 = from_right(t.xp1);
+        if (sides) {
+            t.xm2 = wl ? -t.c : t.xm2;
+            t.xp2 = wr ? -t.c : t.xp2;
+        }
+        if (k0 + r == 1) t.zm2 = zsg * t.c;
+        if (k0 + r == g.nz - 1) t.zp2 = zsg * t.c;
+        return t;
+    };
+#pragma unroll 1
+    for (int s = 0; s < nk; ++s) {
+        T* __restrict__ b = buf[s & 1];
+#pragma unroll
+        for (int r = 0; r < R; ++r) b[(row0 + r) * LW + li] = S[r];
+        __syncthreads();
+        const int ext = 2 * (nk - 1 - s);
+        const int lo = max(vt.hz - ext - (END ? 2 : 0), 1 - kg);
+        const int hi = min(vt.hz + vt.ty - 1 + ext + (END ? 3 : 0), g.nz - 1 - kg);
+        if (w1 < lo || w0 > hi) continue;
+        T v[R + 4], lf[R + 2], rt[R + 2];
+        gather(b, v, lf, rt);
+        const T f = sf.v[s];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            T cc = f;
+            if constexpr (RATIO) cc = T(2) * recip(-lb[r] + T(1) + (lb[r] + T(1)) * f);
+            S[r] = fma(cc, step13(taps(r, v, lf, rt), q[r]), S[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int rr = row0 + r, k = k0 + r;
+        if (li >= vt.hx && li < vt.hx + vt.tx && rr >= vt.hz && rr < vt.hz + vt.ty && col && k >= 1 && k <= g.nz - 1) {
+            Eout[g.at(i, k)] = S[r];
+            stream_ghosts(Eout, g, i, k, S[r], zsg);
+        }
+    }
+    if constexpr (END) {
+        T* __restrict__ b = buf[nk & 1];
+#pragma unroll
+        for (int r = 0; r < R; ++r) b[(row0 + r) * LW + li] = S[r];
+        __syncthreads();
+        T v[R + 4], lf[R + 2], rt[R + 2];
+        gather(b, v, lf, rt);
+        float* __restrict__ res = reinterpret_cast<float*>(buf[1 - (nk & 1)]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const Taps<T> t = taps(r, v, lf, rt);
+            const Tap13d d{t.c, t.xm1, t.xp1, t.xm2, t.xp2, t.zm1, t.zp1, t.zm2, t.zp2, t.mm, t.pm, t.mp, t.pp};
+            res[(row0 + r) * LW + li] =
+                residual32_std(d, en.h, rc[r][0], rc[r][1], rc[r][2], rc[r][3], rc[r][4], rc[r][5]);
+        }
+        __syncthreads();
+        const int ncx = vt.tx / 2, ncz = vt.ty / 2;
+        for (int e = threadIdx.x; e < ncx * ncz; e += NW * 64) {
+            const int ic = tile.x * ncx + 1 + e % ncx, kc = tile.y * ncz + 1 + e / ncx;
+            if (ic > en.go.nx - 1 || kc > en.go.nz - 1) continue;
+            const int p = (2 * kc - kg) * LW + 2 * ic - i0;  // the fine centre
+            const float x = restrict_fw32(res[p - LW - 1], res[p + LW - 1], res[p + LW + 1], res[p - 1], res[p - LW],
+                                          res[p + 1], res[p + LW], res[p]);
+            en.out[en.go.at(ic, kc)] = x;
+            if (en.bout) {
+                const int u = ic * (en.go.nz + 1) + kc;
+                en.bout[u] = (double)x * en.RowB[u];
+            }
+        }
+    }
+}
+
 // one tile holds the interior: no halo
 VisitTile whole_tile(const Grid& g) { return VisitTile{g.nx - 1, g.nz - 1, 0, 0}; }
 
 // tiles of a region of w by r cells for nk sweeps; an axis that the region
-// spans needs no halo
-VisitTile tiles_for(const Grid& g, int w, int r, int nk)
+// spans needs no halo.  end: room for the residual and its restriction (an
+// even number of own cells, so that a coarse point's centre is its tile's)
+VisitTile tiles_for(const Grid& g, int w, int r, int nk, bool end = false)
 {
     VisitTile t = whole_tile(g);
-    if (g.nx > w) { t.hx = 2 * nk; t.tx = w - 4 * nk; }
-    if (g.nz - 1 > r) { t.hz = 2 * nk; t.ty = r - 4 * nk; }
+    const int lo = 2 * nk + (end ? 2 : 0), hi = 2 * nk + (end ? 3 : 0);
+    if (g.nx > w) { t.hx = lo; t.tx = w - lo - hi; if (end) t.tx &= ~1; }
+    if (g.nz - 1 > r) { t.hz = lo; t.ty = r - lo - hi; if (end) t.ty &= ~1; }
     return t;
 }
 dim3 tile_grid(const Grid& g, const VisitTile& t)
@@ -396,6 +651,188 @@ void launch_visit_ref(hipStream_t st, const VisitPlan& p, bool pow2, bool use_ra
     };
     if (pow2) go(std::integral_constant<bool, true>{});
     else go(std::integral_constant<bool, false>{});
+}
+
+// ---- plans of the 13-tap sweeps ---------------------------------------------------
+// The regions: columns, rows; the last three take tiles.
+//   0: 16x16 (4 waves of 4 row groups, 1 row a lane)     whole levels
+//   4: 64x16 (16 waves, 1 row)                            whole levels
+//   1: 64x32 (16 waves, 2 rows)                           whole levels, tiles
+//   2: 32x32 (16 waves of 2 row groups, 1 row)            whole levels, tiles
+//   3: 64x32 (8 waves, 4 rows), FP32; 64x48 (16 waves, 3 rows), FP64     tiles
+static VisitRegion region13(int cfg, bool f32)
+{
+    switch (cfg) {
+    case 0: return {16, 16};
+    case 1: return {64, 32};
+    case 2: return {32, 32};
+    case 3: return f32 ? VisitRegion{64, 32} : VisitRegion{64, 48};
+    default: return {64, 16};
+    }
+}
+
+// The time of a launch as measured on 16x16 to 2048x1024 cells, within about
+// 10%: a part for the launch and its loads, one per sweep, and one per 256
+// tiles beyond the first 256.  us, FP32 (FP64):
+//   32x32 regions   3.4 + 0.2 k, then 1.8      (3.4 + 0.38 k, then 1.9)
+//   64x32, 16 waves 4.0 + 0.35 k, then 2.9     (4.6 + 0.5 k, then 7)
+//   region 3        4.6 + 0.35 k, then 2.2     (5.5 + 0.8 k, then 7)
+// The residual and restriction after the last sweep add 1.4 us, 1.9 in the
+// 64-column regions, and (a second round of their larger state) 5 per 256
+// further tiles; apart (k_residual_restrict32) they take 4.4 us and 5.4 us
+// per million points.
+static double cost13(int cfg, bool f32, int k, double tiles, int cus, bool end)
+{
+    const double more = std::max(0.0, tiles / cus - 1.0);
+    double c;
+    if (cfg == 2) c = f32 ? 3.4 + 0.2 * k + 1.8 * more : 3.4 + 0.38 * k + 1.9 * more;
+    else if (cfg == 1) c = f32 ? 4.0 + 0.35 * k + 2.9 * more : 4.6 + 0.5 * k + 7.0 * more;
+    else c = f32 ? 4.6 + 0.35 * k + 2.2 * more : 5.5 + 0.8 * k + 7.0 * more;
+    if (end) c += (cfg == 2 ? 1.4 : 1.9) + 5.0 * more;
+    return c;
+}
+
+// The launches of a visit of n sweeps.  A level that a region holds runs them
+// (and the residual, with end) in one launch, 8 sweeps (with end): 16x16 4.2
+// us (4.8), 32x32 5.7 (6.8), 64x16 5.6 (6.7), 64x32 7.6 (9.7; as tiles 8.7 and
+// 10.2).  Else the cheapest, by cost13, of launches that share the sweeps
+// evenly and, with end, a last one of 1 to 4 that forms the next right-hand
+// side too.  us a visit of 8 sweeps (before: k_sweep_tb, 4 sweeps a launch),
+// with the residual and restriction: 128x64 9.7 (15.0), 256x128 10.3 (14.6),
+// 512x256 14.7 (21.3); 16 sweeps of 1024x512 44 (85); 10 of 2048x1024, none:
+// 69 (127 as ten launches of one sweep).  only: 0, or the region that
+// tc_set_tb_tile asks for.
+Visit13Plan visit_plan13(const Grid& g, bool f32, int n, bool end, int cus, int only)
+{
+    Visit13Plan p;
+    if (!only)
+        for (int c : {0, 4, 2, 1}) {
+            const VisitRegion rg = region13(c, f32);
+            if (g.nx <= rg.w && g.nz - 1 <= rg.r && (c != 1 || n >= 8)) {
+                p.cfg = p.end_cfg = c;
+                p.whole = true;
+                p.launches = (n + VISIT_KMAX - 1) / VISIT_KMAX;
+                p.end = end;
+                return p;
+            }
+        }
+    auto cost = [&](int c, int k, bool e) {
+        const VisitRegion rg = region13(c, f32);
+        const VisitTile t = tiles_for(g, rg.w, rg.r, k, e);
+        if (t.tx < 2 || t.ty < 2) return 1e30;
+        const dim3 gr = tile_grid(g, t);
+        return cost13(c, f32, k, (double)gr.x * gr.y, cus, e);
+    };
+    // n sweeps shared by m launches of region c
+    auto shared = [&](int c, int sweeps, int m) {
+        if (m == 0) return 0.0;
+        const int k = sweeps / m, more = sweeps - k * m;  // `more` launches of k + 1, the others of k
+        return more * (more ? cost(c, k + 1, false) : 0.0) + (m - more) * cost(c, k, false);
+    };
+    double best = 1e30;
+    const double apart = end ? 4.4 + 5.4e-6 * (double)g.nx * g.nz : 0.0;
+    for (int c = 1; c < 4; ++c) {
+        if (only && c != only) continue;
+        for (int k = 1; k <= 7; ++k) {
+            if (cost(c, k, false) > 1e29) continue;
+            const int m = (n + k - 1) / k;
+            const double all = shared(c, n, m) + apart;
+            if (all < best) {
+                best = all;
+                p.cfg = c;
+                p.launches = m;
+                p.end = false;
+            }
+            if (!end) continue;
+            for (int ke = 1; ke <= 4 && ke <= n; ++ke) {
+                const int me = (n - ke + k - 1) / k;
+                const double body = shared(c, n - ke, me);
+                for (int ce = 1; ce < 4; ++ce) {
+                    const double t = body + cost(ce, ke, true);
+                    if (t < best) {
+                        best = t;
+                        p.cfg = c;
+                        p.launches = me;
+                        p.end = true;
+                        p.end_cfg = ce;
+                        p.end_k = ke;
+                    }
+                }
+            }
+        }
+    }
+    return p;
+}
+
+namespace {
+
+template <typename T>
+H13<T> h13_from(const Spacing& h)
+{
+    return H13<T>{(T)h.idr2, (T)h.ids2, (T)h.idr3, (T)h.ids3, (T)h.idr4,
+                  (T)h.ids4, (T)h.idrds, (T)h.idrds2, (T)h.idr2ds, (T)h.idr2ds2};
+}
+
+template <typename T, int LW, int R, int NW>
+void visit13_go(hipStream_t st, dim3 gr, bool ratio, bool end, const T* in, T* out, const Args13<T>& A, const Grid& g,
+                const H13<T>& h, const VisitTile& vt, const VisitFac<T>& sf, int nk, T zsg, const Prolong13& pr,
+                const End13& en)
+{
+    const dim3 b(NW * 64);
+    if constexpr (sizeof(T) == 4) {
+        if (end) {
+            if (ratio) hipLaunchKernelGGL((k_visit13<T, true, LW, R, NW, true>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
+            else hipLaunchKernelGGL((k_visit13<T, false, LW, R, NW, true>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
+            return;
+        }
+    }
+    if (ratio) hipLaunchKernelGGL((k_visit13<T, true, LW, R, NW, false>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
+    else hipLaunchKernelGGL((k_visit13<T, false, LW, R, NW, false>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
+}
+
+template <typename T>
+void launch13(hipStream_t st, int cfg, bool whole, bool ratio, bool end, const Args13<T>& A, const Grid& g,
+              const Spacing& h, const T* in, T* out, const double* fac, int nk, double zsg, const Prolong13& pr,
+              const End13& en)
+{
+    VisitFac<T> sf;
+    for (int s = 0; s < nk; ++s) sf.v[s] = (T)fac[s];
+    const VisitRegion rg = region13(cfg, sizeof(T) == 4);
+    const VisitTile vt = whole ? whole_tile(g) : tiles_for(g, rg.w, rg.r, nk, end);
+    const dim3 gr = tile_grid(g, vt);
+    const H13<T> hh = h13_from<T>(h);
+    const T z = (T)zsg;
+    switch (cfg) {
+    case 0: visit13_go<T, 16, 1, 4>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en); break;
+    case 1: visit13_go<T, 64, 2, 16>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en); break;
+    case 2: visit13_go<T, 32, 1, 16>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en); break;
+    case 4: visit13_go<T, 64, 1, 16>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en); break;
+    default:
+        if constexpr (sizeof(T) == 4) visit13_go<T, 64, 4, 8>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en);
+        else visit13_go<T, 64, 3, 16>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en);
+        break;
+    }
+}
+
+}  // namespace
+
+void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const float* rhs,
+                       const float* in, float* out, const Spacing& h, const double* fac, int nk, double zsg,
+                       const float* Pc, const Grid* gc, const RRTarget* rr)
+{
+    const Args13<float> A{L.vis32, L.visx32, L.visz32, L.a132, nullptr, nullptr, L.visxz32, rhs, L.dts32, L.lb32};
+    Prolong13 pr{nullptr, L.g};
+    if (Pc) { pr.Ec = Pc; pr.gc = *gc; }
+    End13 en{};
+    if (rr) { en.out = rr->out; en.go = rr->go; en.RowB = rr->RowB; en.bout = rr->bout; en.h = h32_from(h); }
+    launch13<float>(st, cfg, whole, use_ratio, rr != nullptr, A, L.g, h, in, out, fac, nk, zsg, pr, en);
+}
+
+void launch_visit13_64(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const double* rhs,
+                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg)
+{
+    const Args13<double> A{L.vis, L.visx, L.visz, nullptr, L.visxx, L.viszz, L.visxz, rhs, L.dtstream, L.ratio};
+    launch13<double>(st, cfg, whole, use_ratio, false, A, L.g, h, in, out, fac, nk, zsg, Prolong13{nullptr, L.g}, End13{});
 }
 
 }  // namespace tc
