@@ -1,0 +1,40 @@
+"""The C filter's tiles (k_filter_multi) against one launch per iteration, on
+fields that the tracers do not give: random ratios, values beyond [0,1] (the
+clamp) and a NaN, at the heights and widths where a tile ends -- the
+smallest height with tiles, a last tile that overlaps the one before it, one
+column or row more than a tile, every tile height.  Same iterates, stop
+and bits."""
+import numpy as np
+import pytest
+
+from tracer_code_amd import Solver, config
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind", ["ratio", "beyond", "nan"])
+@pytest.mark.parametrize("nx,nz", [(16, 18), (24, 16), (54, 20), (56, 38), (108, 50), (110, 26), (160, 96), (212, 130),
+                                   (1024, 512), (1920, 992)])
+def test_filter_tiles_same_bits(nx, nz, kind):
+    if nx > 1000 and kind != "ratio":
+        pytest.skip("the walls' handling does not depend on the size")
+    params = config.make_params(nx=nx, nz=nz, aspect=nx / nz, grids=2 if nx < 1000 else 6, ivis=2, visC=(1.0 / 30.0,), delta_visC=(1.5,))
+    print(f"[filter tiles] {params.nx}x{params.nz} {kind}", flush=True)
+    assert (params.nx, params.nz) == (nx, nz)
+    rng = np.random.default_rng(nx * 7 + nz)
+    C = rng.integers(0, 21, (nz + 5, nx + 5, 1)) / 20.0
+    if kind == "beyond":
+        C[rng.random(C.shape) < 0.1] = 1.5
+        C[rng.random(C.shape) < 0.1] = -0.25
+    if kind == "nan":
+        C[nz // 2, nx // 2] = np.nan
+    out = []
+    with Solver(params, 0) as g:
+        for blocking in (False, True):
+            g.set_filter_blocking(blocking)
+            g.put("Cnew", C)
+            n0 = g.stats().c_iters
+            n = g.smoother_time()
+            out.append((g.get("Cvis"), n, g.stats().c_iters - n0))
+    assert out[0][1] == out[1][1] and out[0][2] == out[1][2] and out[0][2] > 4
+    assert np.array_equal(out[0][0], out[1][0], equal_nan=True)

@@ -282,12 +282,12 @@ __global__ __launch_bounds__(256) void k_filter_iter(const double* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // Several iterations of smoother_time's C filter per launch, with the
-// iterates held in registers.  Each wavefront owns a tile of FM_TXO x FM_TY
+// iterates held in registers.  Each wavefront owns a tile of FM_TXO x TY
 // cells of the ghosted plane and holds it with a halo of FM_H = K+1 cells:
-// 64 columns, one per lane, by FM_RY rows in the lane's registers.  An
+// 64 columns, one per lane, by TY + 2 FM_H rows in the lane's registers.  An
 // iteration updates the held rows from the previous iterate -- the step at
 // every interior node with the left/right values from the neighbouring
-// lanes (cross-lane shuffles) and the upper/lower ones from the lane's own
+// lanes (cross-lane shifts) and the upper/lower ones from the lane's own
 // rows -- then applies enforceBCs_comp: ghost columns copy the lane they
 // mirror, ghost rows the row they mirror, and the row-1 corner cells
 // (-2 or nx+2, -1 or nz+1) the previous iterate's value at row 1 (nz-1), as
@@ -296,10 +296,15 @@ __global__ __launch_bounds__(256) void k_filter_iter(const double* __restrict__ 
 // of the held region shrinks by one cell per iteration; the halo keeps the
 // tile valid through K iterations and the last iterate's measure.  A ghost
 // takes the step at the cell it mirrors, so a tile starting right of the
-// last interior column (or above the last interior row) holds its region
-// shifted inward by the shortfall.  dts_array is one value on the uniform
-// grids the library accepts.  After each iteration the tile's own nodes give
-// that iterate's smoothness maximum (one slot set per iterate).
+// last interior column holds its region shifted inward by the shortfall.
+// In z the first tile starts at the ghost row -2 and the last one ends at
+// nz+2, the tiles between hold no ghost row (the last of them is moved up
+// where it would, and cells that two tiles own get the same value from
+// both): the ghost rows are then fixed registers of the first and the last
+// tile, and the others have no row test at all.  dts_array is one value on
+// the uniform grids the library accepts.  After each iteration the tile's
+// own nodes give that iterate's smoothness maximum, reduced over the block
+// once per launch (one slot set per iterate).
 //
 // The stop test needs the whole grid's maximum, which a launch only sees
 // for the iterates of the launch before it.  Launch l (iterate m = input)
@@ -310,6 +315,12 @@ __global__ __launch_bounds__(256) void k_filter_iter(const double* __restrict__ 
 // (0,0) records the stop, the stopping iterate and the buffer holding it.
 // Slot sets: 3K, set j mod 3K for iterate j; a launch reads K, writes K and
 // clears the K its successor writes.
+//
+// Bound: FP64 issue (13 instructions a held cell and 10 a measured one per
+// iteration, 4 cycles each) and the halo (26 of 64x26 held cells are own).
+// Measured per launch of 4 iterations, against a form that tested every row
+// against the walls and reduced over the block in every iteration (2500
+// instructions an iteration): FILTER_FIGURES
 // ---------------------------------------------------------------------------
 // a double from lane l-1 (wave_shr:1) or lane l+1 (wave_shl:1) of the
 // wavefront, as DPP moves of its two halves; lane 0 (63) gets 0
@@ -329,24 +340,124 @@ __device__ __forceinline__ double dpp_from_right(double v)
 constexpr int FM_K = 4;                  // iterations per launch
 constexpr int FM_H = FM_K + 1;           // halo: one cell per iteration, one for the last measure
 constexpr int FM_TXO = 64 - 2 * FM_H;    // own columns of a wavefront's tile
-constexpr int FM_TY = 16;                // own rows
-constexpr int FM_RY = FM_TY + 2 * FM_H;  // held rows
 constexpr int FM_WAVES = 4;              // tiles (stacked in z) per workgroup
 constexpr int FM_SETS = 3 * FM_K;
+constexpr int FM_TYS[4] = {8, 11, 16, 21};  // own rows of a tile, chosen by the grid's size
 
 struct FmFac { double v[2 * FM_K]; };    // factors of the previous launch's iterations, then this one's
 struct FmBufs { double* v[3]; };
 
-// FAST: dr^2 and ds^2 are powers of two and D2 is (1, -2, 1) at offsets
-// -1, 0, 1 (the second-order table); the products by 1 and -2 are then exact
-// and are left out, and the quotients are products by the reciprocals: the
-// same bits as the general form.
-template <bool FAST>
+// tiles of TY own rows over rows -SPAN..nz+SPAN: the first from -SPAN, the
+// last up to nz+SPAN, and those between without a ghost row in their halo
+__host__ __device__ inline int fm_tiles(int nz, int TY)
+{
+    const int between = nz - FM_H + 1 - (TY - SPAN);  // rows TY-SPAN .. nz-FM_H
+    return 2 + (between > 0 ? (between + TY - 1) / TY : 0);
+}
+__host__ __device__ inline int fm_tile_row(int nz, int TY, int t, int tiles)
+{
+    if (t == tiles - 1) return nz + SPAN + 1 - TY;
+    const int k = -SPAN + t * TY, last = nz - FM_H - TY + 1;
+    return (t > 0 && k > last) ? last : k;
+}
+
+// One tile's n iterations.  ZK: 0 = no ghost rows held, 1 = the first tile,
+// 2 = the last.  D2 is (1, -2, 1) at offsets -1, 0, 1 (the second-order
+// table): the products by 1 and -2 are exact.  POW2: dr^2 and ds^2 are powers
+// of two, so that the quotients are exact scalings and go into the sum's FMA;
+// else they are divisions.  The values are filter_new's, bit for bit.
+template <bool POW2, int TY, int ZK>
+__device__ __forceinline__ void fm_iterate(double (&c)[TY + 2 * FM_H], double (&mx)[FM_K], int n, bool measure,
+                                           const double* fac, double dtc, const FScale& sc, bool gcols, bool ghost_col,
+                                           bool corner_col, int ml, bool own_col)
+{
+    constexpr int RY = TY + 2 * FM_H;
+    constexpr int R0 = FM_H + SPAN;            // row 0 in the first tile
+    constexpr int RN = TY + FM_H - SPAN - 1;   // row nz in the last tile
+    // rows measured: 1..nz-1 of the own ones
+    constexpr int RA = ZK == 1 ? R0 + 1 : FM_H, RB = ZK == 2 ? RN - 1 : FM_H + TY - 1;
+#pragma unroll 1
+    for (int it = 0; it < n; ++it) {
+        const double cfd = fac[it] * dtc;
+        const double old1 = ZK == 1 ? c[R0 + 1] : (ZK == 2 ? c[RN - 1] : 0.0);
+        // the step (filter_new's operation order) on every held row but the
+        // first and last; ghost cells are overwritten below, cells outside
+        // the plane are never read by the valid part of the region
+        double om = c[0];
+        bool out = false;  // a value beyond [0,1]: the clamp has work
+#pragma unroll
+        for (int r = 1; r < RY - 1; ++r) {
+            const double oc = c[r];
+            const double lf = dpp_from_left(oc), rt = dpp_from_right(oc);
+            const double x = fma(-2.0, oc, lf) + rt, z = fma(-2.0, oc, om) + c[r + 1];
+            double temp;
+            if constexpr (POW2) temp = fma(x, sc.idr2, z * sc.ids2);
+            else temp = div_by(x, sc.dr2, sc.idr2) + div_by(z, sc.ds2, sc.ids2);
+            const double v = oc + cfd * temp;
+            // 0 <= v <= 1 by the bits (a negative or NaN value is above 1's)
+            out = out || (unsigned long long)__double_as_longlong(v) > 0x3FF0000000000000ull;
+            c[r] = v;
+            om = oc;
+        }
+        if (__any(out)) {
+#pragma unroll
+            for (int r = 1; r < RY - 1; ++r) {
+                double v = c[r];
+                if (v < 0.0) v = 0.0;
+                if (v > 1.0) v = 1.0;
+                c[r] = v;
+            }
+        }
+        // ghost columns: the mirrored lane's new value (ghost rows are
+        // overwritten next)
+        if (gcols) {
+#pragma unroll
+            for (int r = 1; r < RY - 1; ++r) {
+                const double mv = __shfl(c[r], ml, 64);
+                c[r] = ghost_col ? mv : c[r];
+            }
+        }
+        // ghost rows: the mirrored row (columns already mirrored), the row-1
+        // corners from the previous iterate
+        if constexpr (ZK == 1) {
+            c[R0 - 1] = corner_col ? old1 : c[R0 + 1];
+            c[R0 - 2] = c[R0 + 2];
+        }
+        if constexpr (ZK == 2) {
+            c[RN + 1] = corner_col ? old1 : c[RN - 1];
+            c[RN + 2] = c[RN - 2];
+        }
+        if (measure) {
+            // the new iterate's smoothness over the tile's own nodes of rows
+            // 1..nz-1: the jumps of smooth_merge, each vertical pair once
+            // (node r's jump up is node r-1's jump down, |x-y| = |y-x|); the
+            // maximum is that of smooth_merge
+            double a = fabs(c[RA - 1] - c[RA]), b = 0.0;
+            double rm = dpp_from_right(c[RA - 1]), r0 = dpp_from_right(c[RA]);  // the right lane's c[r-1], c[r]
+#pragma unroll
+            for (int r = RA; r <= RB; ++r) {
+                const double rp = dpp_from_right(c[r + 1]);
+                a = fmax(a, fabs(rm - c[r]));
+                b = fmax(b, fabs(r0 - c[r]));
+                a = fmax(a, fabs(c[r + 1] - c[r]));
+                b = fmax(b, fabs(rp - c[r]));
+                rm = r0;
+                r0 = rp;
+            }
+            a = own_col ? fmax(fmax(a, b), 0.0) : 0.0;
+#pragma unroll
+            for (int j = 0; j < FM_K; ++j) mx[j] = j == it ? a : mx[j];
+        }
+    }
+}
+
+template <bool POW2, int TY>
 __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, const double* __restrict__ dts, Grid g,
-                                                      FD F, FScale sc, double courant, FmFac fac, int m,
-                                                      double delta, unsigned long long* __restrict__ slots,
+                                                      FScale sc, double courant, FmFac fac, int m, double delta,
+                                                      int tiles, unsigned long long* __restrict__ slots,
                                                       int32_t* __restrict__ ctl)
 {
+    constexpr int RY = TY + 2 * FM_H;
     // ctl[0] = m+1 marks the stop taken by the launch with input iterate m:
     // the later launches return, the blocks of that launch still do its work
     {
@@ -354,6 +465,7 @@ __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, con
         if (s != 0 && s != m + 1) return;
     }
     __shared__ int s_j0;
+    __shared__ double s_mx[FM_WAVES][FM_K];
     const int lane = threadIdx.x, tid = threadIdx.y * 64 + lane;
     // the stop test on the iterates the previous launch produced (or the
     // input): the first wave reads one slot per lane of each set and takes
@@ -382,141 +494,66 @@ __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, con
     const int n = replay ? j0 - (m - FM_K) : FM_K;
     const double* __restrict__ src = replay ? bufs.v[b_prev] : bufs.v[b_in];
     double* __restrict__ dst = bufs.v[b_out];
-    const int fo = replay ? 0 : FM_K;  // factor offset
     if (!replay && first && tid < FILT_SLOTS)
         for (int j = m + FM_K + 1; j <= m + 2 * FM_K; ++j)
             slots[(size_t)(j % FM_SETS) * FILT_SET + tid * FILT_STRIDE] = 0ull;
     const int nx = g.nx, nz = g.nz;
-    const int wy = __builtin_amdgcn_readfirstlane(threadIdx.y);  // the wave's tile (uniform)
-    const int i0 = blockIdx.x * FM_TXO - SPAN, k0 = (blockIdx.y * FM_WAVES + wy) * FM_TY - SPAN;
-    const int sx = i0 - nx + 1 > 0 ? i0 - nx + 1 : 0, sk = k0 - nz + 1 > 0 ? k0 - nz + 1 : 0;
-    const int ri0 = i0 - FM_H - sx, rk0 = k0 - FM_H - sk;  // held region origin
-    const int i = ri0 + lane;                               // this lane's column
-    const bool col_in = i >= -SPAN && i <= nx + SPAN, col_int = i >= 0 && i <= nx;
-    const bool corner_col = i == -SPAN || i == nx + SPAN;
-    const int im = (i < 0) ? -i : (i > nx ? 2 * nx - i : i);
-    int ml = lane + (im - i);                               // lane holding the mirrored column
-    ml = ml < 0 ? 0 : (ml > 63 ? 63 : ml);
-    const double dtc = dts[g.at(0, 0)] * courant;
-    double c[FM_RY];
+    const int wy = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int t = blockIdx.y * FM_WAVES + wy;  // the wave's tile (uniform)
+    double mx[FM_K];
 #pragma unroll
-    for (int r = 0; r < FM_RY; ++r) {
-        const int k = rk0 + r;
-        c[r] = (col_in && k >= -SPAN && k <= nz + SPAN) ? src[g.at(i, k)] : 0.0;
-    }
-    const bool ghost_col = col_in && !col_int;
-    const bool gcols = ri0 <= -1 || ri0 + 63 >= nx + 1;  // the held columns include ghost columns (uniform)
-    const bool own_col = i >= i0 && i < i0 + FM_TXO && i >= 0 && i <= nx - 1;  // columns measured
-    for (int it = 1; it <= n; ++it) {
-        const double cfd = fac.v[fo + it - 1] * dtc;
-        // the row predicates below are recomputed from this copy in every
-        // iteration rather than held across the loop
-        int rk = rk0;
-        asm volatile("" : "+s"(rk));
-        const bool top = rk <= -1, bot = rk + FM_RY - 1 >= nz + 1;  // the held rows include ghost rows
-        // the previous iterate's rows 1 and nz-1 (the row-1 corners read them)
-        double old1 = 0.0, oldn1 = 0.0;
-        if (top) {
+    for (int j = 0; j < FM_K; ++j) mx[j] = 0.0;
+    if (t < tiles) {
+        const int zk = t == 0 ? 1 : (t == tiles - 1 ? 2 : 0);
+        const int i0 = blockIdx.x * FM_TXO - SPAN, k0 = fm_tile_row(nz, TY, t, tiles);
+        const int sx = i0 - nx + 1 > 0 ? i0 - nx + 1 : 0;
+        const int ri0 = i0 - FM_H - sx, rk0 = k0 - FM_H;  // held region origin
+        const int i = ri0 + lane;                          // this lane's column
+        const bool col_in = i >= -SPAN && i <= nx + SPAN, col_int = i >= 0 && i <= nx;
+        const bool corner_col = i == -SPAN || i == nx + SPAN;
+        const int im = (i < 0) ? -i : (i > nx ? 2 * nx - i : i);
+        int ml = lane + (im - i);                               // lane holding the mirrored column
+        ml = ml < 0 ? 0 : (ml > 63 ? 63 : ml);
+        const double dtc = dts[g.at(0, 0)] * courant;
+        double c[RY];
+        const double* __restrict__ sp = src + g.at(col_in ? i : 0, 0);
 #pragma unroll
-            for (int r = 0; r < FM_RY; ++r)
-                if (rk + r == 1) old1 = c[r];
+        for (int r = 0; r < RY; ++r) {
+            // a row beyond the plane (in the first and last tile) reads row 0
+            const int k = rk0 + r;
+            const bool row_in = k >= -SPAN && k <= nz + SPAN;
+            const double v = sp[(ptrdiff_t)(row_in ? k : 0) * g.ld];
+            c[r] = (col_in && row_in) ? v : 0.0;
         }
-        if (bot) {
+        const bool ghost_col = col_in && !col_int;
+        const bool gcols = ri0 <= -1 || ri0 + 63 >= nx + 1;  // the held columns include ghost columns (uniform)
+        const bool own_col = i >= i0 && i < i0 + FM_TXO && i >= 0 && i <= nx - 1;  // columns measured
+        const double* f = replay ? fac.v : fac.v + FM_K;
+        if (zk == 0)
+            fm_iterate<POW2, TY, 0>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col);
+        else if (zk == 1)
+            fm_iterate<POW2, TY, 1>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col);
+        else
+            fm_iterate<POW2, TY, 2>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col);
+        // the tile's own cells of the last iterate
+        if (col_in && i >= i0 && i < i0 + FM_TXO) {
+            double* __restrict__ dp = dst + g.at(i, k0);
 #pragma unroll
-            for (int r = 0; r < FM_RY; ++r)
-                if (rk + r == nz - 1) oldn1 = c[r];
-        }
-        // the step (filter_new's operation order) on every held row but the
-        // first and last; ghost cells are overwritten below, cells outside
-        // the plane are never read by the valid part of the region
-        double om = c[0];
-#pragma unroll
-        for (int r = 1; r < FM_RY - 1; ++r) {
-            const double oc = c[r];
-            const double lf = dpp_from_left(oc), rt = dpp_from_right(oc);
-            double Trr, Tss;
-            if constexpr (FAST) {
-                const double m2 = -2.0 * oc;
-                Trr = ((lf + m2) + rt) * sc.idr2;
-                Tss = ((om + m2) + c[r + 1]) * sc.ids2;
-            } else {
-                double acc = F.D2[1] * lf;
-                acc += F.D2[2] * oc;
-                acc += F.D2[3] * rt;
-                Trr = acc / sc.dr2;
-                acc = F.D2[1] * om;
-                acc += F.D2[2] * oc;
-                acc += F.D2[3] * c[r + 1];
-                Tss = acc / sc.ds2;
-            }
-            const double temp = Trr + Tss;
-            double v = oc + cfd * temp;
-            if (v < 0.0) v = 0.0;
-            if (v > 1.0) v = 1.0;
-            c[r] = v;
-            om = oc;
-        }
-        // ghost columns: the mirrored lane's new value (ghost rows are
-        // overwritten next)
-        if (gcols) {
-#pragma unroll
-            for (int r = 1; r < FM_RY - 1; ++r) {
-                const double mv = __shfl(c[r], ml, 64);
-                c[r] = ghost_col ? mv : c[r];
-            }
-        }
-        // ghost rows: the mirrored row (columns already mirrored), the row-1
-        // corners from the previous iterate
-        if (top) {
-#pragma unroll
-            for (int r = 0; r + 4 < FM_RY; ++r) {
-                if (rk + r == -1) c[r] = corner_col ? old1 : c[r + 2];
-                if (rk + r == -2) c[r] = c[r + 4];
-            }
-        }
-        if (bot) {
-#pragma unroll
-            for (int r = 4; r < FM_RY; ++r) {
-                if (rk + r == nz + 1) c[r] = corner_col ? oldn1 : c[r - 2];
-                if (rk + r == nz + 2) c[r] = c[r - 4];
-            }
-        }
-        if (!replay) {
-            // the new iterate's smoothness over the tile's own nodes of
-            // rows 1..nz-1 (held rows ra..rb): the jumps of smooth_merge,
-            // each vertical pair once (node r's jump up is node r-1's jump
-            // down, |x-y| = |y-x|); the maximum is that of smooth_merge
-            const int ka = k0 > 1 ? k0 : 1, kb = k0 + FM_TY - 1 < nz - 1 ? k0 + FM_TY - 1 : nz - 1;
-            const int ra = ka - rk, rb = kb - rk;  // ra >= FM_H, rb <= FM_RY - 1 - FM_H
-            double a = 0.0;
-            double rm = 0.0, r0 = 0.0;  // the right lane's c[r-1], c[r]
-#pragma unroll
-            for (int r = 1; r < FM_RY - 1; ++r) {
-                // rows outside ra-2..rb are skipped by the whole wave
-                if (r + 2 >= ra && r <= rb) {
-                    const double rp = dpp_from_right(c[r + 1]);
-                    if (r >= ra) {
-                        if (r == ra) a = fmax(a, fabs(c[r - 1] - c[r]));
-                        a = fmax(a, fabs(rm - c[r]));
-                        a = fmax(a, fabs(r0 - c[r]));
-                        a = fmax(a, fabs(c[r + 1] - c[r]));
-                        a = fmax(a, fabs(rp - c[r]));
-                    }
-                    rm = r0;
-                    r0 = rp;
-                }
-            }
-            a = own_col ? a : 0.0;
-            a = block_max(a);
-            if (tid == 0) slot_max(slots + (size_t)((m + it) % FM_SETS) * FILT_SET, a);
+            for (int r = 0; r < TY; ++r) dp[(ptrdiff_t)r * g.ld] = c[FM_H + r];
         }
     }
-    // the tile's own cells of the last iterate
-    const bool own_w = col_in && i >= i0 && i < i0 + FM_TXO;
+    if (!replay) {
 #pragma unroll
-    for (int r = 0; r < FM_RY; ++r) {
-        const int k = rk0 + r;
-        if (own_w && k >= k0 && k < k0 + FM_TY && k >= -SPAN && k <= nz + SPAN) dst[g.at(i, k)] = c[r];
+        for (int j = 0; j < FM_K; ++j) {
+            for (int o = 32; o > 0; o >>= 1) mx[j] = fmax(mx[j], __shfl_xor(mx[j], o, 64));
+            if (lane == 0) s_mx[wy][j] = mx[j];
+        }
+        __syncthreads();
+        if (tid < FM_K) {
+            double a = s_mx[0][tid];
+            for (int w = 1; w < FM_WAVES; ++w) a = fmax(a, s_mx[w][tid]);
+            slot_max(slots + (size_t)((m + tid + 1) % FM_SETS) * FILT_SET, a);
+        }
     }
     if (replay && first && tid == 0) { ctl[0] = m + 1; ctl[1] = j0; ctl[2] = b_out; }
 }
@@ -1064,25 +1101,59 @@ static FScale filter_scale(double dr2, double ds2)
 }
 int filter_multi_k() { return FM_K; }
 
-void launch_filter_multi(hipStream_t st, double* const bufs[3], int b_in, const double* dts, const Grid& g,
-                         const FD& F, double dr2, double ds2, double courant, const double* fac, int m, double delta,
-                         unsigned long long* slots, int32_t* ctl)
+// whether tiles of ty rows fit: the first and the last one hold the ghost
+// rows of their own side only, and those between none
+static bool fm_fits(int nz, int ty) { return nz >= ty + 2 * FM_H - 1; }
+bool filter_multi_takes(const Grid& g, const FD& F)
+{
+    return fm_fits(g.nz, FM_TYS[0]) && F.D2[1] == 1.0 && F.D2[2] == -2.0 && F.D2[3] == 1.0;
+}
+
+template <bool POW2, int TY>
+static void filter_multi_go(hipStream_t st, dim3 gr, const FmBufs& b, int b_in, const double* dts, const Grid& g,
+                            const FScale& sc, double courant, const FmFac& f, int m, double delta,
+                            unsigned long long* slots, int32_t* ctl)
+{
+    hipLaunchKernelGGL((k_filter_multi<POW2, TY>), gr, dim3(64, FM_WAVES), 0, st, b, b_in, dts, g, sc, courant, f, m,
+                       delta, fm_tiles(g.nz, TY), slots, ctl);
+}
+
+void launch_filter_multi(hipStream_t st, double* const bufs[3], int b_in, const double* dts, const Grid& g, double dr2,
+                         double ds2, double courant, const double* fac, int m, double delta,
+                         unsigned long long* slots, int32_t* ctl, int cus)
 {
     FmBufs b{{bufs[0], bufs[1], bufs[2]}};
     FmFac f{};
     for (int j = 0; j < 2 * FM_K; ++j) f.v[j] = fac[j];
-    // tiles of FM_TXO x FM_TY cells over the plane's -SPAN..nx+SPAN x
-    // -SPAN..nz+SPAN, FM_WAVES of them stacked in z per workgroup
-    const int tz = (g.nz + 1 + 2 * SPAN + FM_TY - 1) / FM_TY;
-    dim3 blk(64, FM_WAVES);
-    dim3 gr((unsigned)((g.nx + 1 + 2 * SPAN + FM_TXO - 1) / FM_TXO), (unsigned)((tz + FM_WAVES - 1) / FM_WAVES));
+    // the rows of a tile: a workgroup puts one wave on each SIMD of a CU, so
+    // the launch takes as many rounds as there are workgroups per CU, each
+    // as long as the held rows (and about 6 more for the rest)
+    const unsigned gx = (unsigned)((g.nx + 1 + 2 * SPAN + FM_TXO - 1) / FM_TXO);
+    int best = -1, TY = FM_TYS[0];
+    unsigned gz = 0;
+    for (int ty : FM_TYS) {
+        if (!fm_fits(g.nz, ty)) continue;
+        const unsigned z = (unsigned)((fm_tiles(g.nz, ty) + FM_WAVES - 1) / FM_WAVES);
+        const int cost = (int)((gx * z + cus - 1) / cus) * (ty + 2 * FM_H + 6);
+        if (best < 0 || cost < best) {
+            best = cost;
+            TY = ty;
+            gz = z;
+        }
+    }
+    const dim3 gr(gx, gz);
     const FScale sc = filter_scale(dr2, ds2);
-    if (sc.pow2 && F.D2[1] == 1.0 && F.D2[2] == -2.0 && F.D2[3] == 1.0)
-        hipLaunchKernelGGL((k_filter_multi<true>), gr, blk, 0, st, b, b_in, dts, g, F, sc, courant, f, m, delta, slots,
-                           ctl);
-    else
-        hipLaunchKernelGGL((k_filter_multi<false>), gr, blk, 0, st, b, b_in, dts, g, F, sc, courant, f, m, delta, slots,
-                           ctl);
+    auto go = [&](auto pw) {
+        constexpr bool P = decltype(pw)::value;
+        switch (TY) {
+        case FM_TYS[0]: filter_multi_go<P, FM_TYS[0]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
+        case FM_TYS[1]: filter_multi_go<P, FM_TYS[1]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
+        case FM_TYS[2]: filter_multi_go<P, FM_TYS[2]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
+        default: filter_multi_go<P, FM_TYS[3]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
+        }
+    };
+    if (sc.pow2) go(std::integral_constant<bool, true>{});
+    else go(std::integral_constant<bool, false>{});
 }
 
 void launch_filter_iter(hipStream_t st, bool comp, const double* T0, double* T, const double* dts, const Grid& g,

@@ -19,6 +19,16 @@ __device__ __forceinline__ double sdiv(double a, double d, double inv)
     if constexpr (POW2) return a * inv; else return a / d;
 }
 
+// a/d as the division rounds it, from y = 1/d rounded: two corrections by
+// the FMA remainder (Markstein's theorem: with y correctly rounded and the
+// quotient within an ulp, one more correction rounds correctly).  5
+// instructions instead of the division sequence.
+__device__ __forceinline__ double div_by(double a, double d, double y)
+{
+    double q = a * y;
+    q = __builtin_fma(__builtin_fma(-d, q, a), y, q);
+    return __builtin_fma(__builtin_fma(-d, q, a), y, q);
+}
 struct Spacing {
     double dr, ds, dr2, ds2, dr3, ds3, dr4, ds4, drds, drds2, dr2ds, dr2ds2;
     double idr, ids, idr2, ids2, idr3, ids3, idr4, ids4, idrds, idrds2, idr2ds, idr2ds2;

@@ -91,16 +91,6 @@ struct RefCell {
     double vis, vd, vx2, vz2, vxz4, vis2, rhs, dts;
 };
 
-// a/d as the division rounds it, from y = 1/d rounded: two corrections by
-// the FMA remainder (Markstein's theorem: with y correctly rounded and the
-// quotient within an ulp, one more correction rounds correctly).  5
-// instructions instead of the division sequence.
-__device__ __forceinline__ double div_by(double a, double d, double y)
-{
-    double q = a * y;
-    q = __builtin_fma(__builtin_fma(-d, q, a), y, q);
-    return __builtin_fma(__builtin_fma(-d, q, a), y, q);
-}
 // With spacings that are powers of two (POW2) the quotients are exact
 // scalings: they go into the FMA that follows (fma(x, s, y) rounds once, as
 // the sum of the scaled x does) or, where the quotient is only multiplied by a
