@@ -226,16 +226,44 @@ int put_plane_direct(tc_ctx* ctx, double* dev, const Grid& g, const double* host
 }
 int put_iplane(tc_ctx* ctx, int32_t* dev, const Grid& g, const int32_t* host)
 {
-    const size_t w = (size_t)(g.nx + 2 * SPAN + 1);
-    TC_HIP(hipMemcpy2DAsync(dev + g.at(-SPAN, -SPAN), g.ld * sizeof(int32_t), host, w * sizeof(int32_t),
-                            w * sizeof(int32_t), g.nz + 2 * SPAN + 1, hipMemcpyHostToDevice, ctx->stream));
-    return 0;
+    const size_t w = (size_t)(g.nx + 2 * SPAN + 1) * sizeof(int32_t);
+    return copy_rows_h2d(ctx, dev + g.at(-SPAN, -SPAN), g.ld * sizeof(int32_t), host, w, (size_t)(g.nz + 2 * SPAN + 1));
 }
 int get_iplane(tc_ctx* ctx, const int32_t* dev, const Grid& g, int32_t* host)
 {
-    const size_t w = (size_t)(g.nx + 2 * SPAN + 1);
-    TC_HIP(hipMemcpy2DAsync(host, w * sizeof(int32_t), dev + g.at(-SPAN, -SPAN), g.ld * sizeof(int32_t),
-                            w * sizeof(int32_t), g.nz + 2 * SPAN + 1, hipMemcpyDeviceToHost, ctx->stream));
+    const size_t w = (size_t)(g.nx + 2 * SPAN + 1) * sizeof(int32_t);
+    return copy_rows_d2h(ctx, host, dev + g.at(-SPAN, -SPAN), g.ld * sizeof(int32_t), w, (size_t)(g.nz + 2 * SPAN + 1));
+}
+
+// n bytes of contiguous device memory, in rows that fill the chunk buffers
+int get_flat(tc_ctx* ctx, void* host, const void* dev, size_t n)
+{
+    const size_t row = std::min<size_t>(n, (size_t)64 << 10), rows = n / row, rest = n - rows * row;
+    TC_TRY(copy_rows_d2h(ctx, host, dev, row, row, rows));
+    if (rest)
+        TC_TRY(copy_rows_d2h(ctx, static_cast<char*>(host) + rows * row, static_cast<const char*>(dev) + rows * row, rest,
+                             rest, 1));
+    return 0;
+}
+
+// the n planes of a per-type field (elements of `bytes`) to or from the host
+// in the boundary's type-fastest layout
+int types_xfer(tc_ctx* ctx, const PackPlanes& P, int n, int bytes, void* host, bool get)
+{
+    const Grid& g = ctx->g;
+    const size_t w = (size_t)(g.nx + 2 * SPAN + 1), h = (size_t)(g.nz + 2 * SPAN + 1);
+    if (!ctx->pack_buf) {
+        const int nt = ctx->p.ntype;
+        TC_HIP(hipMalloc(&ctx->pack_buf, w * h * (size_t)std::max(8 * nt, 4 * (nt + 1))));
+    }
+    const size_t row = w * (size_t)(n * bytes);
+    if (get) {
+        launch_pack_types(ctx->stream, P, g, n, bytes, ctx->pack_buf, true);
+        return copy_rows_d2h(ctx, host, ctx->pack_buf, row, row, h);
+    }
+    TC_TRY(copy_rows_h2d(ctx, ctx->pack_buf, row, host, row, h));
+    launch_pack_types(ctx->stream, P, g, n, bytes, ctx->pack_buf, false);
+    TC_HIP(hipStreamSynchronize(ctx->stream));
     return 0;
 }
 
@@ -2302,6 +2330,7 @@ void free_ctx(tc_ctx* ctx)
         if (ctx->xfer_buf[b]) (void)hipHostFree(ctx->xfer_buf[b]);
         if (ctx->xfer_ev[b]) (void)hipEventDestroy(ctx->xfer_ev[b]);
     }
+    if (ctx->pack_buf) (void)hipFree(ctx->pack_buf);
     tc_dev* d = static_cast<tc_dev*>(ctx->impl);
     if (d) {
         F(d->d_scal); F(d->partialA); F(d->partialB); F(d->ctl); F(d->fslots); F(d->fbuf); F(d->diag); F(d->diag_part); F(d->stats_part); F(d->stats_out);
@@ -2776,15 +2805,11 @@ int tc_put_field(tc_ctx* ctx, int field, const void* host)
     }
     if (field == TC_F_CNEW || field == TC_F_CVIS || field == TC_F_CBUOY) {
         if (nt < 1) return TC_ERR_ARG;
-        std::vector<double> tmp(w * h);
-        const double* src = (const double*)host;
-        for (int t = 0; t < nt; ++t) {
-            for (size_t e = 0; e < w * h; ++e) tmp[e] = src[e * nt + t];
-            double* dst = field == TC_F_CNEW ? ctx->Cnew[t] : (field == TC_F_CVIS ? ctx->Cvis[t] : ctx->Cbuoy[t]);
-            TC_TRY(put_plane(ctx, dst, g, tmp.data()));
-            TC_HIP(hipStreamSynchronize(ctx->stream));
-        }
-        return 0;
+        double* const* pl = field == TC_F_CNEW ? ctx->Cnew : (field == TC_F_CVIS ? ctx->Cvis : ctx->Cbuoy);
+        if (nt == 1) return put_plane(ctx, pl[0], g, (const double*)host);
+        PackPlanes P{};
+        for (int t = 0; t < nt; ++t) P.v[t] = pl[t];
+        return types_xfer(ctx, P, nt, 8, const_cast<void*>(host), false);
     }
     if (field == TC_F_NEMPTY) {
         TC_TRY(put_iplane(ctx, ctx->nempty, g, (const int32_t*)host));
@@ -2792,14 +2817,9 @@ int tc_put_field(tc_ctx* ctx, int field, const void* host)
         return 0;
     }
     if (field == TC_F_COUNT_TYPE) {
-        std::vector<int32_t> tmp(w * h);
-        const int32_t* src = (const int32_t*)host;
-        for (int t = 0; t <= nt; ++t) {
-            for (size_t e = 0; e < w * h; ++e) tmp[e] = src[e * (nt + 1) + t];
-            TC_TRY(put_iplane(ctx, ctx->count[t], g, tmp.data()));
-            TC_HIP(hipStreamSynchronize(ctx->stream));
-        }
-        return 0;
+        PackPlanes P{};
+        for (int t = 0; t <= nt; ++t) P.v[t] = ctx->count[t];
+        return types_xfer(ctx, P, nt + 1, 4, const_cast<void*>(host), false);
     }
     return TC_ERR_ARG;
 }
@@ -2831,15 +2851,11 @@ int tc_get_field(tc_ctx* ctx, int field, void* host)
     }
     if (field == TC_F_CNEW || field == TC_F_CVIS || field == TC_F_CBUOY) {
         if (nt < 1) return TC_ERR_ARG;
-        std::vector<double> tmp(w * h);
-        double* dst = (double*)host;
-        for (int t = 0; t < nt; ++t) {
-            const double* src = field == TC_F_CNEW ? ctx->Cnew[t] : (field == TC_F_CVIS ? ctx->Cvis[t] : ctx->Cbuoy[t]);
-            TC_TRY(get_plane(ctx, src, g, tmp.data()));
-            TC_HIP(hipStreamSynchronize(ctx->stream));
-            for (size_t e = 0; e < w * h; ++e) dst[e * nt + t] = tmp[e];
-        }
-        return 0;
+        double* const* pl = field == TC_F_CNEW ? ctx->Cnew : (field == TC_F_CVIS ? ctx->Cvis : ctx->Cbuoy);
+        if (nt == 1) return get_plane(ctx, pl[0], g, (double*)host);
+        PackPlanes P{};
+        for (int t = 0; t < nt; ++t) P.v[t] = pl[t];
+        return types_xfer(ctx, P, nt, 8, host, true);
     }
     if (field == TC_F_NEMPTY) {
         TC_TRY(get_iplane(ctx, ctx->nempty, g, (int32_t*)host));
@@ -2847,14 +2863,9 @@ int tc_get_field(tc_ctx* ctx, int field, void* host)
         return 0;
     }
     if (field == TC_F_COUNT_TYPE) {
-        std::vector<int32_t> tmp(w * h);
-        int32_t* dst = (int32_t*)host;
-        for (int t = 0; t <= nt; ++t) {
-            TC_TRY(get_iplane(ctx, ctx->count[t], g, tmp.data()));
-            TC_HIP(hipStreamSynchronize(ctx->stream));
-            for (size_t e = 0; e < w * h; ++e) dst[e * (nt + 1) + t] = tmp[e];
-        }
-        return 0;
+        PackPlanes P{};
+        for (int t = 0; t <= nt; ++t) P.v[t] = ctx->count[t];
+        return types_xfer(ctx, P, nt + 1, 4, host, true);
     }
     return TC_ERR_ARG;
 }
@@ -2973,12 +2984,12 @@ int tc_get_tracers(tc_ctx* ctx, int which, double* r, double* s)
     if (ctx->tr_id) {
         // node-sorted on the device: back to the caller's order
         launch_scatter_d(ctx->stream, dr, ctx->tr_id, ctx->spare_d, ctx->ntr);
-        TC_HIP(hipMemcpyAsync(r, ctx->spare_d, nb, hipMemcpyDeviceToHost, ctx->stream));
+        TC_TRY(get_flat(ctx, r, ctx->spare_d, nb));
         launch_scatter_d(ctx->stream, ds, ctx->tr_id, ctx->spare_d, ctx->ntr);
-        TC_HIP(hipMemcpyAsync(s, ctx->spare_d, nb, hipMemcpyDeviceToHost, ctx->stream));
+        TC_TRY(get_flat(ctx, s, ctx->spare_d, nb));
     } else {
-        TC_HIP(hipMemcpyAsync(r, dr, nb, hipMemcpyDeviceToHost, ctx->stream));
-        TC_HIP(hipMemcpyAsync(s, ds, nb, hipMemcpyDeviceToHost, ctx->stream));
+        TC_TRY(get_flat(ctx, r, dr, nb));
+        TC_TRY(get_flat(ctx, s, ds, nb));
     }
     TC_HIP(hipStreamSynchronize(ctx->stream));
     return 0;

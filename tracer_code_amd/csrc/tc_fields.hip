@@ -599,6 +599,30 @@ __global__ void k_zero_i32(int32_t* __restrict__ p, size_t n)
     for (; t < n; t += (size_t)gridDim.x * blockDim.x) p[t] = 0;
 }
 
+// The ghosted planes of n types, one word of each at a time, to and from the
+// boundary's layout (type fastest, rows without padding).  Moved on the device
+// in one pass, so that the host copy is one contiguous transfer; gathered on
+// the host type by type, a 2048x1024 composition took 5.0 ms and the counts
+// 15.8 ms, most of it in strided host loops and pageable copies.
+template <typename W>
+__global__ __launch_bounds__(256) void k_pack_types(PackPlanes P, Grid g, int n, W* __restrict__ out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;  // 0..nx+4, 0..nz+4
+    const int w = g.nx + 2 * SPAN + 1;
+    if (i >= w) return;
+    const size_t c = g.at(i - SPAN, k - SPAN), o = ((size_t)k * w + i) * n;
+    for (int t = 0; t < n; ++t) out[o + t] = static_cast<const W*>(P.v[t])[c];
+}
+template <typename W>
+__global__ __launch_bounds__(256) void k_unpack_types(PackPlanes P, Grid g, int n, const W* __restrict__ in)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
+    const int w = g.nx + 2 * SPAN + 1;
+    if (i >= w) return;
+    const size_t c = g.at(i - SPAN, k - SPAN), o = ((size_t)k * w + i) * n;
+    for (int t = 0; t < n; ++t) static_cast<W*>(P.v[t])[c] = in[o + t];
+}
+
 // tracers_to_corners counting loop (composition.f90:704-715): nearest node
 // by Fortran NINT (half away from zero) of r/dr and s/ds, domain check.
 template <bool POW2>
@@ -885,6 +909,18 @@ __global__ __launch_bounds__(256) void k_stability(const double* __restrict__ u,
 }
 
 // ---------------------------------------------------------------------------
+void launch_pack_types(hipStream_t st, const PackPlanes& P, const Grid& g, int n, int bytes, void* buf, bool pack)
+{
+    const dim3 b(256), gr((unsigned)((g.nx + 2 * SPAN + 256) / 256), (unsigned)(g.nz + 2 * SPAN + 1));
+    if (pack) {
+        if (bytes == 8) hipLaunchKernelGGL(k_pack_types<uint64_t>, gr, b, 0, st, P, g, n, static_cast<uint64_t*>(buf));
+        else hipLaunchKernelGGL(k_pack_types<uint32_t>, gr, b, 0, st, P, g, n, static_cast<uint32_t*>(buf));
+    } else {
+        if (bytes == 8) hipLaunchKernelGGL(k_unpack_types<uint64_t>, gr, b, 0, st, P, g, n, static_cast<const uint64_t*>(buf));
+        else hipLaunchKernelGGL(k_unpack_types<uint32_t>, gr, b, 0, st, P, g, n, static_cast<const uint32_t*>(buf));
+    }
+}
+
 void launch_velocities(hipStream_t st, const double* SF, double* u, double* w, const Grid& g, const FD& F, double dr,
                        double ds, int Vbc)
 {

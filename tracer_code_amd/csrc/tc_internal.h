@@ -272,6 +272,7 @@ struct tc_ctx {
     // (tc_get_field / tc_put_field): allocated on first use
     void* xfer_buf[2] = {nullptr, nullptr};
     hipEvent_t xfer_ev[2] = {nullptr, nullptr};
+    void* pack_buf = nullptr;     // device: composition and counts in the boundary's layout, on first use
     // kernel timing (tc_set_profiling)
     bool prof = false;
     std::vector<hipEvent_t> prof_ev;

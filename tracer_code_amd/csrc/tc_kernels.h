@@ -239,6 +239,10 @@ void launch_velocities(hipStream_t st, const double* SF, double* u, double* w, c
                        double ds, int Vbc);
 void launch_strain(hipStream_t st, const double* u, const double* w, double* strain, const Grid& g, const FD& F,
                    double dr, double ds);
+struct PackPlanes { void* v[TC_MAX_TYPES + 1]; };
+// the planes of n types (elements of 4 or 8 bytes) to (pack) or from buf in
+// the boundary's type-fastest layout
+void launch_pack_types(hipStream_t st, const PackPlanes& P, const Grid& g, int n, int bytes, void* buf, bool pack);
 void launch_bcs_T(hipStream_t st, double* T, const Grid& g, int Tbot, const int32_t* stop = nullptr);
 void launch_bcs_comp(hipStream_t st, double* C, const Grid& g, const int32_t* stop = nullptr);
 void launch_zero_i32(hipStream_t st, int32_t* p, size_t n);
