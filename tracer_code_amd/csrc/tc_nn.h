@@ -42,13 +42,14 @@ struct UNet {
     float *ga3 = nullptr, *gs3 = nullptr, *gp3 = nullptr, *ga4 = nullptr, *gb4 = nullptr, *gd3a = nullptr;
     float *gd3b = nullptr, *gd2a = nullptr, *gd2b = nullptr, *gd1a = nullptr, *gd1b = nullptr, *gx0 = nullptr;
     __bf16* dz = nullptr;
-    float *wpart = nullptr, *gw32 = nullptr;
+    float* wpart = nullptr;
     double *hpart = nullptr, *loss_d = nullptr;
     float *out = nullptr, *target = nullptr, *mask = nullptr;
     std::vector<void*> owned;
 
     void layer_defs();
     size_t param_count() const;
+    int split_pixels(const Layer& l) const;
     int alloc(int H, int W, bool train);
     void release();
     void pack(hipStream_t st);

@@ -66,34 +66,44 @@ struct ConvArgs {
     int mode;
 };
 
+// Bound: the latency of the fragment loads (an iteration of 32 depth values
+// is one MFMA after two 16-byte loads).  KS waves share a tile's depth and add
+// up their accumulators in LDS, so that on the small levels, whose tiles
+// leave most CUs idle, the chain of loads is KS times shorter; addresses are
+// clamped and values selected, so that the loads of several iterations are
+// in flight.
+template <int KS>
 __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a)
 {
+    constexpr int TILES = 4 / KS;  // tiles of a workgroup
+    __shared__ f32x4 part[KS > 1 ? 4 : 1][64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int npix = a.H * a.W;
-    const int p0 = (blockIdx.x * 4 + wv) * 16;
+    const int p0 = (blockIdx.x * TILES + wv / KS) * 16, ks = wv % KS;
     const int cb = blockIdx.y;
-    if (p0 >= npix) return;
     const int row = lane & 15, grp = lane >> 4;
     const int p = p0 + row;
     const int py = p / a.W, px = p - py * a.W;
     const int co = cb * 16 + row;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = grp * 8; k0 < a.kp; k0 += 32) {
-        bf16x8 fa, fb;
+    const __bf16* __restrict__ wk = a.wk + (size_t)co * a.kp;
+#pragma unroll 4
+    for (int k0 = ks * 32 + grp * 8; k0 < a.kp; k0 += 32 * KS) {
         const int tap = k0 / a.cinp, ci0 = k0 - tap * a.cinp;
-        bool ok = tap < 9 && p < npix;
-        int q = 0;
-        if (ok) {
-            const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-            const int yy = py + dy, xx = px + dx;
-            ok = yy >= 0 && yy < a.H && xx >= 0 && xx < a.W;
-            q = yy * a.W + xx;
-        }
-        if (ok) fa = *reinterpret_cast<const bf16x8*>(a.in + (size_t)q * a.cs_in + a.off_in + ci0);
-        else
+        const int yy = py + tap / 3 - 1, xx = px + tap % 3 - 1;
+        const bool ok = tap < 9 && p < npix && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W;
+        bf16x8 fa = *reinterpret_cast<const bf16x8*>(a.in + (ok ? (size_t)(yy * a.W + xx) * a.cs_in + a.off_in + ci0
+                                                                  : (size_t)a.off_in));
+        if (!ok)
             for (int j = 0; j < 8; ++j) fa[j] = (__bf16)0.0f;
-        fb = *reinterpret_cast<const bf16x8*>(a.wk + (size_t)co * a.kp + k0);
+        const bf16x8 fb = *reinterpret_cast<const bf16x8*>(wk + k0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, acc, 0, 0, 0);
+    }
+    if constexpr (KS > 1) {
+        part[wv][lane] = acc;
+        __syncthreads();
+        if (ks != 0) return;
+        for (int q = 1; q < KS; ++q) acc += part[wv + q][lane];
     }
     // lane holds D[pixel p0 + grp*4 + i][channel cb*16 + row]
     const int c = cb * 16 + row;
@@ -115,6 +125,19 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a)
     }
 }
 
+// KS = 4 waves a tile while the launch would otherwise hold fewer than 2
+// waves per SIMD of the chip (2048) and a wave has more than 2 iterations:
+// at 32x96 pixels the 27 forward and input-gradient launches of a training
+// step take 138 us instead of 250
+static void launch_conv3x3(hipStream_t st, const ConvArgs& a)
+{
+    const int tiles = (a.H * a.W + 15) / 16, cbs = a.cout / 16;
+    if ((long)tiles * cbs < 2048 && a.kp > 64)
+        hipLaunchKernelGGL(k_conv3x3<4>, dim3(tiles, cbs), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_conv3x3<1>, dim3((tiles + 3) / 4, cbs), dim3(256), 0, st, a);
+}
+
 // Weight gradient: partial[split][co][k] = sum over the split's pixels of
 // dz[p][co] * X[p+off(tap)][ci]; as an MFMA product the rows are output
 // channels, the columns k, the reduction runs over 32 pixels at a time.
@@ -127,9 +150,14 @@ struct WGradArgs {
     int H, W, pix_per_split;
 };
 
-__global__ __launch_bounds__(64) void k_conv3x3_wgrad(WGradArgs a)
+// Bound: the latency of its 2-byte loads; 4 waves share a split's chunks of 32
+// pixels and add up in LDS, and the splits fill the chip (one split of up to
+// 2048 pixels a wave took 148 to 170 us a layer at 32x96 pixels, in 10 to 28
+// waves).
+__global__ __launch_bounds__(256) void k_conv3x3_wgrad(WGradArgs a)
 {
-    const int lane = threadIdx.x;
+    __shared__ f32x4 part[4][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int cb = blockIdx.x, kb = blockIdx.y, split = blockIdx.z;
     const int npix = a.H * a.W;
     const int row = lane & 15, grp = lane >> 4;
@@ -141,47 +169,53 @@ __global__ __launch_bounds__(64) void k_conv3x3_wgrad(WGradArgs a)
     int pend = pbeg + a.pix_per_split;
     if (pend > npix) pend = npix;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int pb = pbeg; pb < pend; pb += 32) {
+    for (int pb = pbeg + 32 * wv; pb < pend; pb += 128) {
         bf16x8 fa, fb;
+        const int p0 = pb + grp * 8;
+        int y = p0 / a.W, x = p0 - y * a.W;
+#pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const int p = pb + grp * 8 + j;
-            __bf16 va = (__bf16)0.0f, vb = (__bf16)0.0f;
-            if (p < pend) {
-                va = a.dz[(size_t)p * a.cout + co];
-                if (tap < 9) {
-                    const int py = p / a.W, px = p - py * a.W;
-                    const int yy = py + dy, xx = px + dx;
-                    if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W)
-                        vb = a.in[(size_t)(yy * a.W + xx) * a.cs_in + a.off_in + ci];
-                }
-            }
-            fa[j] = va;
-            fb[j] = vb;
+            const int p = p0 + j, yy = y + dy, xx = x + dx;
+            const bool in = p < pend, ok = in && tap < 9 && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W;
+            const __bf16 va = a.dz[(size_t)(in ? p : 0) * a.cout + co];
+            const __bf16 vb = a.in[(size_t)(ok ? yy * a.W + xx : 0) * a.cs_in + a.off_in + (ok ? ci : 0)];
+            fa[j] = in ? va : (__bf16)0.0f;
+            fb[j] = ok ? vb : (__bf16)0.0f;
+            if (++x == a.W) { x = 0; ++y; }
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, acc, 0, 0, 0);
     }
+    part[wv][lane] = acc;
+    __syncthreads();
+    if (wv != 0) return;
+    for (int q = 1; q < 4; ++q) acc += part[q][lane];
     // lane holds D[co = cb*16 + grp*4 + i][k = kb*16 + row]
     for (int i = 0; i < 4; ++i)
         a.partial[((size_t)split * a.cout + cb * 16 + grp * 4 + i) * a.kp + kcol] = acc[i];
 }
 
-__global__ __launch_bounds__(256) void k_reduce_splits(const float* __restrict__ partial, int nsplit, size_t n,
-                                                       float* __restrict__ out)
+// The splits' sums into the gradient of W[co][tap][ci], and (the blocks past
+// them, one per output channel) the bias gradient db[c] += sum_p dz[p][c].
+__global__ __launch_bounds__(256) void k_wgrad_finish(const float* __restrict__ partial, int nsplit, int cin, int cinp,
+                                                      int cout, int kp, float* __restrict__ gw, int wblocks,
+                                                      const __bf16* __restrict__ dz, int npix, float* __restrict__ db)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
+    if ((int)blockIdx.x < wblocks) {
+        const int e = blockIdx.x * 256 + threadIdx.x;
+        if (e >= cout * 9 * cin) return;
+        const int ci = e % cin, r = e / cin, tap = r % 9, co = r / 9;
+        const float* __restrict__ q = partial + (size_t)co * kp + tap * cinp + ci;
+        const size_t n = (size_t)cout * kp;
+        float s = 0.0f;
+#pragma unroll 8
+        for (int t = 0; t < nsplit; ++t) s += q[t * n];
+        gw[e] += s;
+        return;
+    }
+    const int c = blockIdx.x - wblocks;
     float s = 0.0f;
-    for (int q = 0; q < nsplit; ++q) s += partial[(size_t)q * n + e];
-    out[e] += s;
-}
-
-// bias gradient: db[c] += sum_p dz[p][c]
-__global__ __launch_bounds__(256) void k_bias_grad(const __bf16* __restrict__ dz, int npix, int cout,
-                                                   float* __restrict__ db)
-{
-    const int c = blockIdx.x;
-    float s = 0.0f;
-    for (int p = threadIdx.x; p < npix; p += blockDim.x) s += (float)dz[(size_t)p * cout + c];
+#pragma unroll 4
+    for (int p = threadIdx.x; p < npix; p += 256) s += (float)dz[(size_t)p * cout + c];
     s = (float)block_sum((double)s);
     if (threadIdx.x == 0) db[c] += s;
 }
@@ -287,12 +321,21 @@ __global__ __launch_bounds__(256) void k_head_back(const float* __restrict__ out
         }
         g[16] = dout;
     }
-    l = block_sum(l);
-    if (threadIdx.x == 0) part[(size_t)blockIdx.x * 18] = l;
-    for (int c = 0; c < 17; ++c) {
-        const double s = block_sum(g[c]);
-        if (threadIdx.x == 0) part[(size_t)blockIdx.x * 18 + 1 + c] = s;
+    // the 18 sums of the block: by shuffles within each wave, then over the
+    // waves in LDS, with one barrier for all (one block reduction each took
+    // 11.2 us at 3072 pixels)
+    __shared__ double sh[4][18];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+    for (int c = 0; c < 18; ++c) {
+        double v = c == 0 ? l : g[c - 1];
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+        if (lane == 0) sh[wv][c] = v;
     }
+    __syncthreads();
+    if (threadIdx.x < 18)
+        part[(size_t)blockIdx.x * 18 + threadIdx.x] =
+            ((sh[0][threadIdx.x] + sh[1][threadIdx.x]) + sh[2][threadIdx.x]) + sh[3][threadIdx.x];
 }
 __global__ __launch_bounds__(256) void k_head_reduce(const double* __restrict__ part, int nb, float* __restrict__ gw,
                                                      float* __restrict__ gb, double* __restrict__ loss)
@@ -345,18 +388,6 @@ __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ w, int c
         if (tp < 9 && ci < cin) v = w[((size_t)co * 9 + (8 - tp)) * cin + ci];
         wt[e] = (__bf16)v;
     }
-}
-
-// gradient of the packed layout back to W[co][tap][ci] (accumulated)
-__global__ __launch_bounds__(256) void k_unpack_grad(const float* __restrict__ gk, int cin, int cinp, int cout, int kp,
-                                                     float* __restrict__ g)
-{
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)cout * 9 * cin) return;
-    const int ci = (int)(e % cin);
-    const size_t r = e / cin;
-    const int tap = (int)(r % 9), co = (int)(r / 9);
-    g[e] += gk[(size_t)co * kp + tap * cinp + ci];
 }
 
 // input assembly: node (i,k) of the solver plane -> pixel k*W+i (8 channels)
@@ -508,6 +539,16 @@ static inline int up8(int c) { return (c + 7) / 8 * 8; }
 static inline int up16(int c) { return (c + 15) / 16 * 16; }
 static inline int up32(int c) { return (c + 31) / 32 * 32; }
 
+// pixels of a split of the weight gradient: multiples of 128 (a chunk of 32
+// for each wave), so that the launch has about 1024 workgroups, in at most
+// 64 splits
+int UNet::split_pixels(const Layer& l) const
+{
+    const int wg = (l.cout / 16) * (l.kp / 16), n = npx[l.lev];
+    const int splits = std::max(1, std::min(64, 1024 / wg));
+    return ((n + splits - 1) / splits + 127) / 128 * 128;
+}
+
 size_t UNet::param_count() const
 {
     size_t n = 0;
@@ -527,6 +568,7 @@ int UNet::alloc(int H_, int W_, bool train)
         owned.push_back(*p);
         return 0;
     };
+    for (int lev = 0; lev < 4; ++lev) npx[lev] = (H >> lev) * (W >> lev);
     nparam = param_count();
     TC_NN_TRY(dmal((void**)&w32, nparam * sizeof(float)));
     if (train) {
@@ -549,8 +591,6 @@ int UNet::alloc(int H_, int W_, bool train)
         TC_NN_TRY(dmal((void**)&l.wt, (size_t)l.cinp16 * l.kpt * sizeof(__bf16)));
     }
     head_off = off;
-    // activations: per level the pixel count
-    for (int lev = 0; lev < 4; ++lev) npx[lev] = (H >> lev) * (W >> lev);
     // buffers (bf16): x0 (8), a1 (16), s1 (48: [up 32 | skip 16]), p1 (16),
     // a2 (32), s2 (96: [up 64 | skip 32]), p2 (32), a3 (64), s3 (192: [up 128 | skip 64]),
     // p3 (64), a4 (128), b4 (128), d3a (64), d3b (64), d2a (32), d2b (32), d1a (16), d1b (16)
@@ -571,12 +611,11 @@ int UNet::alloc(int H_, int W_, bool train)
         TC_NN_TRY(dmal((void**)&dz, (size_t)npx[0] * 192 * sizeof(__bf16)));
         size_t maxpart = 0;
         for (Layer& l : L) {
-            const int pps = 2048;
+            const int pps = split_pixels(l);
             l.nsplit = (npx[l.lev] + pps - 1) / pps;
             maxpart = std::max(maxpart, (size_t)l.nsplit * l.cout * l.kp);
         }
         TC_NN_TRY(dmal((void**)&wpart, maxpart * sizeof(float)));
-        TC_NN_TRY(dmal((void**)&gw32, (size_t)2 * 192 * 9 * 128 * sizeof(float)));
         TC_NN_TRY(dmal((void**)&hpart, (size_t)nblk(npx[0]) * 18 * sizeof(double)));
         TC_NN_TRY(dmal((void**)&loss_d, sizeof(double)));
     }
@@ -606,8 +645,7 @@ void UNet::conv(hipStream_t st, const Layer& l, const __bf16* in, int cs_in, int
 {
     ConvArgs a{in, cs_in, off_in, l.cinp, l.wk, l.kp, l.cout, w32 + l.boff, o, l.z, nullptr, cs_out, off_out,
                H >> l.lev, W >> l.lev, 0};
-    const int tiles = (npx[l.lev] + 15) / 16;
-    hipLaunchKernelGGL(k_conv3x3, dim3((tiles + 3) / 4, l.cout / 16), dim3(256), 0, st, a);
+    launch_conv3x3(st, a);
 }
 
 void UNet::forward(hipStream_t st)
@@ -652,22 +690,18 @@ void UNet::conv_back(hipStream_t st, const Layer& l, float* gy, int cs_y, int of
     const int np = npx[l.lev];
     hipLaunchKernelGGL(k_gelu_back, dim3(nblk((size_t)np * l.cout)), dim3(256), 0, st, gy, cs_y, off_y, l.z, dz, np,
                        l.cout);
-    // weight gradient
-    const int pps = 2048;
+    // weight and bias gradient
+    const int pps = split_pixels(l);
     WGradArgs wa{dz, in, cs_in, off_in, l.cinp, l.kp, l.cout, wpart, H >> l.lev, W >> l.lev, pps};
-    hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(l.cout / 16, l.kp / 16, l.nsplit), dim3(64), 0, st, wa);
-    const size_t n = (size_t)l.cout * l.kp;
-    hipMemsetAsync(gw32, 0, n * sizeof(float), st);
-    hipLaunchKernelGGL(k_reduce_splits, dim3(nblk(n)), dim3(256), 0, st, wpart, l.nsplit, n, gw32);
-    hipLaunchKernelGGL(k_unpack_grad, dim3(nblk((size_t)l.cout * 9 * l.cin)), dim3(256), 0, st, gw32, l.cin, l.cinp,
-                       l.cout, l.kp, g32 + l.woff);
-    hipLaunchKernelGGL(k_bias_grad, dim3(l.cout), dim3(256), 0, st, dz, np, l.cout, g32 + l.boff);
+    hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(l.cout / 16, l.kp / 16, l.nsplit), dim3(256), 0, st, wa);
+    const int wb = (int)nblk((size_t)l.cout * 9 * l.cin);
+    hipLaunchKernelGGL(k_wgrad_finish, dim3(wb + l.cout), dim3(256), 0, st, wpart, l.nsplit, l.cin, l.cinp, l.cout, l.kp,
+                       g32 + l.woff, wb, dz, np, g32 + l.boff);
     // input gradient: conv of dz with the flipped, transposed weights
     if (gin) {
         ConvArgs a{dz, l.cout, 0, l.cout, l.wt, l.kpt, l.cinp16, nullptr, nullptr, nullptr, gin, cs_gin, off_gin,
                    H >> l.lev, W >> l.lev, 1};
-        const int tiles = (np + 15) / 16;
-        hipLaunchKernelGGL(k_conv3x3, dim3((tiles + 3) / 4, l.cinp16 / 16), dim3(256), 0, st, a);
+        launch_conv3x3(st, a);
     }
 }
 
