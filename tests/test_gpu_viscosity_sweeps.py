@@ -1,0 +1,41 @@
+"""The untested passes of smoother_vis several sweeps per launch
+(k_vis_multi), against the oracle's compute_viscosity (iterative_solver.f90:
+331-377): the fine viscosity and the solution of a solve to 1e-3 (few cycles;
+the sweeps run on every level's viscosity), at heights where one tile holds
+all rows, where the tiles overlap, one row more, and where the taller tiles
+are taken; with lengths of the pass that split into one, two and three
+launches.  The operations are the reference's: what differs is exp(), by an
+ulp, which the solution shows times the condition of the fourth-order operator:
+about 4e-16 (nz/32)^4 (nz = 32: 1e-15, 104: 5e-14, 768: 3e-10), so 1e-12 at the
+largest height here, within the bound of 1e-10."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import load_oracle_state, rel_err
+from tracer_code_amd import Solver, config, ic
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nx,nz,ov", [
+    (16, 16, {}), (56, 32, {}), (52, 34, dict(vis_iter=5)), (106, 36, {}), (64, 64, dict(vis_iter=13)),
+    (160, 96, {}), (152, 104, dict(visT=1e4)), (4096, 224, dict(vis_iter=7)),
+])
+def test_viscosity_sweeps_match_oracle(nx, nz, ov):
+    cfg = dict(config.PRESETS["cfg2"], nx=nx, nz=nz, aspect=nx / nz, tpc=2, tolerance=1e-3, Nmulti=20, visT=100.0)
+    cfg.update(ov)
+    params = config.make_params(**cfg)
+    cfg.update(nx=params.nx, nz=params.nz)
+    T, r, s, ty = ic.workload(cfg, seed=3)
+    print(f"[viscosity sweeps] {params.nx}x{params.nz}, {params.grids} levels, pass of {params.vis_iter}", flush=True)
+    o = load_oracle_state(params, T, r, s, ty)
+    with Solver(params, len(r)) as g:
+        g.initialize(T, r, s, ty)
+        q, _, _ = g.multigrid()
+        assert o.multigrid() == 0 and q == int(o.scalar(oracle.ORS_Q))
+        e_vis = rel_err(g.get("vis")[2:-2, 2:-2], o.plane(oracle.OR_VIS, 1)[2:-2, 2:-2])
+        e_sf = rel_err(g.get("SF"), o.plane(oracle.OR_SF))
+        print(f"q={q} vis {e_vis:.1e} SF {e_sf:.1e}", flush=True)
+        assert e_vis <= 1e-13 and e_sf <= 1e-10
+    o.close()

@@ -387,7 +387,11 @@ int smoother_vis_host(tc_ctx* ctx, tc_dev& d, int level, int interpolate)
 // level took, and reads the loop state once per batch; queued iterations
 // after the exit do nothing.  The Chebyshev factors are the host table of
 // the same formula, so the sweeps see the same values.
-int smoother_vis(tc_ctx* ctx, tc_dev& d, int level, int interpolate)
+// The loop's state at entry may stand after sweeps that no test precedes
+// (entered: level 1's first pass done by vis_sweeps); Vfine: the finer
+// level's viscosity (level > 1).
+int smoother_vis(tc_ctx* ctx, tc_dev& d, int level, int interpolate, const double* Vfine = nullptr,
+                 bool entered = false)
 {
     Level& L = ctx->lv[level];
     const tc_params& p = ctx->p;
@@ -395,12 +399,12 @@ int smoother_vis(tc_ctx* ctx, tc_dev& d, int level, int interpolate)
     double lb, la;
     if (level == 1 && interpolate == 0) { option = 1; Niter = 6; lb = -5.0; la = -2.0; }
     else { option = 0; Niter = p.vis_iter; lb = -2.0; la = -1.0; }
-    if (Niter > VIS_CMAX || p.vis_iter > VIS_CMAX) return smoother_vis_host(ctx, d, level, interpolate);
+    if (!entered && (Niter > VIS_CMAX || p.vis_iter > VIS_CMAX)) return smoother_vis_host(ctx, d, level, interpolate);
     if (interpolate == 0 || level == 1) { ctx->Nvis_store = 0; ctx->nn_store = 1; }
     int kmin, kmax;
     if (p.RaT == 0.0) { kmin = 0; kmax = L.g.nz; } else { kmin = 1; kmax = L.g.nz - 1; }
     const Grid* gf = level > 1 ? &ctx->lv[level - 1].g : &L.g;
-    const double* Vf = level > 1 ? ctx->lv[level - 1].vis : nullptr;
+    const double* Vf = level > 1 ? (Vfine ? Vfine : ctx->lv[level - 1].vis) : nullptr;
     auto cfac = [](int N, int nn, double lbv, double lav) {
         const int ntemp = N - nn + 1;
         return 2.0 / (-lbv - lav + (lbv - lav) * std::cos((double)(2 * ntemp - 1) * PII / (double)(2 * N)));
@@ -417,6 +421,7 @@ int smoother_vis(tc_ctx* ctx, tc_dev& d, int level, int interpolate)
     // the state at entry; a first pass that starts beyond its end is only
     // the pass bookkeeping (the reference's inner loop does not run)
     int nn0 = ctx->nn_store, n0 = 0, Nvs = ctx->Nvis_store, tab = (option == 1) ? 0 : 1, Ncur = Niter;
+    if (entered) { n0 = 1; Nvs = 1; Ncur = 6; tab = 1; }
     while (nn0 > Ncur) {
         ++Nvs;
         nn0 = 1;
@@ -444,7 +449,7 @@ int smoother_vis(tc_ctx* ctx, tc_dev& d, int level, int interpolate)
                            d.vdctl + jn * VD_COUNT, d.vslots + j * slot_set, d.vslots + jn * slot_set, P};
             // the ratio's block minima into the slots and the copy that the sweep reads
             launch_vis_grad_eig(ctx->stream, d.pow2[level], L, d.F, d.h[level], p.ivis, e, 1, nullptr,
-                                lp.ctl_in + VC_DONE, L.vtmp, false, d.vslots + j * slot_set);
+                                lp.ctl_in + VC_DONE, L.vtmp, 0, d.vslots + j * slot_set);
             // the decision, the sweep and viscosityBCs in one launch
             launch_vis_sweep_bcs(ctx->stream, d.pow2[level], L.vtmp, L.vis, L.dtvis, L.g, d.F, d.h[level], kmin, kmax,
                                  lp, Vf, *gf, level, p.RaT, p.visT * p.visT);
@@ -492,31 +497,97 @@ int save_restore_level(tc_ctx* ctx, Level& L, bool save)
     return 0;
 }
 
+// The Chebyshev sweeps first..last (of Niter) of a pass of smoother_vis, with
+// their viscosityBCs, from the level's viscosity into dst (the viscosity itself,
+// or another plane of the level); tmp: a third plane.  Nothing to do: dst is
+// not written.
+int vis_sweeps(tc_ctx* ctx, tc_dev& d, int level, int first, int last, int Niter, double lb, double la, double* dst,
+               double* tmp, const double* Vf)
+{
+    Level& L = ctx->lv[level];
+    const tc_params& p = ctx->p;
+    const int n = last - first + 1, K = vis_multi_k();
+    if (n <= 0) return 0;
+    // an even number of launches where the result returns to its source
+    int m = (n + K - 1) / K;
+    if (dst == L.vis && m % 2) ++m;
+    const Grid& gf = level > 1 ? ctx->lv[level - 1].g : L.g;
+    const double* in = L.vis;
+    int nn = first;
+    for (int j = 1; j <= m; ++j) {
+        const int left = m - j + 1, nk = (last - nn + 1 + left - 1) / left;
+        std::vector<double> fac(nk);
+        for (int s = 0; s < nk; ++s) {
+            const int ntemp = Niter - (nn + s) + 1;
+            fac[s] = 2.0 / (-lb - la + (lb - la) * std::cos((double)(2 * ntemp - 1) * PII / (double)(2 * Niter)));
+        }
+        double* out = ((m - j) % 2 == 0) ? dst : tmp;
+        launch_vis_multi(ctx->stream, d.pow2[level], in, out, L.dtvis, L.g, d.h[level], fac.data(), nk, Vf, gf,
+                         p.visT * p.visT, d.cus);
+        in = out;
+        nn += nk;
+    }
+    return 0;
+}
+
 // compute_viscosity (iterative_solver.f90:331-377)
 int compute_viscosity(tc_ctx* ctx, tc_dev& d, int level)
 {
     const tc_params& p = ctx->p;
+    // the passes that run to their end without a test that could stop them
+    // (smoother.f90:165-263) go several sweeps a launch
+    const bool multi = d.std_tables && p.RaT != 0.0 && p.ivis != 0;
     if (level == 1) {
         RaCArr lc{};
         PtrArr cv{};
         for (int t = 0; t < p.ntype; ++t) { lc.v[t] = (p.comp == 1 && p.ivis == 2) ? std::log(p.visC[t]) : 0.0; cv.v[t] = ctx->Cvis[t]; }
         launch_visf(ctx->stream, ctx->lv[1].vis, ctx->Tvis, cv, ctx->zg, ctx->lv[1].g, p.ivis, p.comp, p.ntype, p.RaT,
                     std::log(p.visT), std::log(p.visP), lc);
+        if (multi && p.vis_iter <= VIS_CMAX) {
+            // the first pass of 6; the loop then starts with its first test
+            TC_TRY(vis_sweeps(ctx, d, 1, 1, 6, 6, -5.0, -2.0, ctx->lv[1].vis, ctx->lv[1].vtmp, nullptr));
+            ctx->stats.vis_iters += 6;
+            return smoother_vis(ctx, d, 1, 0, nullptr, true);
+        }
         return smoother_vis(ctx, d, 1, 0);
     }
     Level& Lf = ctx->lv[level - 1];
     Level& L = ctx->lv[level];
-    TC_TRY(save_restore_level(ctx, Lf, true));
-    TC_TRY(smoother_vis(ctx, d, level - 1, 1));
-    launch_restrict(ctx->stream, Lf.vis, Lf.g, L.vis, L.g);
-    launch_visc_bcs(ctx->stream, L.vis, L.g, Lf.vis, Lf.g, level, 1, p.RaT, p.visT * p.visT);
+    const double* Vs = Lf.vis;  // the finer viscosity that the restriction takes
+    if (multi) {
+        // smoother_vis(level - 1, interpolate = 1) on a plane of its own: the
+        // level's viscosity and gradients stay as they are (the reference
+        // saves and restores them).  It sweeps from where the level's own pass
+        // stopped to the end of the pass, or not at all after a whole pass.
+        if (level - 1 == 1) { ctx->Nvis_store = 0; ctx->nn_store = 1; }
+        const int first = ctx->nn_store;
+        const bool sweep = ctx->Nvis_store < 1;
+        if (sweep && first <= p.vis_iter) {
+            TC_TRY(vis_sweeps(ctx, d, level - 1, first, p.vis_iter, p.vis_iter, -2.0, -1.0, Lf.visf, Lf.vtmp,
+                              level > 2 ? ctx->lv[level - 2].vis : nullptr));
+            Vs = Lf.visf;
+        }
+        ctx->stats.vis_iters += (sweep ? std::max(0, p.vis_iter - first + 1) : 0) + 1;
+        if (sweep) { ctx->Nvis_store++; ctx->nn_store = 1; }
+        ctx->ratio_level = level - 1;
+        // the eigenvalue ratios of the smoothed viscosity: the sweeps of a
+        // solve read those of the last level smoothed only
+        if (level == ctx->grids)
+            launch_vis_grad_eig(ctx->stream, d.pow2[level - 1], Lf, d.F, d.h[level - 1], p.ivis, eig_scalars(p, Lf), 1,
+                                nullptr, nullptr, nullptr, 2, nullptr, Vs);
+    } else {
+        TC_TRY(save_restore_level(ctx, Lf, true));
+        TC_TRY(smoother_vis(ctx, d, level - 1, 1));
+    }
+    launch_restrict(ctx->stream, Vs, Lf.g, L.vis, L.g);
+    launch_visc_bcs(ctx->stream, L.vis, L.g, Vs, Lf.g, level, 1, p.RaT, p.visT * p.visT);
     if (level < ctx->grids) {
-        TC_TRY(smoother_vis(ctx, d, level, 0));
+        TC_TRY(smoother_vis(ctx, d, level, 0, Vs));
     } else {
         EigScalars e = eig_scalars(p, L);
         launch_vis_grad_eig(ctx->stream, d.pow2[level], L, d.F, d.h[level], p.ivis, e, 0, nullptr);
     }
-    TC_TRY(save_restore_level(ctx, Lf, false));
+    if (!multi) TC_TRY(save_restore_level(ctx, Lf, false));
     return 0;
 }
 
@@ -563,9 +634,10 @@ bool dc_blocked(const tc_ctx* ctx, const tc_dev& d, int level, bool f32)
 // coarser level's right-hand side; *rr_done says whether it did.
 // res (reference form): the residual of the result goes there where the
 // visit's last launch can form it; *res_done says whether it did.
+// vs (FP64, blocked): what the first launch does before the sweeps.
 int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, const Level& view, const float* rhs32,
                bool* first_sweep, bool zero_start = false, const RRTarget* rr = nullptr, bool* rr_done = nullptr,
-               double* res = nullptr, bool* res_done = nullptr)
+               double* res = nullptr, bool* res_done = nullptr, const VisitStart& vs = VisitStart{})
 {
     if (rr_done) *rr_done = false;
     if (res_done) *res_done = false;
@@ -643,7 +715,7 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
             } else {
                 launch_visit13_64(ctx->stream, cfg, pl.whole, use_ratio, L, view.rhs,
                                   (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk,
-                                  zsg);
+                                  zsg, n == 1 ? vs : VisitStart{});
                 L.cur = 1 - L.cur;
             }
             ++launches;
@@ -659,7 +731,7 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
             if (timed && !timed_visit) TC_TRY(prof_begin(ctx));
             launch_visit_ref(ctx->stream, plan, d.pow2[level], use_ratio, view, view.rhs,
                              (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk, zsg,
-                             with_res ? res : nullptr);
+                             with_res ? res : nullptr, n == 1 ? vs : VisitStart{});
             if (timed && !timed_visit) TC_TRY(prof_end(ctx, 1));
             if (with_res && res_done) *res_done = true;
             L.cur = 1 - L.cur;
@@ -696,13 +768,14 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
 
 // zero_start: the visit starts from a zero correction, which error(level)
 // does not hold yet
-int iterate_stream(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool& first_sweep, bool zero_start)
+int iterate_stream(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool& first_sweep, bool zero_start,
+                   const VisitStart& vs)
 {
     Level& L = ctx->lv[level];
     const tc_params& P = ctx->p;
     bool res_done = false;
     TC_TRY(run_sweeps(ctx, d, level, Niter, dir, false, L, nullptr, &first_sweep, zero_start, nullptr, nullptr,
-                      level > 1 ? L.res : nullptr, &res_done));
+                      level > 1 ? L.res : nullptr, &res_done, vs));
     if (res_done) {
         ctx->stats.residuals_exec[level - 1]++;
         return 0;
@@ -867,6 +940,9 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
     const int* multi = P.multi;
     int q = 1;
     int status = 0;
+    // the restriction or prolongation that the next visit's first launch does
+    const bool fold = P.Nmulti > 0 && ref_blocked(ctx, d);
+    VisitStart vs;
     for (;;) {
         bool done = false;
         for (int p = 1; p <= P.nsteps; ++p) {
@@ -876,7 +952,8 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
             if (multi[p - 1] < multi[p]) {
                 // compute_RHS(level) = restrict(residual of level-1)
                 Level& Lf = ctx->lv[level - 1];
-                launch_restrict(ctx->stream, Lf.res, Lf.g, ctx->lv[level].rhs, ctx->lv[level].g);
+                if (fold && level < G) { vs.resf = Lf.res; vs.gf = Lf.g; }
+                else launch_restrict(ctx->stream, Lf.res, Lf.g, ctx->lv[level].rhs, ctx->lv[level].g);
                 // (the blocked sweeps of a visit start from zeros without a fill)
                 zero_start = (P.fixes & TC_FIX_ZERO_COARSE) && level < G && P.Nmulti > 0 && ref_blocked(ctx, d);
                 if ((P.fixes & TC_FIX_ZERO_COARSE) && !zero_start) {
@@ -885,7 +962,8 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
                 }
             }
             if (level < G) {
-                TC_TRY(iterate_stream(ctx, d, level, P.Nmulti, dir, first_sweep, zero_start));
+                TC_TRY(iterate_stream(ctx, d, level, P.Nmulti, dir, first_sweep, zero_start, vs));
+                vs = VisitStart{};
             } else {
                 Level& Lc = ctx->lv[G];
                 TC_TRY(wait_coarse(ctx, d));
@@ -903,7 +981,8 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
             if (multi[p + 1] < multi[p]) {
                 Level& Lc = ctx->lv[level];
                 Level& Lf = ctx->lv[level - 1];
-                launch_prolong(ctx->stream, Lf.err[Lf.cur], Lf.g, Lc.err[Lc.cur], Lc.g, zsg);
+                if (fold) { vs.Ec = Lc.err[Lc.cur]; vs.gc = Lc.g; }
+                else launch_prolong(ctx->stream, Lf.err[Lf.cur], Lf.g, Lc.err[Lc.cur], Lc.g, zsg);
             }
         }
         ctx->stats.mg_cycles++;
@@ -1131,28 +1210,34 @@ int dc_alloc(tc_ctx* ctx)
 
 // Jacobi-Richardson sweeps of one visit on a correction level (FP32 or
 // FP64), followed (level > 1) by compute_residual of the level.
+// sweeps of a visit; a per-level count applies to the tuned cycle, not to the
+// Nmulti retry
+int dc_visit_sweeps(const tc_ctx* ctx, int level)
+{
+    const int n = ctx->dc_sweeps_active;
+    return (ctx->dc_level_sweeps[level] > 0 && ctx->dc_sweeps > 0 && n == ctx->dc_sweeps) ? ctx->dc_level_sweeps[level] : n;
+}
+
 int dc_iterate(tc_ctx* ctx, tc_dev& d, int level, int dir, bool f32, bool zero_start = false,
-               const RRTarget* rr = nullptr, bool* rr_done = nullptr)
+               const RRTarget* rr = nullptr, bool* rr_done = nullptr, const VisitStart& vs = VisitStart{})
 {
     Level& L = ctx->lv[level];
-    const tc_params& P = ctx->p;
     // level 1 smooths the correction against the defect of psi
     Level view = L;
     if (level == 1) view.rhs = L.res;
     const float* rhs32 = (level == 1) ? L.res32 : L.rhs32;
-    // a per-level count applies to the tuned cycle, not to the Nmulti retry
     if (level == 1) zero_start = dc_blocked(ctx, d, 1, f32);  // e(1) is zero at the start of every visit
-    int n = ctx->dc_sweeps_active;
-    if (ctx->dc_level_sweeps[level] > 0 && ctx->dc_sweeps > 0 && n == ctx->dc_sweeps) n = ctx->dc_level_sweeps[level];
+    const int n = dc_visit_sweeps(ctx, level);
     if (n <= 0 && zero_start) {  // no sweep that would write the zeros
         if (f32) launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err32[L.cur32]), L.g.elems);
         else launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err[L.cur]), 2 * L.g.elems);
     }
-    TC_TRY(run_sweeps(ctx, d, level, n, dir, f32, view, rhs32, nullptr, zero_start, rr, rr_done));
+    TC_TRY(run_sweeps(ctx, d, level, n, dir, f32, view, rhs32, nullptr, zero_start, rr, rr_done, nullptr, nullptr,
+                      vs));
     // FP64: compute_residual now; FP32: fused into the restriction of the
     // next descent (k_residual_restrict32), the only reader of the residual
     if (level > 1 && !f32) {
-        launch_residual(ctx->stream, d.pow2[level], L, L.err[L.cur], L.res, d.F, d.h[level], P.ivis, nullptr);
+        launch_residual(ctx->stream, d.pow2[level], L, L.err[L.cur], L.res, d.F, d.h[level], ctx->p.ivis, nullptr);
         ctx->stats.residuals_exec[level - 1]++;
     }
     return 0;
@@ -1434,6 +1519,10 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
         }
         return st;
     };
+    // FP64 corrections: the restriction or prolongation that the next visit's
+    // first launch does
+    VisitStart vs64;
+    auto fold64 = [&](int level) { return !f32 && level < G && dc_blocked(ctx, d, level, f32) && dc_visit_sweeps(ctx, level) > 0; };
     bool coarse_b_ready = false;  // the coarse right-hand side was formed by the descent
     int rr_level = 0;             // the level whose right-hand side the last visit formed
     // one step p of the cycle schedule: the descent into the level, its
@@ -1471,7 +1560,8 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                 if (!zero_start && level < G)
                     launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err32[L.cur32]), L.g.elems);
             } else {
-                launch_restrict(ctx->stream, Lf.res, Lf.g, L.rhs, L.g);
+                if (fold64(level)) { vs64.resf = Lf.res; vs64.gf = Lf.g; }
+                else launch_restrict(ctx->stream, Lf.res, Lf.g, L.rhs, L.g);
                 if (!zero_start) TC_HIP(hipMemsetAsync(L.err[L.cur], 0, plane_bytes(L.g), ctx->stream));
             }
         }
@@ -1492,7 +1582,8 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                 }
             }
             bool fused = false;
-            TC_TRY(dc_iterate(ctx, d, level, dir, f32, zero_start, want_rr ? &rrt : nullptr, &fused));
+            TC_TRY(dc_iterate(ctx, d, level, dir, f32, zero_start, want_rr ? &rrt : nullptr, &fused, vs64));
+            vs64 = VisitStart{};
             if (fused) {
                 rr_level = level + 1;
                 ctx->stats.residuals_exec[level - 1]++;
@@ -1539,6 +1630,9 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                 ctx->pend_from = level;
             } else if (f32) {
                 launch_prolong32(ctx->stream, Lf.err32[Lf.cur32], Lf.g, L.err32[L.cur32], L.g, zsg);
+            } else if (fold64(level - 1) && multi[p + 1] == level - 1) {
+                vs64.Ec = L.err[L.cur];
+                vs64.gc = L.g;
             } else {
                 launch_prolong(ctx->stream, Lf.err[Lf.cur], Lf.g, L.err[L.cur], L.g, zsg);
             }

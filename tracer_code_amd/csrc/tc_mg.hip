@@ -102,12 +102,7 @@ __global__ __launch_bounds__(256) void k_restrict(const double* __restrict__ in,
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int k = blockIdx.y * blockDim.y + threadIdx.y + 1;
     if (i > go.nx - 1 || k > go.nz - 1) return;
-    const int ii = 2 * i, kk = 2 * k;
-    double corners = (in[gi.at(ii - 1, kk - 1)] + in[gi.at(ii - 1, kk + 1)] + in[gi.at(ii + 1, kk + 1)] +
-                      in[gi.at(ii - 1, kk + 1)]) / 16.0;
-    double sides = (in[gi.at(ii - 1, kk)] + in[gi.at(ii, kk - 1)] + in[gi.at(ii + 1, kk)] + in[gi.at(ii, kk + 1)]) / 8.0;
-    double centre = in[gi.at(ii, kk)] / 4.0;
-    out[go.at(i, k)] = corners + sides + centre;
+    out[go.at(i, k)] = restrict_at(in, gi, i, k);
 }
 
 // prolong (iterative_solver.f90:175-233): one thread per fine interior
@@ -120,15 +115,7 @@ __global__ __launch_bounds__(256) void k_prolong(double* __restrict__ Ef, Grid g
     const int k = blockIdx.y * blockDim.y + threadIdx.y + 1;
     if (i > gf.nx - 1 || k > gf.nz - 1) return;
     const size_t c = gf.at(i, k);
-    double add;
-    const bool ie = (i % 2) == 0, ke = (k % 2) == 0;
-    if (ie && ke) add = Ec[gc.at(i / 2, k / 2)];
-    else if (ie) add = (Ec[gc.at(i / 2, (k - 1) / 2)] + Ec[gc.at(i / 2, (k + 1) / 2)]) / 2.0;
-    else if (ke) add = (Ec[gc.at((i - 1) / 2, k / 2)] + Ec[gc.at((i + 1) / 2, k / 2)]) / 2.0;
-    else
-        add = (Ec[gc.at((i - 1) / 2, (k - 1) / 2)] + Ec[gc.at((i + 1) / 2, (k - 1) / 2)] +
-               Ec[gc.at((i + 1) / 2, (k + 1) / 2)] + Ec[gc.at((i - 1) / 2, (k + 1) / 2)]) / 4.0;
-    double v = Ef[c] + add;
+    double v = Ef[c] + prolong_at(Ec, gc, i, k);
     Ef[c] = v;
     stream_ghosts(Ef, gf, i, k, v, zsg);
 }
@@ -269,9 +256,10 @@ __device__ void vis_decide(double a, const VisDecide& P, int32_t* __restrict__ c
 // minima of the ratio for smoother_vis (smoother.f90:209).  gate: the
 // device-controlled smoother_vis loop has stopped; copy_dst: the plane V is
 // also copied there (the source of the iteration's sweep, which the loop's
-// decision may still switch off; the copy is then unused); store = 0: the gradient and
-// ratio planes are not written (inside the loop only the block minima are
-// read, and the planes are written from the final viscosity after it);
+// decision may still switch off; the copy is then unused); store: 1 = the gradient
+// planes are written, 2 = the ratio plane (inside the loop only the block
+// minima are read, and the planes are written from the final viscosity after
+// it);
 // slots: each block's minimum also goes into slot blk % VIS_SLOTS by atomicMin
 // (the loop's decision reads the minimum of the slots in the next launch).
 template <bool POW2>
@@ -310,7 +298,7 @@ __global__ __launch_bounds__(256) void k_vis_grad_eig(const double* __restrict__
             gzz = sdiv<POW2>(dot3g<1>(F.D2, S), h.ds2, h.ids2);
             gxz = sdiv<POW2>(sum9g(F.Drs, S), h.drds, h.idrds);
         }
-        if (store) { vx[c] = gx; vz[c] = gz; vxx[c] = gxx; vzz[c] = gzz; vxz[c] = gxz; }
+        if (store & 1) { vx[c] = gx; vz[c] = gz; vxx[c] = gxx; vzz[c] = gzz; vxz[c] = gxz; }
         if (want_ratio && ivis != 0) {
             const double vis = S(0, 0);
             // eigI with xr=zs=1, xrr=..=0: only the odd-derivative terms survive
@@ -329,7 +317,7 @@ __global__ __launch_bounds__(256) void k_vis_grad_eig(const double* __restrict__
             double r6 = 2.0 * gz * (0.0 + 0.0);
             double eR = -(r1 + r2 + r3 + r4 + r5 + r6);
             double r = fabs(eR / eI);
-            if (store) ratio[c] = r;
+            if (store & 2) ratio[c] = r;
             m = r;
         }
     }
@@ -568,6 +556,157 @@ __global__ __launch_bounds__(256) void k_vis_sweep_bcs(const double* __restrict_
 }
 
 // ---------------------------------------------------------------------------
+// The sweeps of smoother_vis (smoother.f90:239-263) that no test can cut
+// short, several per launch, with the viscosity in registers: the passes of
+// the interpolation (interpolate = 1) stop after a whole pass, and level 1's
+// first pass (6 sweeps) precedes its first test.  Each iteration of the tested
+// loop is two launches (the eigenvalue ratios, then the sweep) and a copy,
+// 32.4 us at 2048x1024 and 9 us on a small level.
+//
+// Each wavefront holds 64 columns, one per lane, by rows in the lane's
+// registers, with a halo of VM_H cells, as k_filter_multi does: x neighbours
+// by lane shifts, z neighbours from the lane's own rows.  dt_vis is one value
+// on the uniform grids the library accepts.  Rows 0 and nz are not swept
+// (RaT != 0); viscosityBCs gives them the finer level's values on levels > 1.
+// The first tile starts at row 0, the last one ends at row nz, and those
+// between hold neither (ZK = 1, 2, 0); where one tile holds all rows (nz <=
+// VM_ALL - 1) they are its first and row nz (ZK = 3).  The result is written
+// with the ghosts that viscosityBCs leaves after the last sweep.  The values
+// are k_vis_sweep_bcs's, bit for bit.  Measured, 12 sweeps in 2 launches
+// against 24: 2048x1024 42 against 391 us, 64x64 21 against 108, at most 33
+// rows 29 against 106.
+// ---------------------------------------------------------------------------
+constexpr int VM_K = 6;                  // sweeps of a launch
+constexpr int VM_H = VM_K;
+constexpr int VM_TXO = 64 - 2 * VM_H;    // own columns
+constexpr int VM_WAVES = 4;
+constexpr int VM_ALL = 33;               // rows of a tile that holds all of them
+constexpr int VM_TYS[2] = {14, 24};      // own rows of the other tiles (nz >= TY + 2 VM_H + 1)
+
+struct VmFac { double v[VM_K]; };
+
+__device__ __forceinline__ double vm_left(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x138, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(lo, 0x138, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double vm_right(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x130, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(lo, 0x130, 0xF, 0xF, true));
+}
+
+template <bool POW2, int RY, int TY, int ZK>
+__device__ __forceinline__ void vm_iterate(double (&c)[RY], int n, const double* fac, double dt, const Spacing& h,
+                                           bool gcols, bool ghost_col, int ml, double w0, double wn, int nz)
+{
+    constexpr int R0 = ZK == 3 ? 0 : VM_H, RN = VM_H + TY - 1;  // rows 0 and nz of the first and the last tile
+#pragma unroll 1
+    for (int it = 0; it < n; ++it) {
+        const double cd = fac[it] * dt;
+        double om = c[0];
+#pragma unroll
+        for (int r = 1; r < RY - 1; ++r) {
+            const double oc = c[r];
+            const double lf = vm_left(oc), rt = vm_right(oc);
+            const double x = fma(-2.0, oc, lf) + rt, z = fma(-2.0, oc, om) + c[r + 1];
+            double temp;
+            if constexpr (POW2) temp = fma(x, h.idr2, z * h.ids2);
+            else temp = div_by(x, h.dr2, h.idr2) + div_by(z, h.ds2, h.ids2);
+            c[r] = oc + cd * temp;
+            om = oc;
+        }
+        // rows 0 and nz: the values viscosityBCs leaves there
+        if constexpr (ZK == 1 || ZK == 3) c[R0] = w0;
+        if constexpr (ZK == 2) c[RN] = wn;
+        if constexpr (ZK == 3) {
+#pragma unroll
+            for (int r = 1; r < RY; ++r)
+                if (r == nz) c[r] = wn;
+        }
+        // ghost columns: the mirrored lane's new value
+        if (gcols) {
+#pragma unroll
+            for (int r = 0; r < RY; ++r) {
+                const double mv = __shfl(c[r], ml, 64);
+                c[r] = ghost_col ? mv : c[r];
+            }
+        }
+    }
+}
+
+template <bool POW2, int TY, bool ALL>
+__global__ __launch_bounds__(256) void k_vis_multi(const double* __restrict__ V0, double* __restrict__ V,
+                                                   const double* __restrict__ dtv, Grid g, Spacing h, VmFac fac, int n,
+                                                   int tiles, const double* __restrict__ Vf, Grid gf, double visT2)
+{
+    constexpr int RY = ALL ? VM_ALL : TY + 2 * VM_H;
+    const int nx = g.nx, nz = g.nz, lane = threadIdx.x;
+    const int t = blockIdx.y * blockDim.y + __builtin_amdgcn_readfirstlane(threadIdx.y);  // the wave's tile
+    if (t >= tiles) return;
+    const int zk = ALL ? 3 : (t == 0 ? 1 : (t == tiles - 1 ? 2 : 0));
+    int k0 = t * TY;
+    if (!ALL && t > 0) k0 = t == tiles - 1 ? nz + 1 - TY : min(k0, nz - VM_H - TY);
+    const int i0 = blockIdx.x * VM_TXO, rk0 = ALL ? 0 : k0 - VM_H;
+    const int i = i0 - VM_H + lane;
+    const bool col_in = i >= -1 && i <= nx + 1;
+    const int im = (i < 0) ? -i : (i > nx ? 2 * nx - i : i);
+    int ml = lane + (im - i);
+    ml = ml < 0 ? 0 : (ml > 63 ? 63 : ml);
+    const double dt = dtv[g.at(0, 1)] * 0.99;  // (rows 0 and nz are not swept and hold 0)
+    double c[RY];
+    const double* __restrict__ sp = V0 + g.at(col_in ? i : 0, 0);
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+        const int k = rk0 + r;
+        const bool in = k >= 0 && k <= nz;
+        const double v = sp[(ptrdiff_t)(in ? k : 0) * g.ld];
+        c[r] = (col_in && in) ? v : 0.0;
+    }
+    // rows 0 and nz after a sweep's boundary routine
+    const bool own = i >= 0 && i <= nx;
+    double w0 = sp[0], wn = sp[(ptrdiff_t)nz * g.ld];
+    if (Vf && own) {
+        w0 = Vf[gf.at(2 * i, 0)];
+        wn = Vf[gf.at(2 * i, gf.nz)];
+    }
+    const bool gcols = i0 - VM_H <= -1 || i0 - VM_H + 63 >= nx + 1, ghost_col = col_in && !own;
+    if constexpr (ALL) {
+        vm_iterate<POW2, RY, TY, 3>(c, n, fac.v, dt, h, gcols, ghost_col, ml, w0, wn, nz);
+    } else {
+        if (zk == 0) vm_iterate<POW2, RY, TY, 0>(c, n, fac.v, dt, h, gcols, ghost_col, ml, w0, wn, nz);
+        else if (zk == 1) vm_iterate<POW2, RY, TY, 1>(c, n, fac.v, dt, h, gcols, ghost_col, ml, w0, wn, nz);
+        else vm_iterate<POW2, RY, TY, 2>(c, n, fac.v, dt, h, gcols, ghost_col, ml, w0, wn, nz);
+    }
+    if (!own || i < i0 || i >= i0 + VM_TXO) return;
+    const bool lo_i = i >= 1 && i <= SPAN, hi_i = i >= nx - SPAN && i <= nx - 1;
+    constexpr int FIRST = ALL ? 0 : VM_H, OWN = ALL ? VM_ALL : TY;
+#pragma unroll
+    for (int r = 0; r < OWN; ++r) {
+        const int k = k0 + r;
+        if (ALL && k > nz) continue;
+        const double v = c[FIRST + r];
+        V[g.at(i, k)] = v;
+        if (lo_i) V[g.at(-i, k)] = v;
+        if (hi_i) V[g.at(2 * nx - i, k)] = v;
+        if (k >= 1 && k <= SPAN) {
+            const double b = 1.0 / v / visT2;
+            V[g.at(i, -k)] = b;
+            if (lo_i) V[g.at(-i, -k)] = b;
+            if (hi_i) V[g.at(2 * nx - i, -k)] = b;
+        }
+        if (k >= nz - SPAN && k <= nz - 1) {
+            const double b = 1.0 / v;
+            V[g.at(i, 2 * nz - k)] = b;
+            if (lo_i) V[g.at(-i, 2 * nz - k)] = b;
+            if (hi_i) V[g.at(2 * nx - i, 2 * nz - k)] = b;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Host-side launchers
 // ---------------------------------------------------------------------------
 static inline dim3 grid2(int nx, int ny, dim3 b) { return dim3((nx + b.x - 1) / b.x, (ny + b.y - 1) / b.y); }
@@ -657,16 +796,17 @@ void launch_visf(hipStream_t st, double* vis, const double* Tvis, const PtrArr& 
 
 int launch_vis_grad_eig(hipStream_t st, bool pow2, Level& L, const FD& F, const Spacing& h, int ivis,
                         const EigScalars& e, int want_ratio, double* partial, const int32_t* gate,
-                        double* copy_dst, bool store, unsigned long long* slots)
+                        double* copy_dst, int store, unsigned long long* slots, const double* V)
 {
     dim3 b(64, 4);
     dim3 gr = grid2(L.g.nx - 1, L.g.nz - 1, b);
+    if (!V) V = L.vis;
     if (pow2)
-        hipLaunchKernelGGL((k_vis_grad_eig<true>), gr, b, 0, st, L.vis, L.visx, L.visz, L.visxx, L.viszz, L.visxz,
-                           L.ratio, L.g, F, h, ivis, e, want_ratio, partial, gate, copy_dst, store ? 1 : 0, slots);
+        hipLaunchKernelGGL((k_vis_grad_eig<true>), gr, b, 0, st, V, L.visx, L.visz, L.visxx, L.viszz, L.visxz,
+                           L.ratio, L.g, F, h, ivis, e, want_ratio, partial, gate, copy_dst, store, slots);
     else
-        hipLaunchKernelGGL((k_vis_grad_eig<false>), gr, b, 0, st, L.vis, L.visx, L.visz, L.visxx, L.viszz, L.visxz,
-                           L.ratio, L.g, F, h, ivis, e, want_ratio, partial, gate, copy_dst, store ? 1 : 0, slots);
+        hipLaunchKernelGGL((k_vis_grad_eig<false>), gr, b, 0, st, V, L.visx, L.visz, L.visxx, L.viszz, L.visxz,
+                           L.ratio, L.g, F, h, ivis, e, want_ratio, partial, gate, copy_dst, store, slots);
     return (int)(gr.x * gr.y);
 }
 
@@ -701,6 +841,48 @@ void launch_vis_sweep_bcs(hipStream_t st, bool pow2, const double* T0, double* V
     else
         hipLaunchKernelGGL((k_vis_sweep_bcs<false>), gr, b, 0, st, T0, V, dtv, g, F, h, kmin, kmax, lp, Vf, gf, level,
                            RaT, visT2);
+}
+
+int vis_multi_k() { return VM_K; }
+
+template <bool POW2, int TY, bool ALL>
+static void vis_multi_go(hipStream_t st, const double* V0, double* V, const double* dtv, const Grid& g,
+                         const Spacing& h, const VmFac& f, int n, int tiles, const double* Vf, const Grid& gf,
+                         double visT2)
+{
+    const int wz = ALL ? 1 : VM_WAVES;
+    const dim3 gr((unsigned)((g.nx + VM_TXO) / VM_TXO), (unsigned)((tiles + wz - 1) / wz));
+    hipLaunchKernelGGL((k_vis_multi<POW2, TY, ALL>), gr, dim3(64, wz), 0, st, V0, V, dtv, g, h, f, n, tiles, Vf, gf,
+                       visT2);
+}
+
+void launch_vis_multi(hipStream_t st, bool pow2, const double* V0, double* V, const double* dtv, const Grid& g,
+                      const Spacing& h, const double* fac, int n, const double* Vf, const Grid& gf, double visT2,
+                      int cus)
+{
+    VmFac f{};
+    for (int s = 0; s < n; ++s) f.v[s] = fac[s];
+    // rows of a tile: the first and the last, and those between over the rest
+    auto tiles_of = [&](int ty) {
+        const int rest = g.nz + 1 - 2 * ty;
+        return 2 + (rest > 0 ? (rest + ty - 1) / ty : 0);
+    };
+    auto go = [&](auto pw) {
+        constexpr bool P = decltype(pw)::value;
+        if (g.nz < VM_ALL) {
+            vis_multi_go<P, VM_ALL, true>(st, V0, V, dtv, g, h, f, n, 1, Vf, gf, visT2);
+            return;
+        }
+        // the taller tile (less halo) once the shorter ones take more than
+        // a workgroup per CU
+        const int gx = (g.nx + VM_TXO) / VM_TXO;
+        if ((long)gx * ((tiles_of(VM_TYS[0]) + VM_WAVES - 1) / VM_WAVES) <= cus || g.nz < VM_TYS[1] + 2 * VM_H + 1)
+            vis_multi_go<P, VM_TYS[0], false>(st, V0, V, dtv, g, h, f, n, tiles_of(VM_TYS[0]), Vf, gf, visT2);
+        else
+            vis_multi_go<P, VM_TYS[1], false>(st, V0, V, dtv, g, h, f, n, tiles_of(VM_TYS[1]), Vf, gf, visT2);
+    };
+    if (pow2) go(std::integral_constant<bool, true>{});
+    else go(std::integral_constant<bool, false>{});
 }
 
 void launch_visc_bcs(hipStream_t st, double* V, const Grid& g, const double* Vf, const Grid& gf, int level, int init,
