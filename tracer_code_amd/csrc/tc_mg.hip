@@ -102,7 +102,12 @@ __global__ __launch_bounds__(256) void k_restrict(const double* __restrict__ in,
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int k = blockIdx.y * blockDim.y + threadIdx.y + 1;
     if (i > go.nx - 1 || k > go.nz - 1) return;
-    out[go.at(i, k)] = restrict_at(in, gi, i, k);
+    const int ii = 2 * i, kk = 2 * k;
+    double corners = (in[gi.at(ii - 1, kk - 1)] + in[gi.at(ii - 1, kk + 1)] + in[gi.at(ii + 1, kk + 1)] +
+                      in[gi.at(ii - 1, kk + 1)]) / 16.0;
+    double sides = (in[gi.at(ii - 1, kk)] + in[gi.at(ii, kk - 1)] + in[gi.at(ii + 1, kk)] + in[gi.at(ii, kk + 1)]) / 8.0;
+    double centre = in[gi.at(ii, kk)] / 4.0;
+    out[go.at(i, k)] = corners + sides + centre;
 }
 
 // prolong (iterative_solver.f90:175-233): one thread per fine interior
@@ -115,7 +120,15 @@ __global__ __launch_bounds__(256) void k_prolong(double* __restrict__ Ef, Grid g
     const int k = blockIdx.y * blockDim.y + threadIdx.y + 1;
     if (i > gf.nx - 1 || k > gf.nz - 1) return;
     const size_t c = gf.at(i, k);
-    double v = Ef[c] + prolong_at(Ec, gc, i, k);
+    double add;
+    const bool ie = (i % 2) == 0, ke = (k % 2) == 0;
+    if (ie && ke) add = Ec[gc.at(i / 2, k / 2)];
+    else if (ie) add = (Ec[gc.at(i / 2, (k - 1) / 2)] + Ec[gc.at(i / 2, (k + 1) / 2)]) / 2.0;
+    else if (ke) add = (Ec[gc.at((i - 1) / 2, k / 2)] + Ec[gc.at((i + 1) / 2, k / 2)]) / 2.0;
+    else
+        add = (Ec[gc.at((i - 1) / 2, (k - 1) / 2)] + Ec[gc.at((i + 1) / 2, (k - 1) / 2)] +
+               Ec[gc.at((i + 1) / 2, (k + 1) / 2)] + Ec[gc.at((i - 1) / 2, (k + 1) / 2)]) / 4.0;
+    double v = Ef[c] + add;
     Ef[c] = v;
     stream_ghosts(Ef, gf, i, k, v, zsg);
 }
@@ -561,7 +574,7 @@ __global__ __launch_bounds__(256) void k_vis_sweep_bcs(const double* __restrict_
 // the interpolation (interpolate = 1) stop after a whole pass, and level 1's
 // first pass (6 sweeps) precedes its first test.  Each iteration of the tested
 // loop is two launches (the eigenvalue ratios, then the sweep) and a copy,
-// 32.4 us at 2048x1024 and 9 us on a small level.
+// 32.7 us at 2048x1024 and 9 us on a small level.
 //
 // Each wavefront holds 64 columns, one per lane, by rows in the lane's
 // registers, with a halo of VM_H cells, as k_filter_multi does: x neighbours
@@ -572,9 +585,9 @@ __global__ __launch_bounds__(256) void k_vis_sweep_bcs(const double* __restrict_
 // between hold neither (ZK = 1, 2, 0); where one tile holds all rows (nz <=
 // VM_ALL - 1) they are its first and row nz (ZK = 3).  The result is written
 // with the ghosts that viscosityBCs leaves after the last sweep.  The values
-// are k_vis_sweep_bcs's, bit for bit.  Measured, 12 sweeps in 2 launches
-// against 24: 2048x1024 42 against 391 us, 64x64 21 against 108, at most 33
-// rows 29 against 106.
+// are k_vis_sweep_bcs's, bit for bit.  Measured, a launch of 6
+// sweeps: 2048x1024 20.9 us, 128x128 10.7, 64x64 12.0, a level held whole
+// 14.7; one sweep by the two launches: 2048x1024 32.7 us, 152x104 9.0.
 // ---------------------------------------------------------------------------
 constexpr int VM_K = 6;                  // sweeps of a launch
 constexpr int VM_H = VM_K;
