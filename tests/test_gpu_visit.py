@@ -44,6 +44,21 @@ def test_blocked_visits_same_bits(monkeypatch, nx, nz, ov):
     assert np.array_equal(sfa, sfb) and np.array_equal(ra, rb)
 
 
+@pytest.mark.parametrize("nx,nz", [(32, 32), (152, 104), (512, 320)])
+@pytest.mark.parametrize("seq", [
+    [1, 2, 3, 2, 3, 2], [2, 1, 2, 3], [1, 3, 2], [1, 2, 3, 1, 2], [1, 2, 2, 3, 2, 1], [1, 2, 3],
+], ids=lambda s: "".join(map(str, s)))
+def test_schedules_same_bits(monkeypatch, nx, nz, seq):
+    """Schedules other than the presets': they skip or repeat levels, start
+    below level 1, or end on a level from which the next cycle's first visit is
+    more than one level away."""
+    monkeypatch.setattr(config, "cycle_sequence", lambda grids, cycle="W": seq)
+    a, sfa, ra = solve(monkeypatch, "0", nx, nz, Nmulti=7, grids=3)
+    b, sfb, rb = solve(monkeypatch, "1", nx, nz, Nmulti=7, grids=3)
+    assert a == b and a[0] > 0.0
+    assert np.array_equal(sfa, sfb) and np.array_equal(ra, rb)
+
+
 @pytest.mark.parametrize("mode", ["mixed", "dc64"])
 @pytest.mark.parametrize("nx,nz,ov", [
     (32, 32, {}), (66, 34, dict(Nmulti=9)), (128, 32, dict(Nmulti=8)), (152, 104, dict(Nmulti=16)),

@@ -611,7 +611,10 @@ void cheb_factors(int n, int Niter, int dir, double& temp, double& cconst)
 // whether the reference form runs several sweeps per launch
 bool ref_blocked(const tc_ctx* ctx, const tc_dev& d)
 {
-    return d.tb && ctx->mode == TC_MODE_FP64;
+    // a schedule that does not start on level 1 spends the wall reset of a
+    // solve's first sweep on another level, and level 1 keeps SF's walls, which
+    // a blocked visit takes as zero
+    return d.tb && ctx->mode == TC_MODE_FP64 && ctx->p.multi[1] == 1;
 }
 
 // whether a level's visits in the defect-correction cycle run several sweeps
