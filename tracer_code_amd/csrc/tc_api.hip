@@ -637,9 +637,10 @@ bool dc_blocked(const tc_ctx* ctx, const tc_dev& d, int level, bool f32)
 // coarser level's right-hand side; *rr_done says whether it did.
 // res (reference form): the residual of the result goes there where the
 // visit's last launch can form it; *res_done says whether it did.
+// vs (FP64, blocked): what the first launch does before the sweeps.
 int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, const Level& view, const float* rhs32,
                bool* first_sweep, bool zero_start = false, const RRTarget* rr = nullptr, bool* rr_done = nullptr,
-               double* res = nullptr, bool* res_done = nullptr)
+               double* res = nullptr, bool* res_done = nullptr, const VisitStart& vs = VisitStart{})
 {
     if (rr_done) *rr_done = false;
     if (res_done) *res_done = false;
@@ -717,7 +718,7 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
             } else {
                 launch_visit13_64(ctx->stream, cfg, pl.whole, use_ratio, L, view.rhs,
                                   (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk,
-                                  zsg);
+                                  zsg, n == 1 ? vs : VisitStart{});
                 L.cur = 1 - L.cur;
             }
             ++launches;
@@ -733,7 +734,7 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
             if (timed && !timed_visit) TC_TRY(prof_begin(ctx));
             launch_visit_ref(ctx->stream, plan, d.pow2[level], use_ratio, view, view.rhs,
                              (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk, zsg,
-                             with_res ? res : nullptr);
+                             with_res ? res : nullptr, n == 1 ? vs : VisitStart{});
             if (timed && !timed_visit) TC_TRY(prof_end(ctx, 1));
             if (with_res && res_done) *res_done = true;
             L.cur = 1 - L.cur;
@@ -770,13 +771,14 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
 
 // zero_start: the visit starts from a zero correction, which error(level)
 // does not hold yet
-int iterate_stream(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool& first_sweep, bool zero_start)
+int iterate_stream(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool& first_sweep, bool zero_start,
+                   const VisitStart& vs)
 {
     Level& L = ctx->lv[level];
     const tc_params& P = ctx->p;
     bool res_done = false;
     TC_TRY(run_sweeps(ctx, d, level, Niter, dir, false, L, nullptr, &first_sweep, zero_start, nullptr, nullptr,
-                      level > 1 ? L.res : nullptr, &res_done));
+                      level > 1 ? L.res : nullptr, &res_done, vs));
     if (res_done) {
         ctx->stats.residuals_exec[level - 1]++;
         return 0;
@@ -941,6 +943,9 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
     const int* multi = P.multi;
     int q = 1;
     int status = 0;
+    // the restriction or prolongation that the next visit's first launch does
+    const bool fold = P.Nmulti > 0 && ref_blocked(ctx, d);
+    VisitStart vs;
     for (;;) {
         bool done = false;
         for (int p = 1; p <= P.nsteps; ++p) {
@@ -950,7 +955,8 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
             if (multi[p - 1] < multi[p]) {
                 // compute_RHS(level) = restrict(residual of level-1)
                 Level& Lf = ctx->lv[level - 1];
-                launch_restrict(ctx->stream, Lf.res, Lf.g, ctx->lv[level].rhs, ctx->lv[level].g);
+                if (fold && level < G) { vs.resf = Lf.res; vs.gf = Lf.g; }
+                else launch_restrict(ctx->stream, Lf.res, Lf.g, ctx->lv[level].rhs, ctx->lv[level].g);
                 // (the blocked sweeps of a visit start from zeros without a fill)
                 zero_start = (P.fixes & TC_FIX_ZERO_COARSE) && level < G && P.Nmulti > 0 && ref_blocked(ctx, d);
                 if ((P.fixes & TC_FIX_ZERO_COARSE) && !zero_start) {
@@ -959,7 +965,8 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
                 }
             }
             if (level < G) {
-                TC_TRY(iterate_stream(ctx, d, level, P.Nmulti, dir, first_sweep, zero_start));
+                TC_TRY(iterate_stream(ctx, d, level, P.Nmulti, dir, first_sweep, zero_start, vs));
+                vs = VisitStart{};
             } else {
                 Level& Lc = ctx->lv[G];
                 TC_TRY(wait_coarse(ctx, d));
@@ -977,7 +984,13 @@ int run_multigrid(tc_ctx* ctx, int32_t* q_out)
             if (multi[p + 1] < multi[p]) {
                 Level& Lc = ctx->lv[level];
                 Level& Lf = ctx->lv[level - 1];
-                launch_prolong(ctx->stream, Lf.err[Lf.cur], Lf.g, Lc.err[Lc.cur], Lc.g, zsg);
+                // (where the cycle's next visit is that level's)
+                if (fold && p < P.nsteps && multi[p + 1] == level - 1) {
+                    vs.Ec = Lc.err[Lc.cur];
+                    vs.gc = Lc.g;
+                } else {
+                    launch_prolong(ctx->stream, Lf.err[Lf.cur], Lf.g, Lc.err[Lc.cur], Lc.g, zsg);
+                }
             }
         }
         ctx->stats.mg_cycles++;
@@ -1203,30 +1216,36 @@ int dc_alloc(tc_ctx* ctx)
     return 0;
 }
 
+// sweeps of a visit; a per-level count applies to the tuned cycle, not to the
+// Nmulti retry
+int dc_visit_sweeps(const tc_ctx* ctx, int level)
+{
+    const int n = ctx->dc_sweeps_active;
+    return (ctx->dc_level_sweeps[level] > 0 && ctx->dc_sweeps > 0 && n == ctx->dc_sweeps) ? ctx->dc_level_sweeps[level] : n;
+}
+
 // Jacobi-Richardson sweeps of one visit on a correction level (FP32 or
 // FP64), followed (level > 1) by compute_residual of the level.
 int dc_iterate(tc_ctx* ctx, tc_dev& d, int level, int dir, bool f32, bool zero_start = false,
-               const RRTarget* rr = nullptr, bool* rr_done = nullptr)
+               const RRTarget* rr = nullptr, bool* rr_done = nullptr, const VisitStart& vs = VisitStart{})
 {
     Level& L = ctx->lv[level];
-    const tc_params& P = ctx->p;
     // level 1 smooths the correction against the defect of psi
     Level view = L;
     if (level == 1) view.rhs = L.res;
     const float* rhs32 = (level == 1) ? L.res32 : L.rhs32;
-    // a per-level count applies to the tuned cycle, not to the Nmulti retry
     if (level == 1) zero_start = dc_blocked(ctx, d, 1, f32);  // e(1) is zero at the start of every visit
-    int n = ctx->dc_sweeps_active;
-    if (ctx->dc_level_sweeps[level] > 0 && ctx->dc_sweeps > 0 && n == ctx->dc_sweeps) n = ctx->dc_level_sweeps[level];
+    const int n = dc_visit_sweeps(ctx, level);
     if (n <= 0 && zero_start) {  // no sweep that would write the zeros
         if (f32) launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err32[L.cur32]), L.g.elems);
         else launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err[L.cur]), 2 * L.g.elems);
     }
-    TC_TRY(run_sweeps(ctx, d, level, n, dir, f32, view, rhs32, nullptr, zero_start, rr, rr_done));
+    TC_TRY(run_sweeps(ctx, d, level, n, dir, f32, view, rhs32, nullptr, zero_start, rr, rr_done, nullptr, nullptr,
+                      vs));
     // FP64: compute_residual now; FP32: fused into the restriction of the
     // next descent (k_residual_restrict32), the only reader of the residual
     if (level > 1 && !f32) {
-        launch_residual(ctx->stream, d.pow2[level], L, L.err[L.cur], L.res, d.F, d.h[level], P.ivis, nullptr);
+        launch_residual(ctx->stream, d.pow2[level], L, L.err[L.cur], L.res, d.F, d.h[level], ctx->p.ivis, nullptr);
         ctx->stats.residuals_exec[level - 1]++;
     }
     return 0;
@@ -1508,6 +1527,10 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
         }
         return st;
     };
+    // FP64 corrections: the restriction or prolongation that the next visit's
+    // first launch does
+    VisitStart vs64;
+    auto fold64 = [&](int level) { return !f32 && level < G && dc_blocked(ctx, d, level, f32) && dc_visit_sweeps(ctx, level) > 0; };
     bool coarse_b_ready = false;  // the coarse right-hand side was formed by the descent
     int rr_level = 0;             // the level whose right-hand side the last visit formed
     // one step p of the cycle schedule: the descent into the level, its
@@ -1545,7 +1568,8 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                 if (!zero_start && level < G)
                     launch_zero_i32(ctx->stream, reinterpret_cast<int32_t*>(L.err32[L.cur32]), L.g.elems);
             } else {
-                launch_restrict(ctx->stream, Lf.res, Lf.g, L.rhs, L.g);
+                if (fold64(level)) { vs64.resf = Lf.res; vs64.gf = Lf.g; }
+                else launch_restrict(ctx->stream, Lf.res, Lf.g, L.rhs, L.g);
                 if (!zero_start) TC_HIP(hipMemsetAsync(L.err[L.cur], 0, plane_bytes(L.g), ctx->stream));
             }
         }
@@ -1566,7 +1590,8 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                 }
             }
             bool fused = false;
-            TC_TRY(dc_iterate(ctx, d, level, dir, f32, zero_start, want_rr ? &rrt : nullptr, &fused));
+            TC_TRY(dc_iterate(ctx, d, level, dir, f32, zero_start, want_rr ? &rrt : nullptr, &fused, vs64));
+            vs64 = VisitStart{};
             if (fused) {
                 rr_level = level + 1;
                 ctx->stats.residuals_exec[level - 1]++;
@@ -1613,6 +1638,9 @@ int dc_solve(tc_ctx* ctx, int32_t* q_out, int max_cycles)
                 ctx->pend_from = level;
             } else if (f32) {
                 launch_prolong32(ctx->stream, Lf.err32[Lf.cur32], Lf.g, L.err32[L.cur32], L.g, zsg);
+            } else if (fold64(level - 1) && p < P.nsteps && multi[p + 1] == level - 1) {
+                vs64.Ec = L.err[L.cur];
+                vs64.gc = L.g;
             } else {
                 launch_prolong(ctx->stream, Lf.err[Lf.cur], Lf.g, L.err[L.cur], L.g, zsg);
             }

@@ -62,6 +62,30 @@ __device__ __forceinline__ float prolong_add32(const float* __restrict__ Ec, con
     return __fmul_rn(s, 0.25f);
 }
 
+// restrict (iterative_solver.f90:596-626) of a fine plane at the coarse point
+// (i,k)
+__device__ __forceinline__ double restrict_at(const double* __restrict__ in, const Grid& gi, int i, int k)
+{
+    const int ii = 2 * i, kk = 2 * k;
+    const double corners = (in[gi.at(ii - 1, kk - 1)] + in[gi.at(ii - 1, kk + 1)] + in[gi.at(ii + 1, kk + 1)] +
+                            in[gi.at(ii - 1, kk + 1)]) / 16.0;
+    const double sides =
+        (in[gi.at(ii - 1, kk)] + in[gi.at(ii, kk - 1)] + in[gi.at(ii + 1, kk)] + in[gi.at(ii, kk + 1)]) / 8.0;
+    return corners + sides + in[gi.at(ii, kk)] / 4.0;
+}
+// prolong (iterative_solver.f90:175-233) of a coarse correction at the fine
+// interior point (i,k): the value added there.  The four sources are loaded
+// whatever the parity (even indices take one node twice), and the sum the
+// reference takes for it is selected.
+__device__ __forceinline__ double prolong_at(const double* __restrict__ Ec, const Grid& gc, int i, int k)
+{
+    const int i0 = i >> 1, i1 = (i + 1) >> 1, k0 = k >> 1, k1 = (k + 1) >> 1;
+    const double e00 = Ec[gc.at(i0, k0)], e10 = Ec[gc.at(i1, k0)], e11 = Ec[gc.at(i1, k1)], e01 = Ec[gc.at(i0, k1)];
+    const bool ie = (i & 1) == 0, ke = (k & 1) == 0;
+    const double two = (e00 + (ie ? e01 : e10)) / 2.0, four = (e00 + e10 + e11 + e01) / 4.0;
+    return (ie && ke) ? e00 : ((ie || ke) ? two : four);
+}
+
 __device__ __forceinline__ double block_sum(double a) { return block_reduce<0>(a); }
 __device__ __forceinline__ double block_min(double a) { return block_reduce<1>(a); }
 __device__ __forceinline__ double block_max(double a) { return block_reduce<2>(a); }
@@ -207,13 +231,26 @@ struct VisitPlan {
 };
 bool visit_tables(const FD& F);
 VisitPlan visit_plan_ref(const Grid& g, int cus);
+// What an FP64 visit's first launch does before its sweeps, in place of
+// launches of their own (2 to 4.7 us each): resf: the right-hand side is the
+// restriction of the finer level's residual (also written to the level's plane,
+// for the visit's other launches); Ec: the coarser level's correction is
+// prolonged into the start.  The values are launch_restrict's and
+// launch_prolong's.  Solve, before and after: 128x128 15.7 and 14.9 ms, 608x352
+// 25.8 and 25.4, 2048x1024 111.4 and 111.1, dc64 512x256 17.3 and 16.8.
+struct VisitStart {
+    const double* resf = nullptr;
+    Grid gf;
+    const double* Ec = nullptr;
+    Grid gc;
+};
 // nk sweeps of the FP64 reference form from `in` (nullptr: a zero
 // correction) into `out`; fac: the sweeps' factors (use_ratio: the cosines
 // of the per-point factors); res (plan.whole only): the residual of the
 // result.  rhs, walls and bits as launch_sweep / launch_residual.
 void launch_visit_ref(hipStream_t st, const VisitPlan& p, bool pow2, bool use_ratio, const Level& L, const double* rhs,
                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
-                      double* res);
+                      double* res, const VisitStart& vs);
 
 // The next coarser level's right-hand side, formed at the end of a visit's
 // last launch (what launch_residual_restrict32 would form from the visit's
@@ -241,7 +278,8 @@ void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, cons
                        const float* in, float* out, const Spacing& h, const double* fac, int nk, double zsg,
                        const float* Pc, const Grid* gc, const RRTarget* rr);
 void launch_visit13_64(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const double* rhs,
-                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg);
+                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
+                       const VisitStart& vs);
 
 // --- tc_fields.hip -------------------------------------------------------------
 void launch_velocities(hipStream_t st, const double* SF, double* u, double* w, const Grid& g, const FD& F, double dr,

@@ -102,12 +102,7 @@ __global__ __launch_bounds__(256) void k_restrict(const double* __restrict__ in,
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int k = blockIdx.y * blockDim.y + threadIdx.y + 1;
     if (i > go.nx - 1 || k > go.nz - 1) return;
-    const int ii = 2 * i, kk = 2 * k;
-    double corners = (in[gi.at(ii - 1, kk - 1)] + in[gi.at(ii - 1, kk + 1)] + in[gi.at(ii + 1, kk + 1)] +
-                      in[gi.at(ii - 1, kk + 1)]) / 16.0;
-    double sides = (in[gi.at(ii - 1, kk)] + in[gi.at(ii, kk - 1)] + in[gi.at(ii + 1, kk)] + in[gi.at(ii, kk + 1)]) / 8.0;
-    double centre = in[gi.at(ii, kk)] / 4.0;
-    out[go.at(i, k)] = corners + sides + centre;
+    out[go.at(i, k)] = restrict_at(in, gi, i, k);
 }
 
 // prolong (iterative_solver.f90:175-233): one thread per fine interior
@@ -120,15 +115,7 @@ __global__ __launch_bounds__(256) void k_prolong(double* __restrict__ Ef, Grid g
     const int k = blockIdx.y * blockDim.y + threadIdx.y + 1;
     if (i > gf.nx - 1 || k > gf.nz - 1) return;
     const size_t c = gf.at(i, k);
-    double add;
-    const bool ie = (i % 2) == 0, ke = (k % 2) == 0;
-    if (ie && ke) add = Ec[gc.at(i / 2, k / 2)];
-    else if (ie) add = (Ec[gc.at(i / 2, (k - 1) / 2)] + Ec[gc.at(i / 2, (k + 1) / 2)]) / 2.0;
-    else if (ke) add = (Ec[gc.at((i - 1) / 2, k / 2)] + Ec[gc.at((i + 1) / 2, k / 2)]) / 2.0;
-    else
-        add = (Ec[gc.at((i - 1) / 2, (k - 1) / 2)] + Ec[gc.at((i + 1) / 2, (k - 1) / 2)] +
-               Ec[gc.at((i + 1) / 2, (k + 1) / 2)] + Ec[gc.at((i - 1) / 2, (k + 1) / 2)]) / 4.0;
-    double v = Ef[c] + add;
+    double v = Ef[c] + prolong_at(Ec, gc, i, k);
     Ef[c] = v;
     stream_ghosts(Ef, gf, i, k, v, zsg);
 }

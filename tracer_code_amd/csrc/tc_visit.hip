@@ -151,7 +151,9 @@ __device__ __forceinline__ double ref_residual(const Taps<double>& t, const RefC
 }
 
 struct RefArgs {
-    const double *vis, *vx, *vz, *vxx, *vzz, *vxz, *rhs, *dts, *ratio;
+    const double *vis, *vx, *vz, *vxx, *vzz, *vxz;
+    double* rhs;
+    const double *dts, *ratio;
 };
 
 // Bound: FP64 arithmetic and one barrier a sweep (a region of 32x32 cells: 4
@@ -163,7 +165,7 @@ struct RefArgs {
 template <bool POW2, bool RATIO, int LW, int R, int NW, bool RES>
 __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict__ Ein, double* __restrict__ Eout,
                                                        RefArgs A, Grid g, Spacing h, VisitTile vt, VisitFactors sf,
-                                                       int nk, double zsg, double* __restrict__ Rout)
+                                                       int nk, double zsg, double* __restrict__ Rout, VisitStart vs)
 {
     constexpr int GR = 64 / LW, ROWS = NW * GR * R;
     __shared__ double buf[2][ROWS * LW];
@@ -181,7 +183,16 @@ __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict_
         const size_t c = g.at(in ? i : 1, in ? k0 + r : 1);
         S[r] = Ein ? Ein[c] : 0.0;
         const double vis = A.vis[c], vx = A.vx[c], vz = A.vz[c], vxx = A.vxx[c], vzz = A.vzz[c], vxz = A.vxz[c];
-        const double rhs = A.rhs[c], dts = A.dts[c];
+        const double dts = A.dts[c];
+        double rhs;
+        if (vs.resf) {
+            rhs = restrict_at(vs.resf, vs.gf, in ? i : 1, in ? k0 + r : 1);
+            const int rr = row0 + r;
+            if (in && li >= vt.hx && li < vt.hx + vt.tx && rr >= vt.hz && rr < vt.hz + vt.ty) A.rhs[c] = rhs;
+        } else {
+            rhs = A.rhs[c];
+        }
+        if (vs.Ec) S[r] = S[r] + prolong_at(vs.Ec, vs.gc, in ? i : 1, in ? k0 + r : 1);
         if (!in) S[r] = 0.0;
         q[r].vis = in ? vis : 0.0;
         q[r].vd = in ? vxx - vzz : 0.0;
@@ -287,14 +298,14 @@ __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict_
 template <bool POW2, int LW, int R, int NW, bool RES>
 void visit_ref_launch(hipStream_t st, bool ratio, dim3 gr, const double* in, double* out, const RefArgs& A,
                       const Grid& g, const Spacing& h, const VisitTile& vt, const VisitFactors& sf, int nk, double zsg,
-                      double* res)
+                      double* res, const VisitStart& vs)
 {
     if (ratio)
         hipLaunchKernelGGL((k_visit_ref<POW2, true, LW, R, NW, RES>), gr, dim3(NW * 64), 0, st, in, out, A, g, h, vt, sf,
-                           nk, zsg, res);
+                           nk, zsg, res, vs);
     else
         hipLaunchKernelGGL((k_visit_ref<POW2, false, LW, R, NW, RES>), gr, dim3(NW * 64), 0, st, in, out, A, g, h, vt,
-                           sf, nk, zsg, res);
+                           sf, nk, zsg, res, vs);
 }
 
 // ---- the 13-tap operator of the defect-correction cycles ---------------------
@@ -311,7 +322,9 @@ struct H13 {
 };
 template <typename T>
 struct Args13 {
-    const T *vis, *vx, *vz, *a1, *vxx, *vzz, *vxz, *rhs, *dts, *lb;  // FP32: a1, lb; FP64: vxx, vzz, lb = the ratio
+    const T *vis, *vx, *vz, *a1, *vxx, *vzz, *vxz;
+    T* rhs;
+    const T *dts, *lb;  // FP32: a1, lb; FP64: vxx, vzz, lb = the ratio
 };
 // the next level's right-hand side, formed after the last sweep (FP32); RowB
 // and bout: for the coarsest level, the coarse solve's equilibrated
@@ -327,6 +340,10 @@ struct Prolong13 {
     const float* Ec;
     Grid gc;
 };
+// what the first launch of a visit does before its sweeps: FP32 the
+// prolongation, FP64 that or the restriction (VisitStart)
+template <typename T>
+using Start13 = std::conditional_t<sizeof(T) == 4, Prolong13, VisitStart>;
 
 template <typename T>
 __device__ __forceinline__ Cell13<T> weights13(T vis, T vx, T vz, T a1, T vxz, T dts, T rhs, const H13<T>& h)
@@ -396,7 +413,7 @@ __device__ __forceinline__ T step13(const Taps<T>& t, const Cell13<T>& w)
 template <typename T, bool RATIO, int LW, int R, int NW, bool END>
 __global__ __launch_bounds__(NW * 64) void k_visit13(const T* __restrict__ Ein, T* __restrict__ Eout, Args13<T> A,
                                                      Grid g, H13<T> h, VisitTile vt, VisitFac<T> sf, int nk, T zsg,
-                                                     Prolong13 pr, End13 en)
+                                                     Start13<T> pr, End13 en)
 {
     constexpr int GR = 64 / LW, ROWS = NW * GR * R;
     __shared__ T buf[2][ROWS * LW];
@@ -416,7 +433,20 @@ __global__ __launch_bounds__(NW * 64) void k_visit13(const T* __restrict__ Ein, 
         const bool in = col && k >= 1 && k <= g.nz - 1;
         const size_t c = g.at(in ? i : 1, in ? k : 1);
         S[r] = Ein ? Ein[c] : T(0);
-        const T vis = A.vis[c], vx = A.vx[c], vz = A.vz[c], vxz = A.vxz[c], dts = A.dts[c], rhs = A.rhs[c];
+        const T vis = A.vis[c], vx = A.vx[c], vz = A.vz[c], vxz = A.vxz[c], dts = A.dts[c];
+        T rhs;
+        if constexpr (sizeof(T) == 8) {
+            if (pr.resf) {
+                rhs = restrict_at(pr.resf, pr.gf, in ? i : 1, in ? k : 1);
+                const int rr = row0 + r;
+                if (in && li >= vt.hx && li < vt.hx + vt.tx && rr >= vt.hz && rr < vt.hz + vt.ty) A.rhs[c] = rhs;
+            } else {
+                rhs = A.rhs[c];
+            }
+            if (pr.Ec) S[r] = S[r] + prolong_at(pr.Ec, pr.gc, in ? i : 1, in ? k : 1);
+        } else {
+            rhs = A.rhs[c];
+        }
         T a1;
         if constexpr (sizeof(T) == 4) a1 = A.a1[c];
         else a1 = A.vxx[c] - A.vzz[c];
@@ -617,9 +647,10 @@ VisitPlan visit_plan_ref(const Grid& g, int cus)
 
 void launch_visit_ref(hipStream_t st, const VisitPlan& p, bool pow2, bool use_ratio, const Level& L, const double* rhs,
                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
-                      double* res)
+                      double* res, const VisitStart& vs)
 {
-    const RefArgs A{L.vis, L.visx, L.visz, L.visxx, L.viszz, L.visxz, rhs, L.dtstream, L.ratio};
+    // (the plane is written only where vs asks for the restriction)
+    const RefArgs A{L.vis, L.visx, L.visz, L.visxx, L.viszz, L.visxz, const_cast<double*>(rhs), L.dtstream, L.ratio};
     VisitFactors sf;
     for (int s = 0; s < nk; ++s) sf.v[s] = fac[s];
     const VisitRegion rg = VISIT_REGIONS[p.cfg];
@@ -628,15 +659,15 @@ void launch_visit_ref(hipStream_t st, const VisitPlan& p, bool pow2, bool use_ra
     auto go = [&](auto pw) {
         constexpr bool P = decltype(pw)::value;
         if (res) {
-            if (p.cfg == 0) visit_ref_launch<P, 16, 1, 4, true>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, res);
-            else visit_ref_launch<P, 32, 2, 8, true>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, res);
+            if (p.cfg == 0) visit_ref_launch<P, 16, 1, 4, true>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, res, vs);
+            else visit_ref_launch<P, 32, 2, 8, true>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, res, vs);
             return;
         }
         switch (p.cfg) {
-        case 0: visit_ref_launch<P, 16, 1, 4, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr); break;
-        case 1: visit_ref_launch<P, 32, 2, 8, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr); break;
-        case 2: visit_ref_launch<P, 32, 1, 16, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr); break;
-        default: visit_ref_launch<P, 64, 4, 8, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr); break;
+        case 0: visit_ref_launch<P, 16, 1, 4, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr, vs); break;
+        case 1: visit_ref_launch<P, 32, 2, 8, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr, vs); break;
+        case 2: visit_ref_launch<P, 32, 1, 16, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr, vs); break;
+        default: visit_ref_launch<P, 64, 4, 8, false>(st, use_ratio, gr, in, out, A, L.g, h, vt, sf, nk, zsg, nullptr, vs); break;
         }
     };
     if (pow2) go(std::integral_constant<bool, true>{});
@@ -765,7 +796,7 @@ H13<T> h13_from(const Spacing& h)
 
 template <typename T, int LW, int R, int NW>
 void visit13_go(hipStream_t st, dim3 gr, bool ratio, bool end, const T* in, T* out, const Args13<T>& A, const Grid& g,
-                const H13<T>& h, const VisitTile& vt, const VisitFac<T>& sf, int nk, T zsg, const Prolong13& pr,
+                const H13<T>& h, const VisitTile& vt, const VisitFac<T>& sf, int nk, T zsg, const Start13<T>& pr,
                 const End13& en)
 {
     const dim3 b(NW * 64);
@@ -782,7 +813,7 @@ void visit13_go(hipStream_t st, dim3 gr, bool ratio, bool end, const T* in, T* o
 
 template <typename T>
 void launch13(hipStream_t st, int cfg, bool whole, bool ratio, bool end, const Args13<T>& A, const Grid& g,
-              const Spacing& h, const T* in, T* out, const double* fac, int nk, double zsg, const Prolong13& pr,
+              const Spacing& h, const T* in, T* out, const double* fac, int nk, double zsg, const Start13<T>& pr,
               const End13& en)
 {
     VisitFac<T> sf;
@@ -810,7 +841,8 @@ void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, cons
                        const float* in, float* out, const Spacing& h, const double* fac, int nk, double zsg,
                        const float* Pc, const Grid* gc, const RRTarget* rr)
 {
-    const Args13<float> A{L.vis32, L.visx32, L.visz32, L.a132, nullptr, nullptr, L.visxz32, rhs, L.dts32, L.lb32};
+    const Args13<float> A{L.vis32, L.visx32, L.visz32, L.a132, nullptr, nullptr, L.visxz32,
+                         const_cast<float*>(rhs), L.dts32, L.lb32};
     Prolong13 pr{nullptr, L.g};
     if (Pc) { pr.Ec = Pc; pr.gc = *gc; }
     End13 en{};
@@ -819,10 +851,12 @@ void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, cons
 }
 
 void launch_visit13_64(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const double* rhs,
-                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg)
+                       const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
+                       const VisitStart& vs)
 {
-    const Args13<double> A{L.vis, L.visx, L.visz, nullptr, L.visxx, L.viszz, L.visxz, rhs, L.dtstream, L.ratio};
-    launch13<double>(st, cfg, whole, use_ratio, false, A, L.g, h, in, out, fac, nk, zsg, Prolong13{nullptr, L.g}, End13{});
+    const Args13<double> A{L.vis, L.visx, L.visz, nullptr, L.visxx, L.viszz, L.visxz, const_cast<double*>(rhs),
+                           L.dtstream, L.ratio};
+    launch13<double>(st, cfg, whole, use_ratio, false, A, L.g, h, in, out, fac, nk, zsg, vs, End13{});
 }
 
 }  // namespace tc
