@@ -2567,7 +2567,7 @@ int init_ctx(tc_ctx* ctx, const tc_params* p, int64_t ntr)
         TC_TRY(dalloc(ctx, &ctx->Ainv, (size_t)ctx->ngc * ctx->ngc));
         TC_TRY(falloc(ctx, &ctx->Ainv32, (size_t)ctx->ngc * ctx->ngc));
         TC_TRY(dalloc(ctx, &ctx->Bc, ctx->ngc));
-        TC_TRY(dalloc(ctx, &ctx->Ur, (size_t)ctx->ngc * (size_t)(ctx->kl + ctx->ku + 1)));
+        TC_TRY(dalloc(ctx, &ctx->Ur, band_inverse_scratch(ctx->ngc, ctx->kl, ctx->ku)));
         TC_TRY(dalloc_i(ctx, &ctx->ipiv, ctx->ngc));
         TC_TRY(dalloc_i(ctx, &ctx->d_info, 1));
     }

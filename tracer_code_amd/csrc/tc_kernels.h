@@ -161,8 +161,10 @@ struct VisLoopArgs {
 void launch_coarse_assemble(hipStream_t st, double* Mc, double* RowB, const Level& L, const FD& F, const Spacing& h,
                             int ivis, int Vbc, int kl, int ku, int ngc);
 void launch_dgbtf2(hipStream_t st, double* ab, int ldab, int n, int kl, int ku, int32_t* ipiv, int32_t* info);
+// scratch: band_inverse_scratch doubles
+size_t band_inverse_scratch(int n, int kl, int ku);
 void launch_band_inverse(hipStream_t st, const double* ab, int ldab, int n, int kl, int ku, const int32_t* ipiv,
-                         double* Ainv, double* Ur);
+                         double* Ainv, double* scratch);
 void launch_coarse_lusolve(hipStream_t st, const double* ab, int ldab, int n, int kl, int ku, const int32_t* ipiv,
                            const double* RowB, const Level& L, double* E, double zsg);
 void launch_coarse_apply(hipStream_t st, const double* Ainv, const double* RowB, const Level& L, double* E, int ngc,
