@@ -1960,11 +1960,8 @@ int tracers_to_corners(tc_ctx* ctx, tc_dev& d, int which, int smooth, int32_t* n
     double *r, *s;
     tracer_set(ctx, which, &r, &s);
     CntArr cnt{};
-    for (int t = 0; t <= P.ntype; ++t) {
-        cnt.v[t] = ctx->count[t];
-        launch_zero_i32(ctx->stream, ctx->count[t], ctx->g.elems);
-    }
-    launch_zero_i32(ctx->stream, ctx->d_flag, 1);
+    for (int t = 0; t <= P.ntype; ++t) cnt.v[t] = ctx->count[t];
+    launch_zero_counts(ctx->stream, cnt, P.ntype + 1, ctx->g.elems, ctx->d_flag);
     launch_bin(ctx->stream, r, s, ctx->ttype, ctx->ntr, cnt, ctx->g, ctx->lv[1].dr, ctx->lv[1].ds, P.aspect, ctx->d_flag);
     PtrArr cn{};
     for (int t = 0; t < P.ntype; ++t) cn.v[t] = ctx->Cnew[t];
@@ -1976,7 +1973,7 @@ int tracers_to_corners(tc_ctx* ctx, tc_dev& d, int which, int smooth, int32_t* n
         return TC_ERR_TRACER_DOMAIN;
     }
     if (P.comp == 1) {
-        for (int t = 0; t < P.ntype; ++t) launch_bcs_comp(ctx->stream, ctx->Cnew[t], ctx->g);
+        launch_bcs_comp(ctx->stream, cn, P.ntype, ctx->g);
         if (smooth) TC_TRY(smoother_time(ctx, d, n_comp));
     }
     return load_conductivity(ctx, d);

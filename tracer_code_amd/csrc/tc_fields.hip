@@ -580,18 +580,44 @@ __global__ void k_bcs_T(double* __restrict__ T, Grid g, int Tbot, const int32_t*
     }
 }
 
-// enforceBCs_comp (composition.f90:792-803) in the reference's interleaved
-// order, one workgroup.
-__global__ void k_bcs_comp(double* __restrict__ C, Grid g, const int32_t* __restrict__ stop)
+// enforceBCs_comp (composition.f90:792-803) of every type in one pass: a
+// thread per ghost value, each the interior value it mirrors.  Written in the
+// reference's order (columns -i and nx+i, then rows -i and nz+i, for i = 1, 2),
+// the row beyond the wall reads columns -2 and nx+2 before they are renewed:
+// the values that these four corners keep are taken by the thread that
+// renews them.  At 1024x512 one workgroup per type, in that order, took 7.7 us
+// each; two types take 6.0 us here, one 3.9.
+__global__ __launch_bounds__(256) void k_bcs_comp(PtrArr Cs, Grid g)
 {
-    if (stop && stop[0]) return;
-    const int nx = g.nx, nz = g.nz, tid = threadIdx.x, nt = blockDim.x;
-    for (int i = 1; i <= SPAN; ++i) {
-        for (int k = tid; k <= nz; k += nt) { C[g.at(-i, k)] = C[g.at(i, k)]; C[g.at(nx + i, k)] = C[g.at(nx - i, k)]; }
-        __syncthreads();
-        for (int ii = -SPAN + tid; ii <= nx + SPAN; ii += nt) { C[g.at(ii, -i)] = C[g.at(ii, i)]; C[g.at(ii, nz + i)] = C[g.at(ii, nz - i)]; }
-        __syncthreads();
+    double* C = Cs.v[blockIdx.y];
+    const int nx = g.nx, nz = g.nz, cols = 2 * SPAN * (nz + 1), w = nx + 2 * SPAN + 1;
+    int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < cols) {
+        const int k = e % (nz + 1), q = e / (nz + 1), d = q / 2 + 1;  // d cells beyond the wall
+        const int i = (q & 1) ? nx + d : -d, m = (q & 1) ? nx - d : d;
+        if (d == 2) {
+            const double old = C[g.at(i, k)];
+            if (k == 1) C[g.at(i, -1)] = old;
+            if (k == nz - 1) C[g.at(i, nz + 1)] = old;
+        }
+        C[g.at(i, k)] = C[g.at(m, k)];
+        return;
     }
+    e -= cols;
+    if (e >= 2 * SPAN * w) return;
+    const int i = e % w - SPAN, q = e / w, d = q / 2 + 1;
+    if (d == 1 && (i == -2 || i == nx + 2)) return;
+    const int mi = i < 0 ? -i : (i > nx ? 2 * nx - i : i);
+    C[g.at(i, (q & 1) ? nz + d : -d)] = C[g.at(mi, (q & 1) ? nz - d : d)];
+}
+
+// the counts of all types and the out-of-domain flag
+__global__ void k_zero_counts(CntArr cnt, size_t n, int32_t* __restrict__ flag)
+{
+    int32_t* p = cnt.v[blockIdx.y];
+    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0 && blockIdx.y == 0) *flag = 0;
+    for (; t < n; t += (size_t)gridDim.x * blockDim.x) p[t] = 0;
 }
 
 __global__ void k_zero_i32(int32_t* __restrict__ p, size_t n)
@@ -626,42 +652,81 @@ __global__ __launch_bounds__(256) void k_unpack_types(PackPlanes P, Grid g, int 
 
 // tracers_to_corners counting loop (composition.f90:704-715): nearest node
 // by Fortran NINT (half away from zero) of r/dr and s/ds, domain check.
+//
+// Bound: 20 bytes a tracer, and the atomics, which leave for a memory line
+// each where neighbours in storage lie in different rows.  Tracers are stored
+// cell by cell and move less than a cell between sorts, so the consecutive
+// tracers of a workgroup fall on few nodes, but alternate between a cell's
+// corners.  Runs of one counter are summed in the wavefront, the runs in a table
+// of counters in LDS, and each counter of the table goes to memory once; a
+// run that finds its 8 slots taken (tracers in no order) goes there directly.
+// Measured, before (an atomic a run, one tracer a thread) and now: 21 M tracers
+// by node 128 and 93 us (4.5 TB/s), a step's stages 42 M 496 and 187, 10.5 M 207
+// and 60, 0.26 M 10.5 and 5.1; by cell, of random type, 42 M 1122 and 319.  One
+// tracer a thread with the table takes 133, 262, 75, 4.6 and 309; eight 92, 192,
+// 69, and 353 for the last.
+constexpr int BIN_U = 2;  // tracers a thread
 template <bool POW2>
 __global__ __launch_bounds__(256) void k_bin(const double* __restrict__ r, const double* __restrict__ s,
                                              const int32_t* __restrict__ ty, int64_t n, CntArr cnt, Grid g, double dr,
                                              double ds, double idr, double ids, double aspect, int32_t* __restrict__ flag)
 {
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    // key of the (type, node) counter this tracer adds to; none = ~0
-    uint32_t key = ~0u;
-    int t = 0;
-    size_t node = 0;
-    if (id < n) {
-        const double rv = r[id], sv = s[id];
-        // the reference's test (r<=0 or r>=aspect or s<=0 or s>=1), written so
-        // that a NaN position is also rejected before it can form an index
-        if (!(rv > 0.0 && rv < aspect && sv > 0.0 && sv < 1.0)) {
-            atomicOr(flag, 1);
-        } else {
-            const int i = (int)round(sdiv<POW2>(rv, dr, idr));
-            const int k = (int)round(sdiv<POW2>(sv, ds, ids));
-            node = g.at(i, k);
-            t = ty[id];
-            key = (uint32_t)node * (uint32_t)(TC_MAX_TYPES + 1) + (uint32_t)t;
+    constexpr int SLOTS = 256 * BIN_U, BITS = __builtin_ctz(SLOTS), PROBES = 8;
+    __shared__ uint32_t keys[SLOTS];
+    __shared__ int sums[SLOTS];
+    const int64_t base = (int64_t)blockIdx.x * SLOTS + threadIdx.x;
+    double rv[BIN_U], sv[BIN_U];
+    int tv[BIN_U];
+#pragma unroll
+    for (int u = 0; u < BIN_U; ++u) {
+        const int64_t id = base + 256 * u;
+        rv[u] = id < n ? r[id] : 0.0;
+        sv[u] = id < n ? s[id] : 0.0;
+        tv[u] = id < n ? ty[id] : 0;
+        keys[threadIdx.x + 256 * u] = ~0u;
+        sums[threadIdx.x + 256 * u] = 0;
+    }
+    __syncthreads();
+    auto add = [&](uint32_t key, int len) {
+        atomicAdd(&cnt.v[key % (uint32_t)(TC_MAX_TYPES + 1)][key / (uint32_t)(TC_MAX_TYPES + 1)], len);
+    };
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int u = 0; u < BIN_U; ++u) {
+        // key of the (type, node) counter this tracer adds to; none = ~0
+        uint32_t key = ~0u;
+        if (base + 256 * u < n) {
+            // the reference's test (r<=0 or r>=aspect or s<=0 or s>=1), written so
+            // that a NaN position is also rejected before it can form an index
+            if (!(rv[u] > 0.0 && rv[u] < aspect && sv[u] > 0.0 && sv[u] < 1.0)) {
+                atomicOr(flag, 1);
+            } else {
+                const int i = (int)round(sdiv<POW2>(rv[u], dr, idr));
+                const int k = (int)round(sdiv<POW2>(sv[u], ds, ids));
+                key = (uint32_t)g.at(i, k) * (uint32_t)(TC_MAX_TYPES + 1) + (uint32_t)tv[u];
+            }
+        }
+        const uint32_t prev = __shfl_up(key, 1, 64);
+        const bool boundary = lane == 0 || prev != key;
+        const unsigned long long starts = __ballot(boundary);
+        if (boundary && key != ~0u) {
+            const unsigned long long later = (lane == 63) ? 0ull : (starts >> (lane + 1));
+            const int len = later ? __builtin_ctzll(later) + 1 : 64 - lane;
+            uint32_t h = (key * 2654435761u) >> (32 - BITS);
+            int p = 0;
+            for (; p < PROBES; ++p, h = (h + 1) & (SLOTS - 1)) {
+                const uint32_t old = atomicCAS(&keys[h], ~0u, key);
+                if (old == ~0u || old == key) break;
+            }
+            if (p < PROBES) atomicAdd(&sums[h], len);
+            else add(key, len);
         }
     }
-    // wavefront segmented reduction: consecutive lanes with the same key form
-    // a run (tracers are stored node by node, and move less than a cell per
-    // step, so runs of ~tpc are the rule); the run's first lane adds the
-    // run's length, one atomic per run instead of one per tracer
-    const int lane = threadIdx.x & 63;
-    const uint32_t prev = __shfl_up(key, 1, 64);
-    const bool boundary = lane == 0 || prev != key;
-    const unsigned long long starts = __ballot(boundary);
-    if (boundary && key != ~0u) {
-        const unsigned long long later = (lane == 63) ? 0ull : (starts >> (lane + 1));
-        const int len = later ? __builtin_ctzll(later) + 1 : 64 - lane;
-        atomicAdd(&cnt.v[t][node], len);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < BIN_U; ++u) {
+        const int e = threadIdx.x + 256 * u;
+        if (keys[e] != ~0u) add(keys[e], sums[e]);
     }
 }
 
@@ -1114,9 +1179,11 @@ void launch_bcs_T(hipStream_t st, double* T, const Grid& g, int Tbot, const int3
     hipLaunchKernelGGL(k_bcs_T, dim3(1), dim3(1024), 0, st, T, g, Tbot, stop);
 }
 
-void launch_bcs_comp(hipStream_t st, double* C, const Grid& g, const int32_t* stop)
+void launch_bcs_comp(hipStream_t st, const PtrArr& C, int ntype, const Grid& g)
 {
-    hipLaunchKernelGGL(k_bcs_comp, dim3(1), dim3(1024), 0, st, C, g, stop);
+    if (ntype <= 0) return;
+    const int n = 2 * SPAN * (g.nz + 1) + 2 * SPAN * (g.nx + 2 * SPAN + 1);
+    hipLaunchKernelGGL(k_bcs_comp, dim3((n + 255) / 256, ntype), dim3(256), 0, st, C, g);
 }
 
 void launch_smoothness_max(hipStream_t st, const double* T0, const Grid& g, unsigned long long* slots,
@@ -1223,18 +1290,25 @@ void launch_zero_i32(hipStream_t st, int32_t* p, size_t n)
     hipLaunchKernelGGL(k_zero_i32, dim3(nb), dim3(256), 0, st, p, n);
 }
 
+void launch_zero_counts(hipStream_t st, const CntArr& cnt, int n, size_t elems, int32_t* flag)
+{
+    const size_t nb = std::min<size_t>((elems + 255) / 256, 4096);
+    hipLaunchKernelGGL(k_zero_counts, dim3((unsigned)nb, n), dim3(256), 0, st, cnt, elems, flag);
+}
+
 void launch_bin(hipStream_t st, const double* r, const double* s, const int32_t* ty, int64_t n, const CntArr& cnt,
                 const Grid& g, double dr, double ds, double aspect, int32_t* flag)
 {
     if (n <= 0) return;
     int e;
     const bool pow2 = std::frexp(dr, &e) == 0.5 && std::frexp(ds, &e) == 0.5;
+    const dim3 blocks((unsigned)((n + 256 * BIN_U - 1) / (256 * BIN_U)));
     if (pow2)
-        hipLaunchKernelGGL((k_bin<true>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, r, s, ty, n, cnt, g, dr, ds,
-                           1.0 / dr, 1.0 / ds, aspect, flag);
+        hipLaunchKernelGGL((k_bin<true>), blocks, dim3(256), 0, st, r, s, ty, n, cnt, g, dr, ds, 1.0 / dr, 1.0 / ds,
+                           aspect, flag);
     else
-        hipLaunchKernelGGL((k_bin<false>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, r, s, ty, n, cnt, g, dr,
-                           ds, 1.0 / dr, 1.0 / ds, aspect, flag);
+        hipLaunchKernelGGL((k_bin<false>), blocks, dim3(256), 0, st, r, s, ty, n, cnt, g, dr, ds, 1.0 / dr, 1.0 / ds,
+                           aspect, flag);
 }
 
 void launch_ratio(hipStream_t st, const CntArr& cnt, int32_t* nempty, const PtrArr& Cnew, const Grid& g, int ntype,

@@ -293,7 +293,9 @@ struct PackPlanes { void* v[TC_MAX_TYPES + 1]; };
 // the boundary's type-fastest layout
 void launch_pack_types(hipStream_t st, const PackPlanes& P, const Grid& g, int n, int bytes, void* buf, bool pack);
 void launch_bcs_T(hipStream_t st, double* T, const Grid& g, int Tbot, const int32_t* stop = nullptr);
-void launch_bcs_comp(hipStream_t st, double* C, const Grid& g, const int32_t* stop = nullptr);
+void launch_bcs_comp(hipStream_t st, const PtrArr& C, int ntype, const Grid& g);
+// n count planes and the flag
+void launch_zero_counts(hipStream_t st, const CntArr& cnt, int n, size_t elems, int32_t* flag);
 void launch_zero_i32(hipStream_t st, int32_t* p, size_t n);
 int diag_blocks(const Grid& g);
 int stats_np();  // partial sums per block of launch_stats_rest

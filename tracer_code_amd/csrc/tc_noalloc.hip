@@ -67,18 +67,14 @@ extern "C" int tc_bin_tracers_noalloc(int32_t nx, int32_t nz, double aspect, int
     hipStream_t st = static_cast<hipStream_t>(stream);
     int32_t* counts = count_type ? count_type : base;
     CntArr cnt{};
-    for (int t = 0; t <= ntype; ++t) {
-        cnt.v[t] = counts + (size_t)t * g.elems;
-        launch_zero_i32(st, cnt.v[t], g.elems);
-    }
-    launch_zero_i32(st, flag, 1);
+    for (int t = 0; t <= ntype; ++t) cnt.v[t] = counts + (size_t)t * g.elems;
+    launch_zero_counts(st, cnt, ntype + 1, g.elems, flag);
     const double dr = aspect / nx, ds = 1.0 / nz;
     if (ntr > 0) launch_bin(st, r, s, ttype, ntr, cnt, g, dr, ds, aspect, flag);
     PtrArr cn{};
     for (int t = 0; t < ntype; ++t) cn.v[t] = Cnew + (size_t)t * g.elems;
     launch_ratio(st, cnt, nempty, cn, g, ntype, comp);
-    if (comp == 1)
-        for (int t = 0; t < ntype; ++t) launch_bcs_comp(st, cn.v[t], g);
+    if (comp == 1) launch_bcs_comp(st, cn, ntype, g);
     if (hipGetLastError() != hipSuccess) return TC_ERR_HIP;
     int32_t h = 0;
     if (hipMemcpyAsync(&h, flag, sizeof(int32_t), hipMemcpyDeviceToHost, st) != hipSuccess) return TC_ERR_HIP;
