@@ -390,20 +390,6 @@ __global__ __launch_bounds__(256) void k_sweep32(const float* __restrict__ S0, f
     stream_ghosts(E, g, i, k, v, zsg);
 }
 
-__global__ __launch_bounds__(256) void k_residual32(const float* __restrict__ S, float* __restrict__ R,
-                                                    const float* __restrict__ vis, const float* __restrict__ vx,
-                                                    const float* __restrict__ vz, const float* __restrict__ a1,
-                                                    const float* __restrict__ vxz, const float* __restrict__ rhs,
-                                                    Grid g, FD32 F, H32 h)
-{
-    const int2 tile = xcd_tile();
-    const int i = tile.x * blockDim.x + threadIdx.x + 1;
-    const int k = tile.y * blockDim.y + threadIdx.y + 1;
-    if (i > g.nx - 1 || k > g.nz - 1) return;
-    const size_t c = g.at(i, k);
-    R[c] = (float)stream_space32<double>(F, h, S, c, g.ld, vis[c], vx[c], vz[c], a1[c], vxz[c], rhs[c]);
-}
-
 __global__ __launch_bounds__(256) void k_restrict32(const float* __restrict__ in, Grid gi, float* __restrict__ out,
                                                     Grid go)
 {
@@ -422,7 +408,7 @@ __global__ __launch_bounds__(256) void k_restrict32(const float* __restrict__ in
 // one thread per coarse interior point evaluates the 8 fine residuals the
 // restriction weights (the reference's corner set, iterative_solver.f90:
 // 604-609, reads (ii-1,kk+1) twice and not (ii+1,kk-1)), each rounded to FP32
-// exactly as k_residual32 stores it, and combines them in k_restrict32's
+// as an FP32 residual plane would store it, and combines them in k_restrict32's
 // order -- the same values as the two kernels, without the residual plane.
 // With bout (the coarsest level), also the equilibrated right-hand side of
 // the coarse solve at the interior unknowns, as k_coarse_rhs32 forms it.
@@ -878,14 +864,6 @@ void launch_sweep32(hipStream_t st, bool use_ratio, const Level& L, const float*
     else
         hipLaunchKernelGGL((k_sweep32<false>), gr, b, 0, st, S0, E, L.vis32, L.visx32, L.visz32, L.a132, L.visxz32, rhs,
                            L.dts32, L.lb32, L.g, f, hh, (float)temp, (float)cconst, (float)zsg);
-}
-
-void launch_residual32(hipStream_t st, const Level& L, const float* S, float* R, const float* rhs, const FD& F,
-                       const Spacing& h)
-{
-    dim3 b(64, 4);
-    hipLaunchKernelGGL(k_residual32, grid2(L.g.nx - 1, L.g.nz - 1, b), b, 0, st, S, R, L.vis32, L.visx32, L.visz32,
-                       L.a132, L.visxz32, rhs, L.g, fd32_from(F), h32_from(h));
 }
 
 void launch_restrict32(hipStream_t st, const float* in, const Grid& gi, float* out, const Grid& go)

@@ -77,7 +77,7 @@ struct Level {
     float *rhs32 = nullptr, *vis32 = nullptr, *visx32 = nullptr, *visz32 = nullptr, *a132 = nullptr, *visxz32 = nullptr;
     float *dts32 = nullptr, *lb32 = nullptr, *res32 = nullptr;
     float* w13 = nullptr;  // 13 planes: dt-scaled stencil weights of the FP32 operator, per solve
-    int tb_tile = 0;       // tile of the FP32 temporally blocked sweeps: 16, 32, or 0 (by level size)
+    int tb_tile = 0;       // region of the blocked sweeps (tc_set_tb_tile): 16, 32, 48, or 0 (by level size)
     int cur32 = 0;
 };
 

@@ -206,8 +206,6 @@ void launch_prolong_dd(hipStream_t st, double* hi, double* lo, const Grid& gf, c
                        const Grid& gc, double zsg);
 void launch_sweep32(hipStream_t st, bool use_ratio, const Level& L, const float* S0, float* E, const float* rhs,
                     const FD& F, const Spacing& h, double temp, double cconst, double zsg);
-void launch_residual32(hipStream_t st, const Level& L, const float* S, float* R, const float* rhs, const FD& F,
-                       const Spacing& h);
 void launch_restrict32(hipStream_t st, const float* in, const Grid& gi, float* out, const Grid& go);
 // (std_tables: visit_tables(F); the arithmetic of the fused form)
 // with RowB and bout (descent into the coarsest level): also the coarse
