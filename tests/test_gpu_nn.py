@@ -77,6 +77,33 @@ def test_adam_step():
     assert np.max(np.abs(w1 - want)) <= 1e-6
 
 
+def test_sums_do_not_depend_on_the_launch():
+    """Every accumulation is one chain in a fixed order, whatever form of a
+    launch runs it: the upper rows of an image give the same bits, forward and
+    gradients, as the same rows of a taller one, whose convolutions and weight
+    gradients run in other forms.  The mask keeps the loss to rows whose
+    receptive field (44 rows and the pooling's rounding) ends inside the smaller
+    image; pixels keep their index and their split, and what the other rows
+    add is zero."""
+    W, rows = 256, 32
+    rng = np.random.default_rng(9)
+    x = rng.uniform(-1, 1, (512, W, 6))
+    t = rng.standard_normal((512, W))
+    m = np.zeros((512, W))
+    m[:rows] = 1
+    w = unet.init_params(8).astype(np.float32)
+    got = []
+    for H in (112, 512):
+        print(f"[nn launch forms {H}x{W}]", flush=True)
+        with learn.Network(H, W) as net:
+            net.set_weights(w)
+            net.set_sample(x[:H], t[:H], m[:H])
+            out = net.forward()
+            got.append((out[:rows], net.backward(), net.get_grads()))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("level", [1, 3])
 def test_guess_in_solver_keeps_tolerance(level):
     params, cfg = config.preset_params("cfg0", nx=64, nz=64, tpc=4)

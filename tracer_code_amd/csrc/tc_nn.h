@@ -49,7 +49,6 @@ struct UNet {
 
     void layer_defs();
     size_t param_count() const;
-    int split_pixels(const Layer& l) const;
     int alloc(int H, int W, bool train);
     void release();
     void pack(hipStream_t st);

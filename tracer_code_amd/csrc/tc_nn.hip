@@ -30,6 +30,14 @@ namespace tc {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// v, or zeros
+__device__ __forceinline__ bf16x8 keep8(bf16x8 v, bool keep)
+{
+    const u32x4 u = __builtin_bit_cast(u32x4, v);
+    return __builtin_bit_cast(bf16x8, keep ? u : u32x4{0u, 0u, 0u, 0u});
+}
 
 __device__ __forceinline__ float gelu_f(float z)
 {
@@ -66,20 +74,58 @@ struct ConvArgs {
     int mode;
 };
 
-// Bound: the latency of the fragment loads (an iteration of 32 depth values
-// is one MFMA after two 16-byte loads).  KS waves share a tile's depth and add
-// up their accumulators in LDS, so that on the small levels, whose tiles
-// leave most CUs idle, the chain of loads is KS times shorter; addresses are
-// clamped and values selected, so that the loads of several iterations are
-// in flight.
-template <int KS>
-__global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a)
+// One accumulation chain of n MFMAs whose operands NW waves load: a wave
+// takes up to PER consecutive iterations of a round, their loads in flight
+// together, and the accumulator goes from wave to wave through LDS, ending in
+// the last one.  It takes the iterations in their order whatever NW and PER
+// are, so a sum has the same bits in every form of a launch, on every grid.
+// load(it, a, b, ka, kb): the operands of iteration it, from addresses in
+// range, with ka (kb) false where zeros take their place; frag(a, b): the
+// wave's loaded operands into fragments.
+template <int NW, int PER, typename Load, typename Frag>
+__device__ __forceinline__ void relay_chain(f32x4* __restrict__ hand, int n, int wv, int lane, f32x4& acc, Load load,
+                                            Frag frag)
 {
-    constexpr int TILES = 4 / KS;  // tiles of a workgroup
-    __shared__ f32x4 part[KS > 1 ? 4 : 1][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (int i0 = 0; i0 < n; i0 += NW * PER) {
+        const int m = n - i0 < NW * PER ? n - i0 : NW * PER, q = (m + NW - 1) / NW;
+        const int b = wv * q, cnt = (m - b < q ? m - b : q);  // (cnt <= 0: none left for this wave)
+        bf16x8 la[PER], lb[PER];
+        bool ka[PER], kb[PER];
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (u < cnt) load(i0 + b + u, la[u], lb[u], ka[u], kb[u]);
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            if (u < cnt) {
+                la[u] = keep8(la[u], ka[u]);
+                lb[u] = keep8(lb[u], kb[u]);
+            }
+        frag(la, lb);
+        for (int w = 0; w < NW; ++w) {
+            if (wv == w) {
+                if (NW > 1 && i0 + w > 0) acc = hand[lane];
+#pragma unroll
+                for (int u = 0; u < PER; ++u)
+                    if (u < cnt) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la[u], lb[u], acc, 0, 0, 0);
+                if (NW > 1) hand[lane] = acc;
+            }
+            if (NW > 1) __syncthreads();
+        }
+    }
+}
+
+// Bound: the latency of the fragment loads (an iteration of 32 depth values
+// is one MFMA after two 16-byte loads).  KS waves share a tile's depth on the
+// small levels, whose tiles leave most CUs idle; KS = 1: four tiles a
+// workgroup.
+template <int KS, int PER>
+__global__ __launch_bounds__(KS > 4 ? 64 * KS : 256) void k_conv3x3(ConvArgs a)
+{
+    constexpr int TILES = KS > 1 ? 1 : 4;  // tiles of a workgroup
+    __shared__ f32x4 hand[64];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int npix = a.H * a.W;
-    const int p0 = (blockIdx.x * TILES + wv / KS) * 16, ks = wv % KS;
+    const int p0 = (blockIdx.x * TILES + (KS > 1 ? 0 : wv)) * 16;
     const int cb = blockIdx.y;
     const int row = lane & 15, grp = lane >> 4;
     const int p = p0 + row;
@@ -87,24 +133,20 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a)
     const int co = cb * 16 + row;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     const __bf16* __restrict__ wk = a.wk + (size_t)co * a.kp;
-#pragma unroll 4
-    for (int k0 = ks * 32 + grp * 8; k0 < a.kp; k0 += 32 * KS) {
-        const int tap = k0 / a.cinp, ci0 = k0 - tap * a.cinp;
-        const int yy = py + tap / 3 - 1, xx = px + tap % 3 - 1;
-        const bool ok = tap < 9 && p < npix && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W;
-        bf16x8 fa = *reinterpret_cast<const bf16x8*>(a.in + (ok ? (size_t)(yy * a.W + xx) * a.cs_in + a.off_in + ci0
-                                                                  : (size_t)a.off_in));
-        if (!ok)
-            for (int j = 0; j < 8; ++j) fa[j] = (__bf16)0.0f;
-        const bf16x8 fb = *reinterpret_cast<const bf16x8*>(wk + k0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, acc, 0, 0, 0);
-    }
-    if constexpr (KS > 1) {
-        part[wv][lane] = acc;
-        __syncthreads();
-        if (ks != 0) return;
-        for (int q = 1; q < KS; ++q) acc += part[wv + q][lane];
-    }
+    const __bf16* __restrict__ in = a.in + a.off_in;
+    const float rc = 1.0f / (float)a.cinp;
+    auto load = [&](int it, bf16x8& fa, bf16x8& fb, bool& ka, bool& kb) {
+        const int k0 = it * 32 + grp * 8;
+        // (k0 + 1/2) / cinp is at least 1/(2 cinp) from a whole number: no rounding reaches it
+        const int tap = (int)(((float)k0 + 0.5f) * rc), ci0 = k0 - tap * a.cinp, ty = (tap * 11) >> 5;
+        const int yy = py + ty - 1, xx = px + tap - 3 * ty - 1;
+        ka = tap < 9 && p < npix && (unsigned)yy < (unsigned)a.H && (unsigned)xx < (unsigned)a.W;
+        kb = true;
+        fa = *reinterpret_cast<const bf16x8*>(in + (ka ? (size_t)(yy * a.W + xx) * a.cs_in + ci0 : 0));
+        fb = *reinterpret_cast<const bf16x8*>(wk + k0);
+    };
+    relay_chain<KS, PER>(hand, a.kp / 32, KS > 1 ? wv : 0, lane, acc, load, [](bf16x8*, bf16x8*) {});
+    if (KS > 1 && wv != KS - 1) return;
     // lane holds D[pixel p0 + grp*4 + i][channel cb*16 + row]
     const int c = cb * 16 + row;
     for (int i = 0; i < 4; ++i) {
@@ -125,17 +167,22 @@ __global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a)
     }
 }
 
-// KS = 4 waves a tile while the launch would otherwise hold fewer than 2
-// waves per SIMD of the chip (2048) and a wave has more than 2 iterations:
-// at 32x96 pixels the 27 forward and input-gradient launches of a training
-// step take 138 us instead of 250
+// Four waves a tile, eight where a quarter of the depth is more than 5
+// iterations, while the launch would otherwise hold fewer than 2 waves per
+// SIMD of the chip (2048): at 32x96 pixels the 27 forward and input-gradient
+// launches of a training step take 142 us instead of 250.  (With partial
+// accumulators, added at the end, they took 138; but the sums then depended
+// on the launch's form.)
 static void launch_conv3x3(hipStream_t st, const ConvArgs& a)
 {
     const int tiles = (a.H * a.W + 15) / 16, cbs = a.cout / 16;
-    if ((long)tiles * cbs < 2048 && a.kp > 64)
-        hipLaunchKernelGGL(k_conv3x3<4>, dim3(tiles, cbs), dim3(256), 0, st, a);
+    const long wgs = (long)tiles * cbs;
+    if (wgs >= 2048)
+        hipLaunchKernelGGL((k_conv3x3<1, 4>), dim3((tiles + 3) / 4, cbs), dim3(256), 0, st, a);
+    else if (a.kp > 640)
+        hipLaunchKernelGGL((k_conv3x3<8, 7>), dim3(tiles, cbs), dim3(512), 0, st, a);
     else
-        hipLaunchKernelGGL(k_conv3x3<1>, dim3((tiles + 3) / 4, cbs), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((k_conv3x3<4, 5>), dim3(tiles, cbs), dim3(256), 0, st, a);
 }
 
 // Weight gradient: partial[split][co][k] = sum over the split's pixels of
@@ -147,51 +194,83 @@ struct WGradArgs {
     int cs_in, off_in, cinp;
     int kp, cout;
     float* partial;    // [nsplit][cout][kp]
-    int H, W, pix_per_split;
+    int H, W;
 };
+constexpr int WGRAD_PIX = 2048;  // pixels of a split
 
-// Bound: the latency of its 2-byte loads; 4 waves share a split's chunks of 32
-// pixels and add up in LDS, and the splits fill the chip (one split of up to
-// 2048 pixels a wave took 148 to 170 us a layer at 32x96 pixels, in 10 to 28
-// waves).
-__global__ __launch_bounds__(256) void k_conv3x3_wgrad(WGradArgs a)
+// Bound: the latency of the loads and of the chain, up to 64 iterations of 32
+// pixels.  One wave a split, with 2-byte loads of each fragment's values,
+// took 148 to 170 us a layer at 32x96 pixels, in 10 to 28 waves; 16 waves a
+// split and 16-byte loads take 6.4 to 7.3.
+// The reduction runs over pixels, along which neither operand is contiguous:
+// a lane loads 8 channels (16 bytes) of a pixel, LDS holds [pixel][16
+// channels], and the transposing reads give the fragments.
+template <int NW, int PER>
+__global__ __launch_bounds__(64 * NW) void k_conv3x3_wgrad(WGradArgs a)
 {
-    __shared__ f32x4 part[4][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    __shared__ f32x4 hand[64];
+    __shared__ bf16x8 turn[NW][PER][2][64];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cb = blockIdx.x, kb = blockIdx.y, split = blockIdx.z;
-    const int npix = a.H * a.W;
-    const int row = lane & 15, grp = lane >> 4;
-    const int co = cb * 16 + row;   // A row
-    const int kcol = kb * 16 + row; // B column
-    const int tap = kcol / a.cinp, ci = kcol - tap * a.cinp;
+    const int npix = a.H * a.W, hf = lane & 1;
+    const int tap = (kb * 16 + hf * 8) / a.cinp, ci = kb * 16 + hf * 8 - tap * a.cinp;
     const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    const int pbeg = split * a.pix_per_split;
-    int pend = pbeg + a.pix_per_split;
-    if (pend > npix) pend = npix;
+    const int pbeg = split * WGRAD_PIX;
+    const int pend = pbeg + WGRAD_PIX < npix ? pbeg + WGRAD_PIX : npix;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int pb = pbeg + 32 * wv; pb < pend; pb += 128) {
-        bf16x8 fa, fb;
-        const int p0 = pb + grp * 8;
-        int y = p0 / a.W, x = p0 - y * a.W;
+    const __bf16* __restrict__ dz = a.dz + cb * 16 + hf * 8;
+    const __bf16* __restrict__ in = a.in + a.off_in + ci;
+    auto load = [&](int it, bf16x8& va, bf16x8& vb, bool& ka, bool& kb) {
+        const int p = pbeg + it * 32 + (lane >> 1), y = p / a.W, x = p - y * a.W, yy = y + dy, xx = x + dx;
+        ka = p < pend;
+        kb = ka && tap < 9 && (unsigned)yy < (unsigned)a.H && (unsigned)xx < (unsigned)a.W;
+        va = *reinterpret_cast<const bf16x8*>(dz + (size_t)(ka ? p : 0) * a.cout);
+        vb = *reinterpret_cast<const bf16x8*>(kb ? in + (size_t)(yy * a.W + xx) * a.cs_in : a.in);
+    };
+    // lane (grp, row) takes pixels 8 grp .. 8 grp + 7 of channel row: two reads
+    // of 4 pixels, for which each 16 lanes address the 4 pixels' 16 channels
+    auto turned = [&](const bf16x8* p) {
+        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) bf16x4 lds4;
+        const char* q = reinterpret_cast<const char*>(p) + ((lane >> 4) * 8 + ((lane & 15) >> 2)) * 32 + (lane & 3) * 8;
+        const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4*)q);
+        const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds4*)(q + 4 * 32));
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto frag = [&](bf16x8* va, bf16x8* vb) {
+        bf16x8(*t)[2][64] = turn[wv];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int p = p0 + j, yy = y + dy, xx = x + dx;
-            const bool in = p < pend, ok = in && tap < 9 && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W;
-            const __bf16 va = a.dz[(size_t)(in ? p : 0) * a.cout + co];
-            const __bf16 vb = a.in[(size_t)(ok ? yy * a.W + xx : 0) * a.cs_in + a.off_in + (ok ? ci : 0)];
-            fa[j] = in ? va : (__bf16)0.0f;
-            fb[j] = ok ? vb : (__bf16)0.0f;
-            if (++x == a.W) { x = 0; ++y; }
+        for (int u = 0; u < PER; ++u) {
+            t[u][0][lane] = va[u];
+            t[u][1][lane] = vb[u];
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, acc, 0, 0, 0);
-    }
-    part[wv][lane] = acc;
-    __syncthreads();
-    if (wv != 0) return;
-    for (int q = 1; q < 4; ++q) acc += part[q][lane];
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            va[u] = turned(t[u][0]);
+            vb[u] = turned(t[u][1]);
+        }
+    };
+    relay_chain<NW, PER>(hand, (pend - pbeg + 31) / 32, wv, lane, acc, load, frag);
+    if (wv != NW - 1) return;
+    const int row = lane & 15, grp = lane >> 4, kcol = kb * 16 + row;
     // lane holds D[co = cb*16 + grp*4 + i][k = kb*16 + row]
     for (int i = 0; i < 4; ++i)
         a.partial[((size_t)split * a.cout + cb * 16 + grp * 4 + i) * a.kp + kcol] = acc[i];
+}
+
+// A wave for each 4 iterations of a split, up to 16 of them while that is a
+// workgroup per CU (132 KB of LDS each), or 8 while it is two; beyond, 4 waves
+// take the split in rounds: forward and backward at 512x1024 pixels 4.2 ms,
+// with 16 waves always 4.6.
+static void launch_wgrad(hipStream_t st, const WGradArgs& a, int nsplit)
+{
+    const int nit = (std::min(a.H * a.W, WGRAD_PIX) + 31) / 32;
+    const dim3 gr(a.cout / 16, a.kp / 16, nsplit);
+    const long wgs = (long)gr.x * gr.y * gr.z;
+    if (nit > 32 && wgs <= 256) hipLaunchKernelGGL((k_conv3x3_wgrad<16, 4>), gr, dim3(1024), 0, st, a);
+    else if (nit > 16 && wgs <= 512) hipLaunchKernelGGL((k_conv3x3_wgrad<8, 4>), gr, dim3(512), 0, st, a);
+    else if (nit > 4) hipLaunchKernelGGL((k_conv3x3_wgrad<4, 4>), gr, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_conv3x3_wgrad<1, 4>), gr, dim3(64), 0, st, a);
 }
 
 // The splits' sums into the gradient of W[co][tap][ci], and (the blocks past
@@ -539,16 +618,6 @@ static inline int up8(int c) { return (c + 7) / 8 * 8; }
 static inline int up16(int c) { return (c + 15) / 16 * 16; }
 static inline int up32(int c) { return (c + 31) / 32 * 32; }
 
-// pixels of a split of the weight gradient: multiples of 128 (a chunk of 32
-// for each wave), so that the launch has about 1024 workgroups, in at most
-// 64 splits
-int UNet::split_pixels(const Layer& l) const
-{
-    const int wg = (l.cout / 16) * (l.kp / 16), n = npx[l.lev];
-    const int splits = std::max(1, std::min(64, 1024 / wg));
-    return ((n + splits - 1) / splits + 127) / 128 * 128;
-}
-
 size_t UNet::param_count() const
 {
     size_t n = 0;
@@ -611,8 +680,7 @@ int UNet::alloc(int H_, int W_, bool train)
         TC_NN_TRY(dmal((void**)&dz, (size_t)npx[0] * 192 * sizeof(__bf16)));
         size_t maxpart = 0;
         for (Layer& l : L) {
-            const int pps = split_pixels(l);
-            l.nsplit = (npx[l.lev] + pps - 1) / pps;
+            l.nsplit = (npx[l.lev] + WGRAD_PIX - 1) / WGRAD_PIX;
             maxpart = std::max(maxpart, (size_t)l.nsplit * l.cout * l.kp);
         }
         TC_NN_TRY(dmal((void**)&wpart, maxpart * sizeof(float)));
@@ -691,9 +759,7 @@ void UNet::conv_back(hipStream_t st, const Layer& l, float* gy, int cs_y, int of
     hipLaunchKernelGGL(k_gelu_back, dim3(nblk((size_t)np * l.cout)), dim3(256), 0, st, gy, cs_y, off_y, l.z, dz, np,
                        l.cout);
     // weight and bias gradient
-    const int pps = split_pixels(l);
-    WGradArgs wa{dz, in, cs_in, off_in, l.cinp, l.kp, l.cout, wpart, H >> l.lev, W >> l.lev, pps};
-    hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(l.cout / 16, l.kp / 16, l.nsplit), dim3(256), 0, st, wa);
+    launch_wgrad(st, WGradArgs{dz, in, cs_in, off_in, l.cinp, l.kp, l.cout, wpart, H >> l.lev, W >> l.lev}, l.nsplit);
     const int wb = (int)nblk((size_t)l.cout * 9 * l.cin);
     hipLaunchKernelGGL(k_wgrad_finish, dim3(wb + l.cout), dim3(256), 0, st, wpart, l.nsplit, l.cin, l.cinp, l.cout, l.kp,
                        g32 + l.woff, wb, dz, np, g32 + l.boff);
