@@ -4,10 +4,11 @@
 the sweeps run on every level's viscosity), at heights where one tile holds
 all rows, where the tiles overlap, one row more, and where the taller tiles
 are taken; with lengths of the pass that split into one, two and three
-launches.  The operations are the reference's: what differs is exp(), by an
-ulp, which the solution shows times the condition of the fourth-order operator:
-about 4e-16 (nz/32)^4 (nz = 32: 1e-15, 104: 5e-14, 768: 3e-10), so 1e-12 at the
-largest height here, within the bound of 1e-10."""
+launches, and with passes that the host controls.  The operations are the
+reference's: what differs is exp(), by an ulp, which the solution shows times
+the condition of the fourth-order operator: about 4e-16 (nz/32)^4 (nz = 32:
+1e-15, 104: 5e-14, 768: 3e-10), so 1e-12 at the largest height here, within the
+bound of 1e-10."""
 import numpy as np
 import pytest
 
@@ -21,6 +22,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nx,nz,ov", [
     (16, 16, {}), (56, 32, {}), (52, 34, dict(vis_iter=5)), (106, 36, {}), (64, 64, dict(vis_iter=13)),
     (160, 96, {}), (152, 104, dict(visT=1e4)), (4096, 224, dict(vis_iter=7)),
+    # passes longer than the device loop's table: the host-controlled loop on a
+    # level below one whose viscosity was smoothed on a plane of its own
+    (64, 64, dict(vis_iter=33)), (152, 104, dict(vis_iter=40, visT=1e4)),
 ])
 def test_viscosity_sweeps_match_oracle(nx, nz, ov):
     cfg = dict(config.PRESETS["cfg2"], nx=nx, nz=nz, aspect=nx / nz, tpc=2, tolerance=1e-3, Nmulti=20, visT=100.0)

@@ -328,8 +328,9 @@ int grad_eig_min(tc_ctx* ctx, tc_dev& d, int level, double* rmin)
 }
 
 // smoother_vis (smoother.f90:165-263), host-controlled: one read-back of
-// the ratio minimum per iteration (passes longer than VIS_CMAX)
-int smoother_vis_host(tc_ctx* ctx, tc_dev& d, int level, int interpolate)
+// the ratio minimum per iteration (passes longer than VIS_CMAX).  Vfine: the
+// finer level's viscosity (level > 1; nullptr: that level's plane)
+int smoother_vis_host(tc_ctx* ctx, tc_dev& d, int level, int interpolate, const double* Vfine)
 {
     Level& L = ctx->lv[level];
     const tc_params& p = ctx->p;
@@ -342,7 +343,7 @@ int smoother_vis_host(tc_ctx* ctx, tc_dev& d, int level, int interpolate)
     if (p.RaT == 0.0) { kmin = 0; kmax = L.g.nz; } else { kmin = 1; kmax = L.g.nz - 1; }
     int n = 0, trigger = 0;
     const Grid* gf = level > 1 ? &ctx->lv[level - 1].g : &L.g;
-    const double* Vf = level > 1 ? ctx->lv[level - 1].vis : nullptr;
+    const double* Vf = level > 1 ? (Vfine ? Vfine : ctx->lv[level - 1].vis) : nullptr;
     for (;;) {
         for (int nn = ctx->nn_store; nn <= Niter; ++nn) {
             double rmin;
@@ -399,7 +400,8 @@ int smoother_vis(tc_ctx* ctx, tc_dev& d, int level, int interpolate, const doubl
     double lb, la;
     if (level == 1 && interpolate == 0) { option = 1; Niter = 6; lb = -5.0; la = -2.0; }
     else { option = 0; Niter = p.vis_iter; lb = -2.0; la = -1.0; }
-    if (!entered && (Niter > VIS_CMAX || p.vis_iter > VIS_CMAX)) return smoother_vis_host(ctx, d, level, interpolate);
+    if (!entered && (Niter > VIS_CMAX || p.vis_iter > VIS_CMAX))
+        return smoother_vis_host(ctx, d, level, interpolate, Vfine);
     if (interpolate == 0 || level == 1) { ctx->Nvis_store = 0; ctx->nn_store = 1; }
     int kmin, kmax;
     if (p.RaT == 0.0) { kmin = 0; kmax = L.g.nz; } else { kmin = 1; kmax = L.g.nz - 1; }
