@@ -257,8 +257,9 @@ int tc_autotune_dc_sweeps(tc_ctx* ctx, const int32_t* candidates, int32_t n, int
                           double* ms_per_step);
 /* Tile of the mixed mode's temporally blocked sweeps on `level` (2 ..
  * grids-1), as the cells that a workgroup holds, halo of 2 cells a sweep
- * included: 16, 32 or 48 (32x32, 64x32 or 64x32 with more rows a lane), 0 =
- * the whole visit is planned from the level's size. */
+ * included: 16, 32 or 48 (32x32, 64x32 or 64x32 with more rows a lane; a
+ * level that fits is held whole), 0 = the whole visit is planned from the
+ * level's size. */
 int tc_set_tb_tile(tc_ctx* ctx, int32_t level, int32_t tile);
 /* Autotuner of those tiles: level by level from 2, runs steps_each time
  * steps with each tile and keeps the faster (ties: the size-based choice);

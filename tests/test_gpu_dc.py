@@ -120,3 +120,27 @@ def test_tile_choice_and_autotune():
         assert all(t in (16, 32) for t in tiles[1:params.grids - 1])
         g.time_step(1)
         check_dc_solution(params, g, "autotuned tiles")
+
+
+@pytest.mark.parametrize("nx,nz,grids", [(304, 176, 5), (256, 128, 6)])
+def test_forced_tiles(nx, nz, grids):
+    """Every tile that can be forced, on levels larger than its region (ragged
+    tiles at 304x176) and smaller ones (held whole): the mixed mode's solution is
+    at the tolerance, and dc64, whose sweeps the setting does not steer, gives
+    the same bits."""
+    ref = None
+    for tile in (0, 16, 32, 48):
+        params, g, _ = solver_for("cfg2", nx=nx, nz=nz, grids=grids, tpc=4)
+        assert (params.nx, params.nz, params.grids) == (nx, nz, grids)
+        print(f"tile {tile}", flush=True)
+        with g:
+            for L in range(2, params.grids):
+                g.set_tb_tile(L, tile)
+            g.set_mode("dc64")
+            g.multigrid()
+            sf = g.get("SF")
+            ref = sf if ref is None else ref
+            assert np.array_equal(sf, ref)
+            g.set_mode("mixed")
+            g.time_step(1)
+            check_dc_solution(params, g, f"tile {tile}")

@@ -692,8 +692,9 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
     const VisitPlan plan = ref ? visit_plan_ref(L.g, d.cus) : VisitPlan{};
     int n = 1;
     if (tb && Niter > 0) {
-        // the tile asked for by tc_set_tb_tile: 16, 32 or 48, small to large regions
-        const int only = L.tb_tile == 16 ? 2 : (L.tb_tile == 32 ? 1 : (L.tb_tile == 48 ? 3 : 0));
+        // the tile asked for by tc_set_tb_tile (the mixed mode's): 16, 32 or 48,
+        // small to large regions
+        const int only = !f32 ? 0 : (L.tb_tile == 16 ? 2 : (L.tb_tile == 32 ? 1 : (L.tb_tile == 48 ? 3 : 0)));
         const Visit13Plan pl = visit_plan13(L.g, f32, Niter, f32 && rr, d.cus, only);
         const int body = (pl.end && !pl.whole) ? Niter - pl.end_k : Niter;  // sweeps of the equal launches
         double fac[VISIT_KMAX];

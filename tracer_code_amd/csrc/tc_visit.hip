@@ -722,21 +722,21 @@ static double cost13(int cfg, bool f32, int k, double tiles, int cus, bool end)
 // with the residual and restriction: 128x64 9.7 (15.0), 256x128 10.3 (14.6),
 // 512x256 14.7 (21.3); 16 sweeps of 1024x512 44 (85); 10 of 2048x1024, none:
 // 69 (127 as ten launches of one sweep).  only: 0, or the region that
-// tc_set_tb_tile asks for.
+// tc_set_tb_tile asks for; it too runs a level that it holds whole.
 Visit13Plan visit_plan13(const Grid& g, bool f32, int n, bool end, int cus, int only)
 {
     Visit13Plan p;
-    if (!only)
-        for (int c : {0, 4, 2, 1}) {
-            const VisitRegion rg = region13(c, f32);
-            if (g.nx <= rg.w && g.nz - 1 <= rg.r && (c != 1 || n >= 8)) {
-                p.cfg = p.end_cfg = c;
-                p.whole = true;
-                p.launches = (n + VISIT_KMAX - 1) / VISIT_KMAX;
-                p.end = end;
-                return p;
-            }
+    for (int c : {0, 4, 2, 1, 3}) {
+        if (only ? c != only : c == 3) continue;
+        const VisitRegion rg = region13(c, f32);
+        if (g.nx <= rg.w && g.nz - 1 <= rg.r && (only || c != 1 || n >= 8)) {
+            p.cfg = p.end_cfg = c;
+            p.whole = true;
+            p.launches = (n + VISIT_KMAX - 1) / VISIT_KMAX;
+            p.end = end;
+            return p;
         }
+    }
     auto cost = [&](int c, int k, bool e) {
         const VisitRegion rg = region13(c, f32);
         const VisitTile t = tiles_for(g, rg.w, rg.r, k, e);
