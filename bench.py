@@ -208,9 +208,9 @@ def apply_counts(solver, params, counts):
     if params.grids > 2:
         solver.set_dc_level_sweeps(2, counts["level2"])
     if counts.get("tiles"):
-        for L, t in enumerate(counts["tiles"], start=1):
-            if t:
-                solver.set_tb_tile(L, t)
+        # (0: planned from the level's size)
+        for L in range(2, params.grids):
+            solver.set_tb_tile(L, counts["tiles"][L - 1])
 
 
 def run_timed(solver, params, warmup, steps, label, profile=False, until_time=None):

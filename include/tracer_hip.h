@@ -262,8 +262,9 @@ int tc_autotune_dc_sweeps(tc_ctx* ctx, const int32_t* candidates, int32_t n, int
  * level's size. */
 int tc_set_tb_tile(tc_ctx* ctx, int32_t level, int32_t tile);
 /* Autotuner of those tiles: level by level from 2, runs steps_each time
- * steps with each tile and keeps the faster (ties: the size-based choice);
- * tiles[TC_MAX_LEVELS] (may be NULL) receives the tile of each level
+ * steps with the plan by size (0) and with each tile on the levels that no
+ * region holds, and sets the tile that is 2% faster than the plan, else 0;
+ * tiles[TC_MAX_LEVELS] (may be NULL) receives the choice of each level
  * (0 where the level has no such sweeps). */
 int tc_autotune_tb_tiles(tc_ctx* ctx, int32_t steps_each, int32_t* tiles);
 int tc_get_stats(const tc_ctx* ctx, tc_stats* out);

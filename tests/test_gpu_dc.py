@@ -105,8 +105,9 @@ def test_dc_sweeps_retry_and_autotune():
 
 
 def test_tile_choice_and_autotune():
-    """Both tiles of the temporally blocked sweeps give solves at the
-    tolerance; the tile autotuner keeps 16 or 32 on every level it tunes."""
+    """Two tiles of the blocked sweeps give solves at the tolerance; the tile
+    autotuner keeps the plan by size (0) on the levels that a region holds (at
+    256x128 those from 3 down) and may force a tile on the others."""
     params, g, _ = solver_for("cfg2", nx=256, nz=128, tpc=4)
     with g:
         g.set_mode("mixed")
@@ -117,7 +118,8 @@ def test_tile_choice_and_autotune():
             check_dc_solution(params, g, f"tiles {tile}")
         tiles = g.autotune_tb_tiles(1)
         print(f"autotuned tiles {tiles}", flush=True)
-        assert all(t in (16, 32) for t in tiles[1:params.grids - 1])
+        assert all(t in (0, 16, 32, 48) for t in tiles)
+        assert params.grids == 6 and tiles[2:] == [0] * len(tiles[2:])
         g.time_step(1)
         check_dc_solution(params, g, "autotuned tiles")
 

@@ -2780,19 +2780,23 @@ int tc_autotune_tb_tiles(tc_ctx* ctx, int32_t steps_each, int32_t* tiles)
     for (int L = 2; L < ctx->grids; ++L) {
         Level& lv = ctx->lv[L];
         const int keep = lv.tb_tile;
-        // 16, 32 and 48 (where it still gives 128 workgroups); a candidate
-        // replaces the kept tile only when it is 2% faster
-        const int cand[3] = {16, 32, 48};
+        // the plan by size first: a tile replaces it only when it is 2% faster.
+        // A level that a region holds has one launch a visit, which no tile
+        // makes fewer: it keeps the plan
+        const int cand[4] = {0, 16, 32, 48};
         double best_ms = 0.0;
-        int best = keep;
-        for (int c = 0; c < 3; ++c) {
-            const dim3 t = dim3((lv.g.nx - 1 + cand[c] - 1) / cand[c], (lv.g.nz - 1 + cand[c] - 1) / cand[c]);
-            if (cand[c] == 48 && t.x * t.y < 128) continue;
-            double ms = 0.0;
-            lv.tb_tile = cand[c];
-            TC_TRY(step_ms(&ms));
-            if (c == 0 || ms < 0.98 * best_ms) { best_ms = ms; best = cand[c]; }
-        }
+        int best = 0;
+        if (!visit_plan13(lv.g, true, 8, false, DEV(ctx).cus, 0).whole)
+            for (int c = 0; c < 4; ++c) {
+                double ms = 0.0;
+                lv.tb_tile = cand[c];
+                const int st = step_ms(&ms);
+                if (st) {
+                    lv.tb_tile = keep;
+                    return st;
+                }
+                if (c == 0 || ms < 0.98 * best_ms) { best_ms = ms; best = cand[c]; }
+            }
         lv.tb_tile = best;
     }
     if (tiles)

@@ -77,9 +77,8 @@ def make_solvers(cases, mode="mixed", guess="plain", weights=None, level=4, tune
                     n = t["level2"] if L == 2 else t["coarse"]
                     if n:
                         g.set_dc_level_sweeps(L, n)
-                for L, tile in enumerate(t["tiles"], start=1):
-                    if 2 <= L < params.grids and tile:
-                        g.set_tb_tile(L, tile)
+                for L in range(2, params.grids):   # tile 0: planned from the level's size
+                    g.set_tb_tile(L, t["tiles"][L - 1])
         solvers.append(g)
     return solvers, nets
 

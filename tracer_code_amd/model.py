@@ -262,8 +262,9 @@ class Solver:
         self._check(self.lib.tc_set_tb_tile(self.h, int(level), int(tile)), "set_tb_tile")
 
     def autotune_tb_tiles(self, steps_each=1):
-        """Level-by-level choice of the temporally blocked tile (16 or 32);
-        returns the tile of each level (index 0 = level 1)."""
+        """Level-by-level choice of the blocked sweeps' tile (0: the plan by the
+        level's size, else 16, 32 or 48); returns the tile of each level (index
+        0 = level 1)."""
         t = np.zeros(_abi.TC_MAX_LEVELS, dtype=np.int32)
         self._check(self.lib.tc_autotune_tb_tiles(self.h, int(steps_each), t.ctypes.data), "autotune_tb_tiles")
         return t.tolist()
