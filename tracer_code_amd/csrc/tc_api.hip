@@ -1919,7 +1919,7 @@ int smoother_time(tc_ctx* ctx, tc_dev& d, int32_t* n_comp)
             return 2.0 / (-lb - la + (lb - la) * std::cos((double)(2 * ntemp - 1) * PII / (double)(2 * N)));
         };
         int iters = 0;
-        if (ctx->filter_blocking && filter_multi_takes(ctx->g, d.F))
+        if (ctx->filter_blocking && filter_multi_takes(d.F))
             TC_TRY(filter_loop_multi(ctx, d, ctx->Cvis[t], ctx->tmp2, d.fbuf, P.delta_C[t], P.courantC, cfac, &iters));
         else
             TC_TRY(filter_loop(ctx, d, ctx->Cvis[t], ctx->tmp2, true, P.delta_C[t], P.courantC, cfac, &iters));

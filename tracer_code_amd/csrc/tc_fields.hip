@@ -301,7 +301,9 @@ __global__ __launch_bounds__(256) void k_filter_iter(const double* __restrict__ 
 // nz+2, the tiles between hold no ghost row (the last of them is moved up
 // where it would, and cells that two tiles own get the same value from
 // both): the ghost rows are then fixed registers of the first and the last
-// tile, and the others have no row test at all.  dts_array is one value on
+// tile, and the others have no row test at all.  Below 17 rows the two ends
+// would share a tile; there one tile holds all rows (FM_ALL of them at most,
+// no halo in z) and tests each against row nz.  dts_array is one value on
 // the uniform grids the library accepts.  After each iteration the tile's
 // own nodes give that iterate's smoothness maximum, reduced over the block
 // once per launch (one slot set per iterate).
@@ -344,6 +346,7 @@ constexpr int FM_TXO = 64 - 2 * FM_H;    // own columns of a wavefront's tile
 constexpr int FM_WAVES = 4;              // tiles (stacked in z) per workgroup
 constexpr int FM_SETS = 3 * FM_K;
 constexpr int FM_TYS[4] = {8, 11, 16, 21};  // own rows of a tile, chosen by the grid's size
+constexpr int FM_ALL = FM_TYS[0] + 2 * FM_H - 2 + 2 * SPAN + 1;  // rows of a tile that holds all of them (nz <= 16)
 
 struct FmFac { double v[2 * FM_K]; };    // factors of the previous launch's iterations, then this one's
 struct FmBufs { double* v[3]; };
@@ -363,24 +366,30 @@ __host__ __device__ inline int fm_tile_row(int nz, int TY, int t, int tiles)
 }
 
 // One tile's n iterations.  ZK: 0 = no ghost rows held, 1 = the first tile,
-// 2 = the last.  D2 is (1, -2, 1) at offsets -1, 0, 1 (the second-order
+// 2 = the last, 3 = all rows, from row -2.  D2 is (1, -2, 1) at offsets -1, 0, 1 (the second-order
 // table): the products by 1 and -2 are exact.  POW2: dr^2 and ds^2 are powers
 // of two, so that the quotients are exact scalings and go into the sum's FMA;
 // else they are divisions.  The values are filter_new's, bit for bit.
-template <bool POW2, int TY, int ZK>
-__device__ __forceinline__ void fm_iterate(double (&c)[TY + 2 * FM_H], double (&mx)[FM_K], int n, bool measure,
+template <bool POW2, int TY, int RY, int ZK>
+__device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], int n, bool measure,
                                            const double* fac, double dtc, const FScale& sc, bool gcols, bool ghost_col,
-                                           bool corner_col, int ml, bool own_col)
+                                           bool corner_col, int ml, bool own_col, int nz)
 {
-    constexpr int RY = TY + 2 * FM_H;
-    constexpr int R0 = FM_H + SPAN;            // row 0 in the first tile
-    constexpr int RN = TY + FM_H - SPAN - 1;   // row nz in the last tile
+    constexpr int R0 = ZK == 3 ? SPAN : FM_H + SPAN;  // row 0 in the first tile
+    constexpr int RN = TY + FM_H - SPAN - 1;          // row nz in the last tile
+    const int rn = nz + SPAN;                         // row nz in a tile of all rows
     // rows measured: 1..nz-1 of the own ones
-    constexpr int RA = ZK == 1 ? R0 + 1 : FM_H, RB = ZK == 2 ? RN - 1 : FM_H + TY - 1;
+    constexpr int RA = ZK & 1 ? R0 + 1 : FM_H, RB = ZK == 3 ? RY - 2 : (ZK == 2 ? RN - 1 : FM_H + TY - 1);
 #pragma unroll 1
     for (int it = 0; it < n; ++it) {
         const double cfd = fac[it] * dtc;
-        const double old1 = ZK == 1 ? c[R0 + 1] : (ZK == 2 ? c[RN - 1] : 0.0);
+        const double old1 = ZK & 1 ? c[R0 + 1] : (ZK == 2 ? c[RN - 1] : 0.0);
+        double oldn = 0.0;
+        if constexpr (ZK == 3) {
+#pragma unroll
+            for (int r = R0; r < RY; ++r)
+                if (r == rn - 1) oldn = c[r];
+        }
         // the step (filter_new's operation order) on every held row but the
         // first and last; ghost cells are overwritten below, cells outside
         // the plane are never read by the valid part of the region
@@ -420,9 +429,16 @@ __device__ __forceinline__ void fm_iterate(double (&c)[TY + 2 * FM_H], double (&
         }
         // ghost rows: the mirrored row (columns already mirrored), the row-1
         // corners from the previous iterate
-        if constexpr (ZK == 1) {
+        if constexpr (ZK & 1) {
             c[R0 - 1] = corner_col ? old1 : c[R0 + 1];
             c[R0 - 2] = c[R0 + 2];
+        }
+        if constexpr (ZK == 3) {
+#pragma unroll
+            for (int r = R0 + 2; r < RY; ++r) {
+                if (r == rn + 1) c[r] = corner_col ? oldn : c[r - 2];
+                if (r == rn + 2) c[r] = c[r - 4];
+            }
         }
         if constexpr (ZK == 2) {
             c[RN + 1] = corner_col ? old1 : c[RN - 1];
@@ -437,6 +453,7 @@ __device__ __forceinline__ void fm_iterate(double (&c)[TY + 2 * FM_H], double (&
             double rm = dpp_from_right(c[RA - 1]), r0 = dpp_from_right(c[RA]);  // the right lane's c[r-1], c[r]
 #pragma unroll
             for (int r = RA; r <= RB; ++r) {
+                if (ZK == 3 && r >= rn) break;
                 const double rp = dpp_from_right(c[r + 1]);
                 a = fmax(a, fabs(rm - c[r]));
                 b = fmax(b, fabs(r0 - c[r]));
@@ -452,13 +469,14 @@ __device__ __forceinline__ void fm_iterate(double (&c)[TY + 2 * FM_H], double (&
     }
 }
 
-template <bool POW2, int TY>
+// ALL: one tile of all rows, the waves of a workgroup beside each other in x
+template <bool POW2, int TY, bool ALL>
 __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, const double* __restrict__ dts, Grid g,
                                                       FScale sc, double courant, FmFac fac, int m, double delta,
                                                       int tiles, unsigned long long* __restrict__ slots,
                                                       int32_t* __restrict__ ctl)
 {
-    constexpr int RY = TY + 2 * FM_H;
+    constexpr int RY = ALL ? FM_ALL : TY + 2 * FM_H;
     // ctl[0] = m+1 marks the stop taken by the launch with input iterate m:
     // the later launches return, the blocks of that launch still do its work
     {
@@ -500,15 +518,16 @@ __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, con
             slots[(size_t)(j % FM_SETS) * FILT_SET + tid * FILT_STRIDE] = 0ull;
     const int nx = g.nx, nz = g.nz;
     const int wy = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int t = blockIdx.y * FM_WAVES + wy;  // the wave's tile (uniform)
+    const int t = ALL ? 0 : blockIdx.y * FM_WAVES + wy;  // the wave's tile (uniform)
+    const int i0 = (ALL ? blockIdx.x * FM_WAVES + wy : blockIdx.x) * FM_TXO - SPAN;
     double mx[FM_K];
 #pragma unroll
     for (int j = 0; j < FM_K; ++j) mx[j] = 0.0;
-    if (t < tiles) {
-        const int zk = t == 0 ? 1 : (t == tiles - 1 ? 2 : 0);
-        const int i0 = blockIdx.x * FM_TXO - SPAN, k0 = fm_tile_row(nz, TY, t, tiles);
+    if (ALL ? i0 <= nx + SPAN : t < tiles) {
+        const int zk = ALL ? 3 : (t == 0 ? 1 : (t == tiles - 1 ? 2 : 0));
+        const int k0 = ALL ? -SPAN : fm_tile_row(nz, TY, t, tiles);
         const int sx = i0 - nx + 1 > 0 ? i0 - nx + 1 : 0;
-        const int ri0 = i0 - FM_H - sx, rk0 = k0 - FM_H;  // held region origin
+        const int ri0 = i0 - FM_H - sx, rk0 = ALL ? k0 : k0 - FM_H;  // held region origin
         const int i = ri0 + lane;                          // this lane's column
         const bool col_in = i >= -SPAN && i <= nx + SPAN, col_int = i >= 0 && i <= nx;
         const bool corner_col = i == -SPAN || i == nx + SPAN;
@@ -530,17 +549,20 @@ __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, con
         const bool gcols = ri0 <= -1 || ri0 + 63 >= nx + 1;  // the held columns include ghost columns (uniform)
         const bool own_col = i >= i0 && i < i0 + FM_TXO && i >= 0 && i <= nx - 1;  // columns measured
         const double* f = replay ? fac.v : fac.v + FM_K;
-        if (zk == 0)
-            fm_iterate<POW2, TY, 0>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col);
-        else if (zk == 1)
-            fm_iterate<POW2, TY, 1>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col);
-        else
-            fm_iterate<POW2, TY, 2>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col);
+        auto go = [&](auto z) {
+            fm_iterate<POW2, TY, RY, decltype(z)::value>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml,
+                                                         own_col, nz);
+        };
+        if constexpr (ALL) go(std::integral_constant<int, 3>{});
+        else if (zk == 0) go(std::integral_constant<int, 0>{});
+        else if (zk == 1) go(std::integral_constant<int, 1>{});
+        else go(std::integral_constant<int, 2>{});
         // the tile's own cells of the last iterate
         if (col_in && i >= i0 && i < i0 + FM_TXO) {
             double* __restrict__ dp = dst + g.at(i, k0);
 #pragma unroll
-            for (int r = 0; r < TY; ++r) dp[(ptrdiff_t)r * g.ld] = c[FM_H + r];
+            for (int r = 0; r < (ALL ? RY : TY); ++r)
+                if (!ALL || k0 + r <= nz + SPAN) dp[(ptrdiff_t)r * g.ld] = c[(ALL ? 0 : FM_H) + r];
         }
     }
     if (!replay) {
@@ -1208,18 +1230,15 @@ int filter_multi_k() { return FM_K; }
 // whether tiles of ty rows fit: the first and the last one hold the ghost
 // rows of their own side only, and those between none
 static bool fm_fits(int nz, int ty) { return nz >= ty + 2 * FM_H - 1; }
-bool filter_multi_takes(const Grid& g, const FD& F)
-{
-    return fm_fits(g.nz, FM_TYS[0]) && F.D2[1] == 1.0 && F.D2[2] == -2.0 && F.D2[3] == 1.0;
-}
+bool filter_multi_takes(const FD& F) { return F.D2[1] == 1.0 && F.D2[2] == -2.0 && F.D2[3] == 1.0; }
 
-template <bool POW2, int TY>
+template <bool POW2, int TY, bool ALL = false>
 static void filter_multi_go(hipStream_t st, dim3 gr, const FmBufs& b, int b_in, const double* dts, const Grid& g,
                             const FScale& sc, double courant, const FmFac& f, int m, double delta,
                             unsigned long long* slots, int32_t* ctl)
 {
-    hipLaunchKernelGGL((k_filter_multi<POW2, TY>), gr, dim3(64, FM_WAVES), 0, st, b, b_in, dts, g, sc, courant, f, m,
-                       delta, fm_tiles(g.nz, TY), slots, ctl);
+    hipLaunchKernelGGL((k_filter_multi<POW2, TY, ALL>), gr, dim3(64, FM_WAVES), 0, st, b, b_in, dts, g, sc, courant, f,
+                       m, delta, ALL ? 1 : fm_tiles(g.nz, TY), slots, ctl);
 }
 
 void launch_filter_multi(hipStream_t st, double* const bufs[3], int b_in, const double* dts, const Grid& g, double dr2,
@@ -1249,6 +1268,13 @@ void launch_filter_multi(hipStream_t st, double* const bufs[3], int b_in, const 
     const FScale sc = filter_scale(dr2, ds2);
     auto go = [&](auto pw) {
         constexpr bool P = decltype(pw)::value;
+        // fewer rows than the lowest tiles need (11 iterations of 64x16: 109 us,
+        // one launch each 186)
+        if (best < 0) {
+            filter_multi_go<P, FM_TYS[0], true>(st, dim3((gx + FM_WAVES - 1) / FM_WAVES), b, b_in, dts, g, sc, courant, f, m,
+                                                delta, slots, ctl);
+            return;
+        }
         switch (TY) {
         case FM_TYS[0]: filter_multi_go<P, FM_TYS[0]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
         case FM_TYS[1]: filter_multi_go<P, FM_TYS[1]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
