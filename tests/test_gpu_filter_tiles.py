@@ -1,6 +1,6 @@
 """The C filter's tiles (k_filter_multi) against one launch per iteration, on
 fields that the tracers do not give: random ratios, values beyond [0,1] (the
-clamp) and a NaN, at the heights and widths where a tile ends -- heights that
+clamp), a NaN, and infinities and values whose quotients overflow, at the heights and widths where a tile ends -- heights that
 one tile holds (4 to 16 rows), the smallest height with tiles, a last tile
 that overlaps the one before it, one column or row more than a tile.  Same
 iterates, stop and bits."""
@@ -12,7 +12,7 @@ from tracer_code_amd import Solver, config
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kind", ["ratio", "beyond", "nan"])
+@pytest.mark.parametrize("kind", ["ratio", "beyond", "nan", "huge"])
 @pytest.mark.parametrize("nx,nz", [(12, 4), (52, 6), (10, 16), (24, 16), (104, 10),
                                    (300, 14), (16, 18), (54, 20), (56, 38), (108, 50), (110, 26), (160, 96), (212, 130),
                                    (1024, 512), (1920, 992)])
@@ -31,6 +31,8 @@ def test_filter_tiles_same_bits(nx, nz, kind):
         C[rng.random(C.shape) < 0.1] = -0.25
     if kind == "nan":
         C[nz // 2, nx // 2] = np.nan
+    if kind == "huge":
+        C[1, nx // 3], C[nz // 2, 2], C[nz - 1, nx // 2], C[nz // 2, nx - 1] = np.inf, -np.inf, 1e307, -1e307
     out = []
     with Solver(params, 0) as g:
         for blocking in (False, True):

@@ -367,10 +367,15 @@ __host__ __device__ inline int fm_tile_row(int nz, int TY, int t, int tiles)
 
 // One tile's n iterations.  ZK: 0 = no ghost rows held, 1 = the first tile,
 // 2 = the last, 3 = all rows, from row -2.  D2 is (1, -2, 1) at offsets -1, 0, 1 (the second-order
-// table): the products by 1 and -2 are exact.  POW2: dr^2 and ds^2 are powers
-// of two, so that the quotients are exact scalings and go into the sum's FMA;
-// else they are divisions.  The values are filter_new's, bit for bit.
-template <bool POW2, int TY, int RY, int ZK>
+// table): the products by 1 and -2 are exact.  FORM: where dr^2 and ds^2 are
+// powers of two (FM_POW2) the quotients are exact scalings and go into the
+// sum's FMA; else they are div_by's, or (FM_WIDE) divisions: a tile that holds
+// a value beyond FM_HUGE, whose quotient may be infinite, which div_by makes a
+// NaN.  The values are filter_new's, bit for bit (down to quotients of 1e-290,
+// where div_by's remainder is no longer exact).
+enum { FM_POW2, FM_DIV, FM_WIDE };
+constexpr double FM_HUGE = 1e150;
+template <int FORM, int TY, int RY, int ZK>
 __device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], int n, bool measure,
                                            const double* fac, double dtc, const FScale& sc, bool gcols, bool ghost_col,
                                            bool corner_col, int ml, bool own_col, int nz)
@@ -401,8 +406,9 @@ __device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], 
             const double lf = dpp_from_left(oc), rt = dpp_from_right(oc);
             const double x = fma(-2.0, oc, lf) + rt, z = fma(-2.0, oc, om) + c[r + 1];
             double temp;
-            if constexpr (POW2) temp = fma(x, sc.idr2, z * sc.ids2);
-            else temp = div_by(x, sc.dr2, sc.idr2) + div_by(z, sc.ds2, sc.ids2);
+            if constexpr (FORM == FM_POW2) temp = fma(x, sc.idr2, z * sc.ids2);
+            else if constexpr (FORM == FM_DIV) temp = div_by(x, sc.dr2, sc.idr2) + div_by(z, sc.ds2, sc.ids2);
+            else temp = x / sc.dr2 + z / sc.ds2;
             const double v = oc + cfd * temp;
             // 0 <= v <= 1 by the bits (a negative or NaN value is above 1's)
             out = out || (unsigned long long)__double_as_longlong(v) > 0x3FF0000000000000ull;
@@ -549,9 +555,19 @@ __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, con
         const bool gcols = ri0 <= -1 || ri0 + 63 >= nx + 1;  // the held columns include ghost columns (uniform)
         const bool own_col = i >= i0 && i < i0 + FM_TXO && i >= 0 && i <= nx - 1;  // columns measured
         const double* f = replay ? fac.v : fac.v + FM_K;
+        bool wide = false;  // (never set with POW2; a NaN stays one in either form)
+        if constexpr (!POW2) {
+#pragma unroll
+            for (int r = 0; r < RY; ++r) wide = wide || fabs(c[r]) > FM_HUGE;
+            wide = __any(wide);
+        }
         auto go = [&](auto z) {
-            fm_iterate<POW2, TY, RY, decltype(z)::value>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml,
-                                                         own_col, nz);
+            constexpr int ZK = decltype(z)::value;
+            if (!POW2 && wide)
+                fm_iterate<FM_WIDE, TY, RY, ZK>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col, nz);
+            else
+                fm_iterate<POW2 ? FM_POW2 : FM_DIV, TY, RY, ZK>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col,
+                                                                ml, own_col, nz);
         };
         if constexpr (ALL) go(std::integral_constant<int, 3>{});
         else if (zk == 0) go(std::integral_constant<int, 0>{});
