@@ -43,3 +43,23 @@ def test_filter_tiles_same_bits(nx, nz, kind):
             out.append((g.get("Cvis"), n, g.stats().c_iters - n0))
     assert out[0][1] == out[1][1] and out[0][2] == out[1][2] and out[0][2] > 4
     assert np.array_equal(out[0][0], out[1][0], equal_nan=True)
+
+
+@pytest.mark.parametrize("nx,nz", [(24, 16), (64, 32), (108, 50), (256, 128)])
+def test_other_table_same_bits(nx, nz):
+    """A second-derivative table that is not (1, -2, 1), on spacings that are
+    powers of two and not."""
+    params = config.make_params(nx=nx, nz=nz, aspect=nx / nz, grids=2, ivis=2, visC=(1.0 / 30.0,), delta_visC=(1.5,))
+    params.D2[1], params.D2[2], params.D2[3] = 0.96, -1.93, 0.98
+    print(f"[filter tiles] {params.nx}x{params.nz} other table", flush=True)
+    C = np.random.default_rng(nx).integers(0, 21, (nz + 5, nx + 5, 1)) / 20.0
+    out = []
+    with Solver(params, 0) as g:
+        for blocking in (False, True):
+            g.set_filter_blocking(blocking)
+            g.put("Cnew", C)
+            n0 = g.stats().c_iters
+            n = g.smoother_time()
+            out.append((g.get("Cvis"), n, g.stats().c_iters - n0))
+    assert out[0][1:] == out[1][1:] and out[0][2] > 4
+    assert np.array_equal(out[0][0], out[1][0])

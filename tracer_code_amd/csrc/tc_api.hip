@@ -1858,7 +1858,7 @@ int filter_loop_multi(tc_ctx* ctx, tc_dev& d, double* A, double* B, double* C, d
                 fac[j] = (m - K + j >= 0) ? cfac(m - K + j) : 0.0;
                 fac[K + j] = cfac(m + j);
             }
-            launch_filter_multi(ctx->stream, bufs, l % 3, ctx->dts, ctx->g, ctx->lv[1].dr2, ctx->lv[1].ds2, courant,
+            launch_filter_multi(ctx->stream, bufs, l % 3, ctx->dts, ctx->g, d.F, ctx->lv[1].dr2, ctx->lv[1].ds2, courant,
                                 fac.data(), m, delta, d.fslots, d.ctl, d.cus);
         }
         TC_HIP(hipGetLastError());
@@ -1919,7 +1919,7 @@ int smoother_time(tc_ctx* ctx, tc_dev& d, int32_t* n_comp)
             return 2.0 / (-lb - la + (lb - la) * std::cos((double)(2 * ntemp - 1) * PII / (double)(2 * N)));
         };
         int iters = 0;
-        if (ctx->filter_blocking && filter_multi_takes(d.F))
+        if (ctx->filter_blocking)
             TC_TRY(filter_loop_multi(ctx, d, ctx->Cvis[t], ctx->tmp2, d.fbuf, P.delta_C[t], P.courantC, cfac, &iters));
         else
             TC_TRY(filter_loop(ctx, d, ctx->Cvis[t], ctx->tmp2, true, P.delta_C[t], P.courantC, cfac, &iters));

@@ -366,19 +366,24 @@ __host__ __device__ inline int fm_tile_row(int nz, int TY, int t, int tiles)
 }
 
 // One tile's n iterations.  ZK: 0 = no ghost rows held, 1 = the first tile,
-// 2 = the last, 3 = all rows, from row -2.  D2 is (1, -2, 1) at offsets -1, 0, 1 (the second-order
-// table): the products by 1 and -2 are exact.  FORM: where dr^2 and ds^2 are
-// powers of two (FM_POW2) the quotients are exact scalings and go into the
-// sum's FMA; else they are div_by's, or (FM_WIDE) divisions: a tile that holds
-// a value beyond FM_HUGE, whose quotient may be infinite, which div_by makes a
-// NaN.  The values are filter_new's, bit for bit (down to quotients of 1e-290,
-// where div_by's remainder is no longer exact).
-enum { FM_POW2, FM_DIV, FM_WIDE };
-constexpr double FM_HUGE = 1e150;
+// 2 = the last, 3 = all rows, from row -2.  FORM: with D2 = (1, -2, 1) at
+// offsets -1, 0, 1 (the second-order table) the products by 1 and -2 are exact,
+// and where dr^2 and ds^2 are powers of two (FM_POW2) the quotients are exact
+// scalings that go into the sum's FMA; else they are div_by's (FM_DIV).
+// FM_ANY: products with the table and divisions, for another table and for a
+// tile that holds a value from 2^500 on, whose quotient may be infinite, which
+// div_by makes a NaN.  The values are filter_new's, bit for bit (down to
+// quotients of 1e-290, where div_by's remainder is no longer exact).
+enum { FM_POW2, FM_DIV, FM_ANY };
+constexpr unsigned FM_HUGE = 0x5f300000u;  // high word of 2^500
+struct FmTable {
+    double d[3];  // D2 at offsets -1, 0, 1
+    int other;    // not the second-order table
+};
 template <int FORM, int TY, int RY, int ZK>
 __device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], int n, bool measure,
-                                           const double* fac, double dtc, const FScale& sc, bool gcols, bool ghost_col,
-                                           bool corner_col, int ml, bool own_col, int nz)
+                                           const double* fac, double dtc, const FScale& sc, const FmTable& tb,
+                                           bool gcols, bool ghost_col, bool corner_col, int ml, bool own_col, int nz)
 {
     constexpr int R0 = ZK == 3 ? SPAN : FM_H + SPAN;  // row 0 in the first tile
     constexpr int RN = TY + FM_H - SPAN - 1;          // row nz in the last tile
@@ -404,11 +409,15 @@ __device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], 
         for (int r = 1; r < RY - 1; ++r) {
             const double oc = c[r];
             const double lf = dpp_from_left(oc), rt = dpp_from_right(oc);
-            const double x = fma(-2.0, oc, lf) + rt, z = fma(-2.0, oc, om) + c[r + 1];
             double temp;
-            if constexpr (FORM == FM_POW2) temp = fma(x, sc.idr2, z * sc.ids2);
-            else if constexpr (FORM == FM_DIV) temp = div_by(x, sc.dr2, sc.idr2) + div_by(z, sc.ds2, sc.ids2);
-            else temp = x / sc.dr2 + z / sc.ds2;
+            if constexpr (FORM == FM_ANY) {
+                const double x = tb.d[0] * lf + tb.d[1] * oc + tb.d[2] * rt, z = tb.d[0] * om + tb.d[1] * oc + tb.d[2] * c[r + 1];
+                temp = x / sc.dr2 + z / sc.ds2;
+            } else {
+                const double x = fma(-2.0, oc, lf) + rt, z = fma(-2.0, oc, om) + c[r + 1];
+                if constexpr (FORM == FM_POW2) temp = fma(x, sc.idr2, z * sc.ids2);
+                else temp = div_by(x, sc.dr2, sc.idr2) + div_by(z, sc.ds2, sc.ids2);
+            }
             const double v = oc + cfd * temp;
             // 0 <= v <= 1 by the bits (a negative or NaN value is above 1's)
             out = out || (unsigned long long)__double_as_longlong(v) > 0x3FF0000000000000ull;
@@ -478,8 +487,8 @@ __device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], 
 // ALL: one tile of all rows, the waves of a workgroup beside each other in x
 template <bool POW2, int TY, bool ALL>
 __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, const double* __restrict__ dts, Grid g,
-                                                      FScale sc, double courant, FmFac fac, int m, double delta,
-                                                      int tiles, unsigned long long* __restrict__ slots,
+                                                      FScale sc, FmTable tb, double courant, FmFac fac, int m,
+                                                      double delta, int tiles, unsigned long long* __restrict__ slots,
                                                       int32_t* __restrict__ ctl)
 {
     constexpr int RY = ALL ? FM_ALL : TY + 2 * FM_H;
@@ -555,19 +564,21 @@ __global__ __launch_bounds__(256) void k_filter_multi(FmBufs bufs, int b_in, con
         const bool gcols = ri0 <= -1 || ri0 + 63 >= nx + 1;  // the held columns include ghost columns (uniform)
         const bool own_col = i >= i0 && i < i0 + FM_TXO && i >= 0 && i <= nx - 1;  // columns measured
         const double* f = replay ? fac.v : fac.v + FM_K;
-        bool wide = false;  // (never set with POW2; a NaN stays one in either form)
+        bool any = false;  // (not with POW2; by the magnitudes' high words, NaNs included)
         if constexpr (!POW2) {
+            unsigned top = 0;
 #pragma unroll
-            for (int r = 0; r < RY; ++r) wide = wide || fabs(c[r]) > FM_HUGE;
-            wide = __any(wide);
+            for (int r = 0; r < RY; ++r) top = max(top, (unsigned)__double2hiint(c[r]) & 0x7fffffffu);
+            any = __any(top >= FM_HUGE) || tb.other;
         }
         auto go = [&](auto z) {
             constexpr int ZK = decltype(z)::value;
-            if (!POW2 && wide)
-                fm_iterate<FM_WIDE, TY, RY, ZK>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col, ml, own_col, nz);
+            if (!POW2 && any)
+                fm_iterate<FM_ANY, TY, RY, ZK>(c, mx, n, !replay, f, dtc, sc, tb, gcols, ghost_col, corner_col, ml, own_col,
+                                               nz);
             else
-                fm_iterate<POW2 ? FM_POW2 : FM_DIV, TY, RY, ZK>(c, mx, n, !replay, f, dtc, sc, gcols, ghost_col, corner_col,
-                                                                ml, own_col, nz);
+                fm_iterate<POW2 ? FM_POW2 : FM_DIV, TY, RY, ZK>(c, mx, n, !replay, f, dtc, sc, tb, gcols, ghost_col,
+                                                                corner_col, ml, own_col, nz);
         };
         if constexpr (ALL) go(std::integral_constant<int, 3>{});
         else if (zk == 0) go(std::integral_constant<int, 0>{});
@@ -1246,19 +1257,18 @@ int filter_multi_k() { return FM_K; }
 // whether tiles of ty rows fit: the first and the last one hold the ghost
 // rows of their own side only, and those between none
 static bool fm_fits(int nz, int ty) { return nz >= ty + 2 * FM_H - 1; }
-bool filter_multi_takes(const FD& F) { return F.D2[1] == 1.0 && F.D2[2] == -2.0 && F.D2[3] == 1.0; }
 
 template <bool POW2, int TY, bool ALL = false>
 static void filter_multi_go(hipStream_t st, dim3 gr, const FmBufs& b, int b_in, const double* dts, const Grid& g,
-                            const FScale& sc, double courant, const FmFac& f, int m, double delta,
+                            const FScale& sc, const FmTable& tb, double courant, const FmFac& f, int m, double delta,
                             unsigned long long* slots, int32_t* ctl)
 {
-    hipLaunchKernelGGL((k_filter_multi<POW2, TY, ALL>), gr, dim3(64, FM_WAVES), 0, st, b, b_in, dts, g, sc, courant, f,
-                       m, delta, ALL ? 1 : fm_tiles(g.nz, TY), slots, ctl);
+    hipLaunchKernelGGL((k_filter_multi<POW2, TY, ALL>), gr, dim3(64, FM_WAVES), 0, st, b, b_in, dts, g, sc, tb, courant,
+                       f, m, delta, ALL ? 1 : fm_tiles(g.nz, TY), slots, ctl);
 }
 
-void launch_filter_multi(hipStream_t st, double* const bufs[3], int b_in, const double* dts, const Grid& g, double dr2,
-                         double ds2, double courant, const double* fac, int m, double delta,
+void launch_filter_multi(hipStream_t st, double* const bufs[3], int b_in, const double* dts, const Grid& g,
+                         const FD& F, double dr2, double ds2, double courant, const double* fac, int m, double delta,
                          unsigned long long* slots, int32_t* ctl, int cus)
 {
     FmBufs b{{bufs[0], bufs[1], bufs[2]}};
@@ -1282,23 +1292,24 @@ void launch_filter_multi(hipStream_t st, double* const bufs[3], int b_in, const 
     }
     const dim3 gr(gx, gz);
     const FScale sc = filter_scale(dr2, ds2);
+    const FmTable tb{{F.D2[1], F.D2[2], F.D2[3]}, F.D2[1] != 1.0 || F.D2[2] != -2.0 || F.D2[3] != 1.0};
     auto go = [&](auto pw) {
         constexpr bool P = decltype(pw)::value;
         // fewer rows than the lowest tiles need (11 iterations of 64x16: 109 us,
         // one launch each 186)
         if (best < 0) {
-            filter_multi_go<P, FM_TYS[0], true>(st, dim3((gx + FM_WAVES - 1) / FM_WAVES), b, b_in, dts, g, sc, courant, f, m,
+            filter_multi_go<P, FM_TYS[0], true>(st, dim3((gx + FM_WAVES - 1) / FM_WAVES), b, b_in, dts, g, sc, tb, courant, f, m,
                                                 delta, slots, ctl);
             return;
         }
         switch (TY) {
-        case FM_TYS[0]: filter_multi_go<P, FM_TYS[0]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
-        case FM_TYS[1]: filter_multi_go<P, FM_TYS[1]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
-        case FM_TYS[2]: filter_multi_go<P, FM_TYS[2]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
-        default: filter_multi_go<P, FM_TYS[3]>(st, gr, b, b_in, dts, g, sc, courant, f, m, delta, slots, ctl); break;
+        case FM_TYS[0]: filter_multi_go<P, FM_TYS[0]>(st, gr, b, b_in, dts, g, sc, tb, courant, f, m, delta, slots, ctl); break;
+        case FM_TYS[1]: filter_multi_go<P, FM_TYS[1]>(st, gr, b, b_in, dts, g, sc, tb, courant, f, m, delta, slots, ctl); break;
+        case FM_TYS[2]: filter_multi_go<P, FM_TYS[2]>(st, gr, b, b_in, dts, g, sc, tb, courant, f, m, delta, slots, ctl); break;
+        default: filter_multi_go<P, FM_TYS[3]>(st, gr, b, b_in, dts, g, sc, tb, courant, f, m, delta, slots, ctl); break;
         }
     };
-    if (sc.pow2) go(std::integral_constant<bool, true>{});
+    if (sc.pow2 && !tb.other) go(std::integral_constant<bool, true>{});
     else go(std::integral_constant<bool, false>{});
 }
 
