@@ -88,3 +88,33 @@ def test_defect_correction_visits_reach_the_same_solution(monkeypatch, mode, nx,
             got.append((q, g.get("SF")))
     assert abs(got[0][0] - got[1][0]) <= 1
     assert np.max(np.abs(got[0][1] - got[1][1])) <= (1e-6 if mode == "mixed" else 1e-9) * np.max(np.abs(got[0][1]))
+
+
+@pytest.mark.parametrize("mode", ["mixed", "dc64"])
+@pytest.mark.parametrize("nx,nz", [(32, 32), (152, 104), (256, 128)])
+def test_other_tables_stay_blocked(monkeypatch, mode, nx, nz):
+    """Finite-difference tables other than the second-order ones: the
+    defect-correction visits still run several sweeps per launch, and solve the
+    same equation as one sweep per launch does (to the bars above)."""
+    tol = 1e-9 if mode == "mixed" else 1e-11
+    cfg = dict(config.PRESETS["cfg0"], nx=nx, nz=nz, aspect=nx / nz, tpc=2, tolerance=tol, fixes=1, Nmulti=20)
+    params = config.make_params(**cfg)
+    cfg.update(nx=params.nx, nz=params.nz)
+    for t, f in ((params.D1, 1.01), (params.D2, 0.99), (params.D3, 1.02), (params.D4, 0.98)):
+        for j in range(5):
+            t[j] *= f
+    T, r, s, ty = ic.workload(cfg, seed=5)
+    got = []
+    for tb in ("0", "1"):
+        monkeypatch.setenv("TC_TB", tb)
+        print(f"[other tables] {mode} {params.nx}x{params.nz}, {params.grids} levels, TC_TB={tb}", flush=True)
+        with Solver(params, len(r)) as g:
+            g.initialize(T, r, s, ty)
+            g.set_mode(mode)
+            g.set_profiling(True)
+            q, resid, ref = g.multigrid()
+            assert resid <= tol * ref
+            got.append((q, g.get("SF"), g.kernel_timing()[1], g.stats().sweeps_exec[0]))
+    assert abs(got[0][0] - got[1][0]) <= 1
+    assert np.max(np.abs(got[0][1] - got[1][1])) <= (1e-6 if mode == "mixed" else 1e-9) * np.max(np.abs(got[0][1]))
+    assert got[0][2] == got[0][3] and 4 * got[1][2] <= got[1][3]   # launches and sweeps of level 1

@@ -72,8 +72,8 @@ struct tc_dev {
     bool coarse_ready = false;
     bool trace = false;
     bool coarse_lu = false;
-    bool tb = true;            // several sweeps per launch (TC_TB=0, or FD tables other than the second-order ones: one)
-    bool std_tables = false;   // the FD tables are those that the kernels of tc_visit.hip have built in
+    bool tb = true;            // several sweeps per launch (TC_TB=0, and the reference form with other FD tables: one)
+    bool std_tables = false;   // the FD tables are the second-order ones (visit_tables)
     bool fuse_rr = true;       // residual+restriction in the last launch of a visit (TC_FUSED_RR=0: apart)
     // defect-correction cycle: level-1 residual updated by increments (k_absorb_inc) with an exact
     // double-double residual before the stop test accepts (TC_INC_RESID=0: exact after every correction)
@@ -616,7 +616,7 @@ bool ref_blocked(const tc_ctx* ctx, const tc_dev& d)
     // a schedule that does not start on level 1 spends the wall reset of a
     // solve's first sweep on another level, and level 1 keeps SF's walls, which
     // a blocked visit takes as zero
-    return d.tb && ctx->mode == TC_MODE_FP64 && ctx->p.multi[1] == 1;
+    return d.tb && d.std_tables && ctx->mode == TC_MODE_FP64 && ctx->p.multi[1] == 1;
 }
 
 // whether a level's visits in the defect-correction cycle run several sweeps
@@ -692,10 +692,12 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
     const VisitPlan plan = ref ? visit_plan_ref(L.g, d.cus) : VisitPlan{};
     int n = 1;
     if (tb && Niter > 0) {
+        const FD* tables = d.std_tables ? nullptr : &d.F;
         // the tile asked for by tc_set_tb_tile (the mixed mode's): 16, 32 or 48,
         // small to large regions
-        const int only = !f32 ? 0 : (L.tb_tile == 16 ? 2 : (L.tb_tile == 32 ? 1 : (L.tb_tile == 48 ? 3 : 0)));
-        const Visit13Plan pl = visit_plan13(L.g, f32, Niter, f32 && rr, d.cus, only);
+        const int tile = !f32 ? 0 : (L.tb_tile == 16 ? 2 : (L.tb_tile == 32 ? 1 : (L.tb_tile == 48 ? 3 : 0)));
+        const int only = tables ? OTHER_TABLES_CFG : tile;
+        const Visit13Plan pl = visit_plan13(L.g, f32, Niter, f32 && rr && !tables, d.cus, only);
         const int body = (pl.end && !pl.whole) ? Niter - pl.end_k : Niter;  // sweeps of the equal launches
         double fac[VISIT_KMAX];
         for (int j = 0; j < pl.launches || n <= Niter; ++j) {
@@ -714,14 +716,14 @@ int run_sweeps(tc_ctx* ctx, tc_dev& d, int level, int Niter, int dir, bool f32, 
                 const bool with_rr = last && pl.end;
                 launch_visit13_32(ctx->stream, cfg, pl.whole, use_ratio, L, rhs32, in, L.err32[1 - L.cur32], d.h[level],
                                   fac, nk, zsg, pro ? ctx->pend_src : nullptr,
-                                  pro ? &ctx->lv[ctx->pend_from].g : nullptr, with_rr ? rr : nullptr);
+                                  pro ? &ctx->lv[ctx->pend_from].g : nullptr, with_rr ? rr : nullptr, tables);
                 if (with_rr && rr_done) *rr_done = true;
                 if (pro) ctx->pend_src = nullptr;
                 L.cur32 = 1 - L.cur32;
             } else {
                 launch_visit13_64(ctx->stream, cfg, pl.whole, use_ratio, L, view.rhs,
                                   (zero_start && n == 1) ? nullptr : L.err[L.cur], L.err[1 - L.cur], d.h[level], fac, nk,
-                                  zsg, n == 1 ? vs : VisitStart{});
+                                  zsg, n == 1 ? vs : VisitStart{}, tables);
                 L.cur = 1 - L.cur;
             }
             ++launches;
@@ -2494,7 +2496,6 @@ int init_ctx(tc_ctx* ctx, const tc_params* p, int64_t ntr)
             d->F.Drrss[t] = p->D2[dk + 2] * p->D2[di + 2];
         }
     d->std_tables = visit_tables(d->F);
-    d->tb = d->tb && d->std_tables;
     // level hierarchy (basics.f90:167-182)
     for (int j = 1; j <= ctx->grids; ++j) {
         Level& L = ctx->lv[j];

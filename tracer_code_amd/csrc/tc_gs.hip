@@ -29,8 +29,7 @@ static_assert(GS_T == 3 * 16 && GS_THREADS == 16 * 16, "one 3x3 block of the til
 #pragma clang fp contract(fast)
 // The 13 dt-scaled tap weights of every interior cell of a level, once per
 // solve (the operator's coefficients are fixed during a solve), for any
-// tables: plane q of W holds tap q in the order c, xm1, xp1, xm2, xp2, zm1,
-// zp1, zm2, zp2, mm, pm, mp, pp.
+// tables: plane q of W holds tap q in tap_weights' order.
 struct GsCoefs {
     const float *vis, *vx, *vz, *a1, *vxz, *dts;
 };
@@ -41,16 +40,8 @@ __global__ __launch_bounds__(256) void k_tb_weights32(GsCoefs C, FD32 F, H32 h, 
     if (i > g.nx - 1 || k > g.nz - 1) return;
     const size_t c = g.at(i, k), n = g.elems;
     const float vis = C.vis[c], vx = C.vx[c], vz = C.vz[c], a1 = C.a1[c], vxz = C.vxz[c], dts = C.dts[c];
-    // axis parts: a1 (S_rr - S_ss) + 2 vx S_rrr + 2 vz S_sss + vis (S_rrrr + S_ssss)
-    auto wx = [&](int d) { return a1 * F.D2[d + 2] * h.idr2 + 2.0f * vx * F.D3[d + 2] * h.idr3 + vis * F.D4[d + 2] * h.idr4; };
-    auto wz = [&](int d) { return -a1 * F.D2[d + 2] * h.ids2 + 2.0f * vz * F.D3[d + 2] * h.ids3 + vis * F.D4[d + 2] * h.ids4; };
-    // 3x3 part: 4 vxz S_rs + 2 vx S_rss + 2 vz S_rrs + 2 vis S_rrss
-    auto wb = [&](int di, int dk) {
-        return 4.0f * vxz * F.D1[dk + 2] * F.D1[di + 2] * h.idrds + 2.0f * vx * F.D2[dk + 2] * F.D1[di + 2] * h.idrds2 +
-               2.0f * vz * F.D1[dk + 2] * F.D2[di + 2] * h.idr2ds + 2.0f * vis * F.D2[dk + 2] * F.D2[di + 2] * h.idr2ds2;
-    };
-    const float v[13] = {wx(0) + wz(0) + wb(0, 0), wx(-1) + wb(-1, 0), wx(1) + wb(1, 0), wx(-2), wx(2),
-                         wz(-1) + wb(0, -1), wz(1) + wb(0, 1), wz(-2), wz(2), wb(-1, -1), wb(1, -1), wb(-1, 1), wb(1, 1)};
+    float v[13];
+    tap_weights<float>(F, h, vis, vx, vz, a1, vxz, v);
 #pragma unroll
     for (int q = 0; q < 13; ++q) W[q * n + c] = dts * v[q];
 }

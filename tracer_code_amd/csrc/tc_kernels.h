@@ -273,13 +273,15 @@ struct Visit13Plan {
 Visit13Plan visit_plan13(const Grid& g, bool f32, int n, bool end, int cus, int only);
 // nk sweeps of the 13-tap form from `in` (nullptr: a zero correction) into
 // `out`; Pc (optional): a coarse correction on grid *gc prolonged into `in`
-// first; rr (optional): also form its right-hand side
+// first; rr (optional): also form its right-hand side; tables: nullptr for the
+// second-order ones, else cfg is OTHER_TABLES_CFG and rr nullptr
+constexpr int OTHER_TABLES_CFG = 2;
 void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const float* rhs,
                        const float* in, float* out, const Spacing& h, const double* fac, int nk, double zsg,
-                       const float* Pc, const Grid* gc, const RRTarget* rr);
+                       const float* Pc, const Grid* gc, const RRTarget* rr, const FD* tables);
 void launch_visit13_64(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const double* rhs,
                        const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
-                       const VisitStart& vs);
+                       const VisitStart& vs, const FD* tables);
 
 // --- tc_fields.hip -------------------------------------------------------------
 void launch_velocities(hipStream_t st, const double* SF, double* u, double* w, const Grid& g, const FD& F, double dr,

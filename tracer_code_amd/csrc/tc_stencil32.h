@@ -93,6 +93,26 @@ struct LdsAt {
     __device__ __forceinline__ float operator()(int di, int dk) const { return f[c + dk * ld + di]; }
 };
 
+// The weights of the 13 taps of one point for any tables F (D1..D4 at
+// offsets -2..2) and reciprocal spacings h: c, xm1, xp1, xm2, xp2, zm1, zp1,
+// zm2, zp2, mm, pm, mp, pp
+template <typename T, typename TAB, typename H>
+__device__ __forceinline__ void tap_weights(const TAB& F, const H& h, T vis, T vx, T vz, T a1, T vxz, T (&v)[13])
+{
+    // axis parts: a1 (S_rr - S_ss) + 2 vx S_rrr + 2 vz S_sss + vis (S_rrrr + S_ssss)
+    auto wx = [&](int d) { return a1 * F.D2[d + 2] * h.idr2 + T(2) * vx * F.D3[d + 2] * h.idr3 + vis * F.D4[d + 2] * h.idr4; };
+    auto wz = [&](int d) { return -a1 * F.D2[d + 2] * h.ids2 + T(2) * vz * F.D3[d + 2] * h.ids3 + vis * F.D4[d + 2] * h.ids4; };
+    // 3x3 part: 4 vxz S_rs + 2 vx S_rss + 2 vz S_rrs + 2 vis S_rrss
+    auto wb = [&](int di, int dk) {
+        return T(4) * vxz * F.D1[dk + 2] * F.D1[di + 2] * h.idrds + T(2) * vx * F.D2[dk + 2] * F.D1[di + 2] * h.idrds2 +
+               T(2) * vz * F.D1[dk + 2] * F.D2[di + 2] * h.idr2ds + T(2) * vis * F.D2[dk + 2] * F.D2[di + 2] * h.idr2ds2;
+    };
+    const T w[13] = {wx(0) + wz(0) + wb(0, 0), wx(-1) + wb(-1, 0), wx(1) + wb(1, 0), wx(-2), wx(2),
+                     wz(-1) + wb(0, -1), wz(1) + wb(0, 1), wz(-2), wz(2), wb(-1, -1), wb(1, -1), wb(-1, 1), wb(1, 1)};
+#pragma unroll
+    for (int q = 0; q < 13; ++q) v[q] = w[q];
+}
+
 // restrict (iterative_solver.f90:596-626) at one coarse point from the fine
 // residuals around its fine centre: the reference's weights, whose corner sum
 // counts (ii-1,kk+1) twice and (ii+1,kk-1) not at all

@@ -373,6 +373,22 @@ __device__ __forceinline__ Cell13<T> weights13(T vis, T vx, T vz, T a1, T vxz, T
     return w;
 }
 
+// the same for any tables
+template <typename T>
+struct Tables13 {
+    T D1[5], D2[5], D3[5], D4[5];
+};
+struct NoTables {};
+template <typename T>
+__device__ __forceinline__ Cell13<T> weights13_any(const Tables13<T>& F, T vis, T vx, T vz, T a1, T vxz, T dts, T rhs,
+                                                   const H13<T>& h)
+{
+    T v[13];
+    tap_weights<T>(F, h, vis, vx, vz, a1, vxz, v);
+    return Cell13<T>{dts * v[0], dts * v[1], dts * v[2], dts * v[3],  dts * v[4],  dts * v[5],  dts * v[6],
+                     dts * v[7], dts * v[8], dts * v[9], dts * v[10], dts * v[11], dts * v[12], dts * rhs};
+}
+
 // 1/x of the per-point factor (1 <= x <= 5): the hardware's reciprocal with a
 // Newton step, which rounds to within an ulp of the quotient
 __device__ __forceinline__ float recip(float x)
@@ -410,10 +426,11 @@ __device__ __forceinline__ T step13(const Taps<T>& t, const Cell13<T>& w)
 // its restriction to the next level (residual32_std, restrict_fw32: the
 // values of k_residual_restrict32), for which the region reaches 2 cells
 // before and 3 behind the own ones.
-template <typename T, bool RATIO, int LW, int R, int NW, bool END>
+// TAB: NoTables for the second-order tables, else the tables.
+template <typename T, bool RATIO, int LW, int R, int NW, bool END, typename TAB = NoTables>
 __global__ __launch_bounds__(NW * 64) void k_visit13(const T* __restrict__ Ein, T* __restrict__ Eout, Args13<T> A,
                                                      Grid g, H13<T> h, VisitTile vt, VisitFac<T> sf, int nk, T zsg,
-                                                     Start13<T> pr, End13 en)
+                                                     Start13<T> pr, End13 en, TAB tab)
 {
     constexpr int GR = 64 / LW, ROWS = NW * GR * R;
     __shared__ T buf[2][ROWS * LW];
@@ -465,7 +482,8 @@ __global__ __launch_bounds__(NW * 64) void k_visit13(const T* __restrict__ Ein, 
             }
         }
         if (!in) S[r] = T(0);
-        q[r] = weights13<T>(vis, vx, vz, a1, vxz, in ? dts : T(0), rhs, h);
+        if constexpr (std::is_same_v<TAB, NoTables>) q[r] = weights13<T>(vis, vx, vz, a1, vxz, in ? dts : T(0), rhs, h);
+        else q[r] = weights13_any<T>(tab, vis, vx, vz, a1, vxz, in ? dts : T(0), rhs, h);
         if constexpr (END) { rc[r][0] = vis; rc[r][1] = vx; rc[r][2] = vz; rc[r][3] = a1; rc[r][4] = vxz; rc[r][5] = rhs; }
         if constexpr (RATIO) {
             if constexpr (sizeof(T) == 4) {
@@ -589,8 +607,8 @@ dim3 tile_grid(const Grid& g, const VisitTile& t)
 
 }  // namespace
 
-// Whether the FD tables are the second-order ones that the kernels of this
-// file have built in (config.fd_coefficients(2), main.f90:350-469).
+// Whether the FD tables are the second-order ones that k_visit_ref and
+// k_visit13's weights have built in (config.fd_coefficients(2), main.f90:350-469).
 bool visit_tables(const FD& F)
 {
     static const double d1[3] = {-0.5, 0.0, 0.5}, d2[3] = {1.0, -2.0, 1.0};
@@ -722,7 +740,8 @@ static double cost13(int cfg, bool f32, int k, double tiles, int cus, bool end)
 // with the residual and restriction: 128x64 9.7 (15.0), 256x128 10.3 (14.6),
 // 512x256 14.7 (21.3); 16 sweeps of 1024x512 44 (85); 10 of 2048x1024, none:
 // 69 (127 as ten launches of one sweep).  only: 0, or the region that
-// tc_set_tb_tile asks for; it too runs a level that it holds whole.
+// tc_set_tb_tile asks for (it too runs a level that it holds whole), or the
+// one that other tables than the second-order ones take.
 Visit13Plan visit_plan13(const Grid& g, bool f32, int n, bool end, int cus, int only)
 {
     Visit13Plan p;
@@ -802,19 +821,19 @@ void visit13_go(hipStream_t st, dim3 gr, bool ratio, bool end, const T* in, T* o
     const dim3 b(NW * 64);
     if constexpr (sizeof(T) == 4) {
         if (end) {
-            if (ratio) hipLaunchKernelGGL((k_visit13<T, true, LW, R, NW, true>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
-            else hipLaunchKernelGGL((k_visit13<T, false, LW, R, NW, true>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
+            if (ratio) hipLaunchKernelGGL((k_visit13<T, true, LW, R, NW, true>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en, NoTables{});
+            else hipLaunchKernelGGL((k_visit13<T, false, LW, R, NW, true>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en, NoTables{});
             return;
         }
     }
-    if (ratio) hipLaunchKernelGGL((k_visit13<T, true, LW, R, NW, false>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
-    else hipLaunchKernelGGL((k_visit13<T, false, LW, R, NW, false>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en);
+    if (ratio) hipLaunchKernelGGL((k_visit13<T, true, LW, R, NW, false>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en, NoTables{});
+    else hipLaunchKernelGGL((k_visit13<T, false, LW, R, NW, false>), gr, b, 0, st, in, out, A, g, h, vt, sf, nk, zsg, pr, en, NoTables{});
 }
 
 template <typename T>
 void launch13(hipStream_t st, int cfg, bool whole, bool ratio, bool end, const Args13<T>& A, const Grid& g,
               const Spacing& h, const T* in, T* out, const double* fac, int nk, double zsg, const Start13<T>& pr,
-              const End13& en)
+              const End13& en, const FD* tables)
 {
     VisitFac<T> sf;
     for (int s = 0; s < nk; ++s) sf.v[s] = (T)fac[s];
@@ -823,6 +842,19 @@ void launch13(hipStream_t st, int cfg, bool whole, bool ratio, bool end, const A
     const dim3 gr = tile_grid(g, vt);
     const H13<T> hh = h13_from<T>(h);
     const T z = (T)zsg;
+    if (tables) {
+        // (cfg is OTHER_TABLES_CFG)
+        Tables13<T> tb;
+        for (int j = 0; j < 5; ++j) {
+            tb.D1[j] = (T)tables->D1[j];
+            tb.D2[j] = (T)tables->D2[j];
+            tb.D3[j] = (T)tables->D3[j];
+            tb.D4[j] = (T)tables->D4[j];
+        }
+        if (ratio) hipLaunchKernelGGL((k_visit13<T, true, 32, 1, 16, false, Tables13<T>>), gr, dim3(1024), 0, st, in, out, A, g, hh, vt, sf, nk, z, pr, en, tb);
+        else hipLaunchKernelGGL((k_visit13<T, false, 32, 1, 16, false, Tables13<T>>), gr, dim3(1024), 0, st, in, out, A, g, hh, vt, sf, nk, z, pr, en, tb);
+        return;
+    }
     switch (cfg) {
     case 0: visit13_go<T, 16, 1, 4>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en); break;
     case 1: visit13_go<T, 64, 2, 16>(st, gr, ratio, end, in, out, A, g, hh, vt, sf, nk, z, pr, en); break;
@@ -839,7 +871,7 @@ void launch13(hipStream_t st, int cfg, bool whole, bool ratio, bool end, const A
 
 void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const float* rhs,
                        const float* in, float* out, const Spacing& h, const double* fac, int nk, double zsg,
-                       const float* Pc, const Grid* gc, const RRTarget* rr)
+                       const float* Pc, const Grid* gc, const RRTarget* rr, const FD* tables)
 {
     const Args13<float> A{L.vis32, L.visx32, L.visz32, L.a132, nullptr, nullptr, L.visxz32,
                          const_cast<float*>(rhs), L.dts32, L.lb32};
@@ -847,16 +879,16 @@ void launch_visit13_32(hipStream_t st, int cfg, bool whole, bool use_ratio, cons
     if (Pc) { pr.Ec = Pc; pr.gc = *gc; }
     End13 en{};
     if (rr) { en.out = rr->out; en.go = rr->go; en.RowB = rr->RowB; en.bout = rr->bout; en.h = h32_from(h); }
-    launch13<float>(st, cfg, whole, use_ratio, rr != nullptr, A, L.g, h, in, out, fac, nk, zsg, pr, en);
+    launch13<float>(st, cfg, whole, use_ratio, rr != nullptr, A, L.g, h, in, out, fac, nk, zsg, pr, en, tables);
 }
 
 void launch_visit13_64(hipStream_t st, int cfg, bool whole, bool use_ratio, const Level& L, const double* rhs,
                        const double* in, double* out, const Spacing& h, const double* fac, int nk, double zsg,
-                       const VisitStart& vs)
+                       const VisitStart& vs, const FD* tables)
 {
     const Args13<double> A{L.vis, L.visx, L.visz, nullptr, L.visxx, L.viszz, L.visxz, const_cast<double*>(rhs),
                            L.dtstream, L.ratio};
-    launch13<double>(st, cfg, whole, use_ratio, false, A, L.g, h, in, out, fac, nk, zsg, vs, End13{});
+    launch13<double>(st, cfg, whole, use_ratio, false, A, L.g, h, in, out, fac, nk, zsg, vs, End13{}, tables);
 }
 
 }  // namespace tc
