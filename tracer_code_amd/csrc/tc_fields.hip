@@ -325,21 +325,6 @@ __global__ __launch_bounds__(256) void k_filter_iter(const double* __restrict__ 
 // instructions an iteration): 2048x1024 22.6 against 33.9 us, 1024x512 10.2
 // against 18.2, 608x352 (quotients by remainders) 9.5 against 22.2.
 // ---------------------------------------------------------------------------
-// a double from lane l-1 (wave_shr:1) or lane l+1 (wave_shl:1) of the
-// wavefront, as DPP moves of its two halves; lane 0 (63) gets 0
-__device__ __forceinline__ double dpp_from_left(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x138, 0xF, 0xF, true),
-                            __builtin_amdgcn_mov_dpp(lo, 0x138, 0xF, 0xF, true));
-}
-__device__ __forceinline__ double dpp_from_right(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x130, 0xF, 0xF, true),
-                            __builtin_amdgcn_mov_dpp(lo, 0x130, 0xF, 0xF, true));
-}
-
 constexpr int FM_K = 4;                  // iterations per launch
 constexpr int FM_H = FM_K + 1;           // halo: one cell per iteration, one for the last measure
 constexpr int FM_TXO = 64 - 2 * FM_H;    // own columns of a wavefront's tile
@@ -408,7 +393,7 @@ __device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], 
 #pragma unroll
         for (int r = 1; r < RY - 1; ++r) {
             const double oc = c[r];
-            const double lf = dpp_from_left(oc), rt = dpp_from_right(oc);
+            const double lf = from_left(oc), rt = from_right(oc);
             double temp;
             if constexpr (FORM == FM_ANY) {
                 const double x = tb.d[0] * lf + tb.d[1] * oc + tb.d[2] * rt, z = tb.d[0] * om + tb.d[1] * oc + tb.d[2] * c[r + 1];
@@ -465,11 +450,11 @@ __device__ __forceinline__ void fm_iterate(double (&c)[RY], double (&mx)[FM_K], 
             // (node r's jump up is node r-1's jump down, |x-y| = |y-x|); the
             // maximum is that of smooth_merge
             double a = fabs(c[RA - 1] - c[RA]), b = 0.0;
-            double rm = dpp_from_right(c[RA - 1]), r0 = dpp_from_right(c[RA]);  // the right lane's c[r-1], c[r]
+            double rm = from_right(c[RA - 1]), r0 = from_right(c[RA]);  // the right lane's c[r-1], c[r]
 #pragma unroll
             for (int r = RA; r <= RB; ++r) {
                 if (ZK == 3 && r >= rn) break;
-                const double rp = dpp_from_right(c[r + 1]);
+                const double rp = from_right(c[r + 1]);
                 a = fmax(a, fabs(rm - c[r]));
                 b = fmax(b, fabs(r0 - c[r]));
                 a = fmax(a, fabs(c[r + 1] - c[r]));

@@ -17,6 +17,30 @@ struct EigScalars {
     double Trs_max, Trss_max, Trrs_max, Trrss_max;
 };
 
+// The value of the previous lane of the wavefront (wave_shr:1) and of the next
+// (wave_shl:1), as DPP moves of a double's two halves; the first (last) lane
+// gets 0.
+__device__ __forceinline__ float from_left(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float from_right(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double from_left(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x138, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(lo, 0x138, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double from_right(double v)
+{
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x130, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(lo, 0x130, 0xF, 0xF, true));
+}
+
 // Block-wide reductions (any block shape up to 1024 threads, wave64).
 // The combination order is fixed, so results are run-to-run deterministic.
 __device__ __forceinline__ int flat_tid() { return threadIdx.z * blockDim.x * blockDim.y + threadIdx.y * blockDim.x + threadIdx.x; }

@@ -594,19 +594,6 @@ constexpr int VM_TYS[2] = {14, 24};      // own rows of the other tiles (nz >= T
 
 struct VmFac { double v[VM_K]; };
 
-__device__ __forceinline__ double vm_left(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x138, 0xF, 0xF, true),
-                            __builtin_amdgcn_mov_dpp(lo, 0x138, 0xF, 0xF, true));
-}
-__device__ __forceinline__ double vm_right(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x130, 0xF, 0xF, true),
-                            __builtin_amdgcn_mov_dpp(lo, 0x130, 0xF, 0xF, true));
-}
-
 template <bool POW2, int RY, int TY, int ZK>
 __device__ __forceinline__ void vm_iterate(double (&c)[RY], int n, const double* fac, double dt, const Spacing& h,
                                            bool gcols, bool ghost_col, int ml, double w0, double wn, int nz)
@@ -619,7 +606,7 @@ __device__ __forceinline__ void vm_iterate(double (&c)[RY], int n, const double*
 #pragma unroll
         for (int r = 1; r < RY - 1; ++r) {
             const double oc = c[r];
-            const double lf = vm_left(oc), rt = vm_right(oc);
+            const double lf = from_left(oc), rt = from_right(oc);
             const double x = fma(-2.0, oc, lf) + rt, z = fma(-2.0, oc, om) + c[r + 1];
             double temp;
             if constexpr (POW2) temp = fma(x, h.idr2, z * h.ids2);

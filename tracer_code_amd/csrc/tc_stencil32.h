@@ -85,14 +85,6 @@ struct Patch7At {
     __device__ __forceinline__ float operator()(int di, int dk) const { return p[(b + dk + 3) * 7 + a + di + 3]; }
 };
 
-// S(i+di, k+dk) of a tile staged in LDS with row pitch ld
-struct LdsAt {
-    const float* f;
-    int c;
-    int ld;
-    __device__ __forceinline__ float operator()(int di, int dk) const { return f[c + dk * ld + di]; }
-};
-
 // The weights of the 13 taps of one point for any tables F (D1..D4 at
 // offsets -2..2) and reciprocal spacings h: c, xm1, xp1, xm2, xp2, zm1, zp1,
 // zm2, zp2, mm, pm, mp, pp

@@ -33,31 +33,9 @@ namespace tc {
 namespace {
 
 // ---- lane shifts -------------------------------------------------------------
-// the value of the previous lane (wave_shr:1) or the next (wave_shl:1); the
-// first (last) lane gets 0.  Between the row groups of a wavefront the
-// shifts cross from one group's last column to the next group's first: both
-// are cells of the halo or a wall (or beyond it), see the tile rule below.
-__device__ __forceinline__ double from_left(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x138, 0xF, 0xF, true),
-                            __builtin_amdgcn_mov_dpp(lo, 0x138, 0xF, 0xF, true));
-}
-__device__ __forceinline__ double from_right(double v)
-{
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0x130, 0xF, 0xF, true),
-                            __builtin_amdgcn_mov_dpp(lo, 0x130, 0xF, 0xF, true));
-}
-
-__device__ __forceinline__ float from_left(float v)
-{
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float from_right(float v)
-{
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xF, 0xF, true));
-}
+// Between the row groups of a wavefront from_left and from_right cross from one
+// group's last column to the next group's first: both are cells of the halo or
+// a wall (or beyond it), see the tile rule below.
 
 // ---- geometry ------------------------------------------------------------------
 // The region of tile (X, Y) starts at column 1 + X*tx - hx, row 1 + Y*ty - hz.
@@ -215,8 +193,7 @@ __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict_
     const int w0 = wv * GR * R, w1 = w0 + GR * R - 1;
     const int kg = 1 + tile.y * vt.ty - vt.hz;
     const int own0 = vt.hz, own1 = vt.hz + vt.ty - 1;
-    auto taps = [&](const double* __restrict__ b, int r, const double (&v)[R + 4], const double (&lf)[R + 2],
-                    const double (&rt)[R + 2]) {
+    auto taps = [&](int r, const double (&v)[R + 4], const double (&lf)[R + 2], const double (&rt)[R + 2]) {
         Taps<double> t;
         t.c = v[r + 2];
         t.zm1 = v[r + 1]; t.zp1 = v[r + 3]; t.zm2 = v[r]; t.zp2 = v[r + 4];
@@ -229,7 +206,6 @@ __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict_
         }
         if (k0 + r == 1) t.zm2 = zsg * t.c;
         if (k0 + r == g.nz - 1) t.zp2 = zsg * t.c;
-        (void)b;
         return t;
     };
     // the rows -2..R+1 around the lane's own, and their neighbours along x
@@ -263,7 +239,7 @@ __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict_
         const double f = sf.v[s];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const Taps<double> t = taps(b, r, v, lf, rt);
+            const Taps<double> t = taps(r, v, lf, rt);
             double cc = f;
             if constexpr (RATIO) cc = 2.0 / (-lb[r] + 1.0 + (lb[r] + 1.0) * f);
             n[r] = S[r] + cc * q[r].dts * ref_residual<POW2>(t, q[r], h);
@@ -288,7 +264,7 @@ __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict_
         gather(b, v, lf, rt);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const Taps<double> t = taps(b, r, v, lf, rt);
+            const Taps<double> t = taps(r, v, lf, rt);
             const double res = ref_residual<POW2>(t, q[r], h);
             if (col && k0 + r >= 1 && k0 + r <= g.nz - 1) Rout[g.at(i, k0 + r)] = res;
         }
