@@ -2,8 +2,8 @@
 fields that the tracers do not give: random ratios, values beyond [0,1] (the
 clamp), a NaN, and infinities and values whose quotients overflow, at the heights and widths where a tile ends -- heights that
 one tile holds (4 to 16 rows), the smallest height with tiles, a last tile
-that overlaps the one before it, one column or row more than a tile.  Same
-iterates, stop and bits."""
+that overlaps the one before it, one column or row more than a tile, and
+every tile height.  Same iterates, stop and bits."""
 import numpy as np
 import pytest
 
@@ -12,14 +12,14 @@ from tracer_code_amd import Solver, config
 pytestmark = pytest.mark.gpu
 
 
+# the larger grids take tiles of 11, 16 and 21 rows (on 256 CUs), the smaller
+# ones of 8; spacings that are powers of two at 512 and 1024 rows
 @pytest.mark.parametrize("kind", ["ratio", "beyond", "nan", "huge"])
 @pytest.mark.parametrize("nx,nz", [(12, 4), (52, 6), (10, 16), (24, 16), (104, 10),
                                    (300, 14), (16, 18), (54, 20), (56, 38), (108, 50), (110, 26), (160, 96), (212, 130),
-                                   (1024, 512), (1920, 992)])
+                                   (1952, 192), (1024, 512), (1952, 288), (544, 1024), (1920, 992), (2048, 1024)])
 def test_filter_tiles_same_bits(nx, nz, kind):
-    if nx > 1000 and kind != "ratio":
-        pytest.skip("the walls' handling does not depend on the size")
-    params = config.make_params(nx=nx, nz=max(nz, 8), aspect=nx / nz, grids=2 if nx < 1000 else 6, ivis=2,
+    params = config.make_params(nx=nx, nz=max(nz, 8), aspect=nx / nz, grids=2 if nx * nz < 50000 else 6, ivis=2,
                                 visC=(1.0 / 30.0,), delta_visC=(1.5,))
     params.nz = nz   # (make_params keeps 4 cells on the coarsest level, the library 2)
     print(f"[filter tiles] {params.nx}x{params.nz} {kind}", flush=True)
