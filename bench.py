@@ -600,7 +600,7 @@ def main():
         "boundary_form": dict(bnd, steps_per_s_with_copies=1e3 / (head["ms_per_step"] + bnd["ms_per_step"])),
         "roofline": {
             "kernel": f"{kname} level 1 (Jacobi-Richardson smoother)",
-            "bound": "hbm",
+            "bound": "instruction issue" if (sweeps_per_launch or 1.0) > 1.01 else "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -610,8 +610,8 @@ def main():
             "sweeps_per_launch": sweeps_per_launch,
             "us_per_sweep": avg_us / sweeps_per_launch if sweeps_per_launch else None,
             "launches": head["sweep_launches"],
-            "note": "a launch moves its arrays once for several sweeps: below the HBM peak by design, "
-                    "bound by instruction issue" if (sweeps_per_launch or 1.0) > 1.01 else "",
+            "note": "a launch moves its arrays once for several sweeps: below the HBM peak by design "
+                    "(issue shares: profiles/counters_visits_filter.md)" if (sweeps_per_launch or 1.0) > 1.01 else "",
             "algorithmic_bytes_per_launch": bytes_per_launch,
             "kernel_bytes_per_launch": KERNEL_BYTES_PER_POINT[args.mode] * pts1,
         },

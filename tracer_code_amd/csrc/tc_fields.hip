@@ -318,12 +318,15 @@ __global__ __launch_bounds__(256) void k_filter_iter(const double* __restrict__ 
 // Slot sets: 3K, set j mod 3K for iterate j; a launch reads K, writes K and
 // clears the K its successor writes.
 //
-// Bound: FP64 issue (13 instructions a held cell and 10 a measured one per
-// iteration, 4 cycles each) and the halo (26 of 64x26 held cells are own).
-// Measured per launch of 4 iterations, against a form that tested every row
-// against the walls and reduced over the block in every iteration (2500
-// instructions an iteration): 2048x1024 22.6 against 33.9 us, 1024x512 10.2
-// against 18.2, 608x352 (quotients by remainders) 9.5 against 22.2.
+// Bound: one or two waves per SIMD, which wait for their loads and for the
+// dependent FP64 operations of an iteration (VALU issue, 13 instructions a held
+// cell and 10 a measured one, fills 36% of a launch at 2048x1024 and 21% at
+// 608x352), and the halo: 54 TY of 64 (TY + 10) held cells are own, 38% at TY =
+// 8, 57% at 21.  Measured per launch of 4 iterations, against a form that
+// tested every row against the walls and reduced over the block in every
+// iteration (2500 instructions an iteration): 2048x1024 21.4 against 33.9 us,
+// 1024x512 10.0 against 18.2, 608x352 (quotients by remainders) 9.6 against
+// 22.2.
 // ---------------------------------------------------------------------------
 constexpr int FM_K = 4;                  // iterations per launch
 constexpr int FM_H = FM_K + 1;           // halo: one cell per iteration, one for the last measure

@@ -134,11 +134,14 @@ struct RefArgs {
     const double *dts, *ratio;
 };
 
-// Bound: FP64 arithmetic and one barrier a sweep (a region of 32x32 cells: 4
+// Bound: VALU issue and one barrier a sweep (a region of 32x32 cells: 4
 // rows of 64 cells per SIMD, about 85 instructions of 4 cycles each, 0.65 us
 // with the barrier), plus 2.5 to 3 us for the launch and the loads of 9
-// planes, which the launch's sweeps share.  On the levels that do not fit
-// the L2s (1024x512 and up) the loads: 72 B per staged cell.
+// planes, which the launch's sweeps share.  By counters, issue fills 71% of a
+// launch that holds 32x32 cells (35% at 16x16, one wave a SIMD: there the chain
+// of LDS round trip, barrier and FMAs is longer), 29 to 48% of the tiles of
+// region 2 and 46 to 58% of region 3's, which move 2.1 to 3.0 TB/s beside it
+// (72 B per staged cell).
 // RES (one tile holds the level): the residual of the result goes to R.
 template <bool POW2, bool RATIO, int LW, int R, int NW, bool RES>
 __global__ __launch_bounds__(NW * 64) void k_visit_ref(const double* __restrict__ Ein, double* __restrict__ Eout,
@@ -396,8 +399,10 @@ __device__ __forceinline__ T step13(const Taps<T>& t, const Cell13<T>& w)
 
 // Bound: the launch and the loads (3.4 us with a 32x32 region of one row a
 // lane, of which 256 fit the chip), then 0.2 us a sweep (about 25
-// instructions a point and the barrier); on the levels of more tiles, the
-// loads of the staged cells (32 B each, FP32).
+// instructions a point and the barrier).  By counters, VALU issue fills 25 to
+// 34% of such launches and 63 to 75% of those that hold a level of 64 columns;
+// on the levels of more tiles 52 to 71%, beside loads of 32 B per staged cell
+// (FP32, 1.9 to 3.4 TB/s).
 // END: after the last sweep, FP32: the residual in FP64 of the held cells and
 // its restriction to the next level (residual32_std, restrict_fw32: the
 // values of k_residual_restrict32), for which the region reaches 2 cells
