@@ -201,7 +201,10 @@ constexpr int WGRAD_PIX = 2048;  // pixels of a split
 // Bound: the latency of the loads and of the chain, up to 64 iterations of 32
 // pixels.  One wave a split, with 2-byte loads of each fragment's values,
 // took 148 to 170 us a layer at 32x96 pixels, in 10 to 28 waves; 16 waves a
-// split and 16-byte loads take 6.4 to 7.3.
+// split and 16-byte loads take 6.4 to 7.3 (8 waves of 8 iterations 6.0 to 6.8,
+// within the noise of a step; 4 of 16 11.4 to 12.0).  Splits that fill the chip
+// took 3.4, a step 13 us less of 805, with sums that depend on the image's
+// size.
 // The reduction runs over pixels, along which neither operand is contiguous:
 // a lane loads 8 channels (16 bytes) of a pixel, LDS holds [pixel][16
 // channels], and the transposing reads give the fragments.
